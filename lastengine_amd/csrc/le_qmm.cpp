@@ -82,7 +82,7 @@ struct le_ctx {
     int mq = 1;              /* decode matvec on MFMA where available */
     int mq_waves_auto = 1;   /* double mq_waves for grids smaller than the chip */
     int mq_waves = 4, mq_steps = 2, mq_blocks_per_cu = 2;
-    int ms = 1, ms_p = 2;    /* staged MFMA variant and its super-blocks per row and step */
+    int ms = 1, ms_p = 0;    /* staged MFMA variant and its super-blocks per row and item (0: chosen in mq_launch; so the others below) */
     int rd_nt = 1, rd_u = 4, rd_blocks_per_cu = 1, rd_block = 512; /* le_stream_read probe shape */
     int ms_t = 1;            /* Q4_K with 2..8 tokens per pass on the staged MFMA kernel */
     int gm_mh = 1;           /* le_gemm, Q4_K, 3..8 tokens: the staged f16 MFMA kernel */
@@ -91,17 +91,16 @@ struct le_ctx {
     /* Q8_0 and Q4_0 batch-1 matvec on the staged MFMA kernels, with ms_p80 / ms_p40 super-blocks per
      * item (Q8_0 32000x4096: 29.7 us against the vector kernel's 36.5; Q4_0 14336x4096: 10.7 against
      * 12.6, 4096x4096: 5.4 against 11.1) */
-    int ms80 = 1, ms_p80 = 1, ms40 = 1, ms_p40 = 2;
-    int ms_wide = 1;         /* down shapes on 12-16 waves, every type but Q6_K and Q8_0 (below) */
-    int ms2s = 1, ms_p2s = 1; /* IQ2_S on the Q6_K kernel's map (14336x4096: 13.0 us against the vector kernel's 13.9, 4096x4096: 6.2 against 8.7) */
-    int ms3k = 1, ms_p3k = 2; /* Q3_K on the Q6_K kernel's map (14336x4096: 11.7 us against the vector kernel's 15.7, 4096x4096: 5.4 against 9.5) */
-    int ms5k = 1, ms_p5k = 1; /* Q5_K the same way (the Q4_K kernel with the fifth bit from qh; 14336x4096: 11.1 us against the vector kernel's 14.5, 4096x4096: 4.9 against 8.5) */
+    int ms80 = 1, ms_p80 = 0, ms40 = 1, ms_p40 = 0;
+    int ms_wide = 1;         /* down shapes on 16 waves (mq_launch) */
+    int ms2s = 1, ms_p2s = 0; /* IQ2_S on the Q6_K kernel's map (14336x4096: 13.0 us against the vector kernel's 13.9, 4096x4096: 6.2 against 8.7) */
+    int ms3k = 1, ms_p3k = 0; /* Q3_K on the Q6_K kernel's map (14336x4096: 11.7 us against the vector kernel's 15.7, 4096x4096: 5.4 against 9.5) */
+    int ms5k = 1, ms_p5k = 0; /* Q5_K the same way (the Q4_K kernel with the fifth bit from qh; 14336x4096: 11.1 us against the vector kernel's 14.5, 4096x4096: 4.9 against 8.5) */
     int mq_q8 = 1;           /* int8 mode on the staged MFMA kernels: Q4_K 14336x4096 13.1 -> 9.9 us, Q6_K 4096x14336
                                 27.7 -> 15.3, IQ3_XXS 16.6 -> 15.7 against the vector kernels (IQ2_XXS stays
                                 there: 10.5 against 11.3) */
-    int mq6 = 1, ms_p6 = 1;  /* Q6_K decode matvec on the staged MFMA kernels, super-blocks per step (1: 1024x4096 5.6 -> 5.0 us,
-                                4096x4096 6.3 -> 5.5, 14336x4096 14.8 -> 14.2 against 2) */
-    int mqiq = 1, ms_piq = 2; /* IQ2_XXS / IQ3_XXS likewise */
+    int mq6 = 1, ms_p6 = 0;  /* Q6_K decode matvec on the staged MFMA kernels */
+    int mqiq = 1, ms_piq = 0; /* IQ2_XXS / IQ3_XXS likewise */
     int moe_fast = 1;        /* decode-shaped MoE kernels */
     int moe_chunk = 1;       /* decode-form MoE above 8 tokens: consecutive calls of at most 8 tokens */
     int moe_mfma = 1;        /* decode-shaped MoE on the staged MFMA kernels where the types allow */
@@ -239,7 +238,8 @@ int mq_launch(le_ctx *c, int ty, const void *const *ptrs, const void *w, const f
     const long long ntile = (rows + 15) / 16;
     const int nsb = cols / 256, U = c->mq_steps;
     /* when the row tiles alone leave CUs idle, split K over twice the waves (shorter chains) */
-    const int NW = c->mq_waves_auto && ntile * slots <= c->cus && c->mq_waves < 8 ? 2 * c->mq_waves : c->mq_waves;
+    const bool few = c->mq_waves_auto && ntile * slots <= c->cus;
+    const int NW = few && c->mq_waves < 8 ? 2 * c->mq_waves : c->mq_waves;
     long long gx = ntile, cap = (long long)c->cus * c->mq_blocks_per_cu;
     if (gx > cap) {
         const long long it = (gx + cap - 1) / cap;
@@ -262,37 +262,44 @@ int mq_launch(le_ctx *c, int ty, const void *const *ptrs, const void *w, const f
     void *args[] = {&a};
     char name[64];
     size_t lds = (size_t)nsb * 608 + (size_t)NW * 64;
-    /* staged variant: P super-blocks per row and item, NWs waves splitting K evenly */
-    int P = ty == LE_TYPE_Q6_K ? c->ms_p6 : ty == LE_TYPE_Q4_K ? c->ms_p : ty == LE_TYPE_Q8_0 ? c->ms_p80 : ty == LE_TYPE_Q4_0 ? c->ms_p40 : ty == LE_TYPE_Q5_K ? c->ms_p5k : ty == LE_TYPE_Q3_K ? c->ms_p3k : ty == LE_TYPE_IQ2_S ? c->ms_p2s : c->ms_piq, NWs = NW;
+    /* Staged variant: items of P super-blocks per row, dealt to NWs waves in turn; they need not divide
+     * evenly. What counts is the waves' longest chain of items, so the split follows the number of
+     * super-blocks and not its divisors (27 super-blocks: 8 waves of 3-4 instead of one wave of 27,
+     * Q6_K 2560 x 6912 21.9 -> 6.9 us, Q4_K 13824 x 2560 13.4 -> 7.8; 43 super-blocks, 3328 rows of
+     * Q4_K: 7.4 us on 16 waves, 8.4 on 8, 10.9 on 4). By rows and K, us measured on all types:
+     *  - no more row tiles than CUs (one block per CU): 16 waves from 40 super-blocks (Q4_K 4096 x
+     *    14336 8.8 against 10.4 on 8, Q6_K 13.2 / 14.1, IQ3_XXS 11.3 / 11.9, Q8_0 16.3 / 16.6; at 28
+     *    super-blocks 8 waves win, Q4_K 5.2 / 5.9), items of two for the K-quants that gain by it
+     *    (Q4_K 8.8 / 9.4, Q6_K 13.2 / 13.9) and one otherwise; fewer super-blocks: 8 waves, items
+     *    of one (Q6_K 2304 x 7168 6.9 / 8.1), but two for Q4_K where that shortens the chain (1536 x
+     *    5632 4.4 / 5.0);
+     *  - more row tiles: 4 waves, items of two from 16 super-blocks (14336 x 4096 Q4_K 8.8 / 9.8, Q5_K
+     *    11.0 / 11.7, Q6_K 13.9 / 14.9, IQ3_XXS 11.6 / 12.1; not Q8_0, 32000 x 4096 25.8 / 25.4), of
+     *    one below (12288 x 3072: within 2%). */
+    const int pset = ty == LE_TYPE_Q6_K ? c->ms_p6 : ty == LE_TYPE_Q4_K ? c->ms_p : ty == LE_TYPE_Q8_0 ? c->ms_p80 : ty == LE_TYPE_Q4_0 ? c->ms_p40 : ty == LE_TYPE_Q5_K ? c->ms_p5k : ty == LE_TYPE_Q3_K ? c->ms_p3k : ty == LE_TYPE_IQ2_S ? c->ms_p2s : c->ms_piq;
+    const bool k456 = ty == LE_TYPE_Q4_K || ty == LE_TYPE_Q5_K || ty == LE_TYPE_Q6_K;
+    int NWs = few && c->ms_wide && nsb >= 40 ? 16 : NW, P = pset;
+    if (!pset) {
+        if (!few) P = nsb >= 16 && ty != LE_TYPE_Q8_0 ? 2 : 1;
+        else if (NWs == 16) P = k456 ? 2 : 1;
+        else P = ty == LE_TYPE_Q4_K && nsb >= 2 * NWs && (nsb + 2 * NWs - 1) / (2 * NWs) * 2 <= (nsb + NWs - 1) / NWs + 1 ? 2 : 1;
+    }
     while (P > 1 && nsb % P) P >>= 1;
-    /* keep the waves and give up super-blocks per item when both do not divide K (4096 x 14336, 56
-     * super-blocks, P=1 on 8 waves against P=2 on 4: Q6_K 14.1 against 16.0 us, Q4_K 10.6 / 12.1,
-     * Q4_0 13.6 / 14.0, Q3_K 13.4 / 14.0, IQ2_S 12.7 / 16.1); IQ3_XXS keeps P (15.4 against 20.0
-     * us; its down shapes take the wider split below) */
-    if (ty != LE_TYPE_IQ3_XXS && nsb % (NWs * P) && nsb % NWs == 0) P = 1;
-    /* with no more row tiles than CUs and K of 48 super-blocks or more (a down projection: one tile
-     * per block), K is split over 12-16 waves of two super-blocks each: 4096 x 14336 IQ3_XXS 15.5
-     * -> 12.8 us, IQ2_XXS 12.1 -> 10.9, IQ2_S 13.2 -> 12.5, Q4_0 13.9 -> 10.8, Q4_K 10.6 -> 9.8,
-     * Q5_K 12.4 -> 11.7, Q3_K 13.6 -> 12.4; IQ3_XXS 4096 x 12288 11.9 -> 11.0 (2048 x 8192, 32
-     * super-blocks: 8.2 -> 8.8, so not there); Q6_K 14.3 -> 14.8 and Q8_0 17.0 -> 28.4 lose */
-    if (ty != LE_TYPE_Q6_K && ty != LE_TYPE_Q8_0 && c->ms_wide && (rows + 15) / 16 * (long long)slots <= c->cus && nsb >= 48 && nsb % 2 == 0)
-        for (const int w : {16, 14, 12})
-            if ((nsb / 2) % w == 0) { NWs = w; P = 2; break; }
-    while (NWs > 1 && nsb % (NWs * P)) NWs >>= 1;
-    /* only some (P, NWs) pairs are instantiated (e.g. no P = 4 with 8 waves): lower P until the
-     * kernel exists, else fall through to the unstaged or vector kernels */
-    while (c->ms && P > 1 && !c->fn(std::string("le_ms_") + std::to_string(ty) + "_p" + std::to_string(P) + "_w" +
-                                    std::to_string(NWs) + (xq8 ? "_q8" : "")))
-        P >>= 1;
-    if (c->ms && nsb % (NWs * P) == 0 &&
-        c->fn(std::string("le_ms_") + std::to_string(ty) + "_p" + std::to_string(P) + "_w" + std::to_string(NWs) + (xq8 ? "_q8" : ""))) {
-        const int cps = ty == LE_TYPE_Q6_K ? 14 : ty == LE_TYPE_IQ2_XXS ? 5 : ty == LE_TYPE_IQ3_XXS ? 7 : ty == LE_TYPE_Q8_0 ? 17 : ty == LE_TYPE_Q5_K ? 11 : ty == LE_TYPE_Q3_K ? 7 : ty == LE_TYPE_IQ2_S ? 6 : 9;
-        const int cpr = cps * P + 1, ni = (16 * cpr + 63) / 64;
+    /* Only some (P, NWs) pairs are instantiated (no P = 4 with 8 waves, P = 2 with 16 for the K-quants
+     * only), every wave needs an item, and the waves' images, staging and tables must fit the LDS:
+     * smaller items, then fewer waves, until one does; else the unstaged or vector kernels. */
+    const int cps = ty == LE_TYPE_Q6_K ? 14 : ty == LE_TYPE_IQ2_XXS ? 5 : ty == LE_TYPE_IQ3_XXS ? 7 : ty == LE_TYPE_Q8_0 ? 17 : ty == LE_TYPE_Q5_K ? 11 : ty == LE_TYPE_Q3_K ? 7 : ty == LE_TYPE_IQ2_S ? 6 : 9;
+    const size_t tab = ty == LE_TYPE_IQ2_S ? 9216 : ty == LE_TYPE_IQ2_XXS || ty == LE_TYPE_IQ3_XXS ? 3072 : 0;
+    while (c->ms) {
+        const int cpr = (cps * P) | 1;                   /* 16-byte slots of a staged row */
+        const int most = (nsb / P + NWs - 1) / NWs * P;  /* super-blocks of the wave that has the most */
+        const size_t need = (size_t)NWs * ((size_t)most * 608 + (size_t)cpr * 256 + 128);
         snprintf(name, sizeof name, "le_ms_%d_p%d_w%d%s", ty, P, NWs, xq8 ? "_q8" : "");
-        lds = (size_t)NWs * ((size_t)(nsb / NWs) * 608 + (size_t)ni * 1024) + (size_t)NWs * 128;
-        if (lds <= c->lds_limit)
-            return c->launch(name, dim3((unsigned)gx, (unsigned)slots), NWs * 64, lds, st, args);
-        lds = (size_t)nsb * 608 + (size_t)NW * 64;
+        if (nsb >= NWs * P && need + tab <= c->lds_limit && c->fn(name))
+            return c->launch(name, dim3((unsigned)gx, (unsigned)slots), NWs * 64, need, st, args);
+        if (P > 1) P >>= 1;
+        else if (NWs > 1) NWs >>= 1;
+        else break;
     }
     /* no unstaged MFMA variant for the other types, nor one that forms silu(gate) * up: the caller
      * falls back to the vector kernels */
@@ -316,7 +323,7 @@ int ms_t_launch(le_ctx *c, const void *const *ptrs, const void *w, const float *
     const int ncand = wide ? 4 : 3;
     for (int i = 0; i < ncand; i++) {
         const int P = cand[i][0], NW = cand[i][1];
-        if (P > c->ms_p || nsb % (NW * P)) continue;
+        if (P > (c->ms_p ? c->ms_p : 2) || nsb % (NW * P)) continue;
         const int ni = (16 * (9 * P + 1) + 63) / 64;
         const size_t lds = (size_t)NW * ((size_t)T * (nsb / NW) * 624 + (size_t)ni * 1024) + (size_t)NW * T * 128;
         if (lds > c->lds_limit) continue;
@@ -971,7 +978,7 @@ static int mh_launch(le_ctx *c, const void *w, const float *x, int m, float *y, 
     const int ncand = 4;
     for (int i = 0; i < ncand; i++) {
         const int P = c->gm_mh_shape ? c->gm_mh_shape / 10 : cand[i][0], NW = c->gm_mh_shape ? c->gm_mh_shape % 10 : cand[i][1];
-        if (P > c->ms_p || nsb % (NW * P)) continue;
+        if (P > (c->ms_p ? c->ms_p : 2) || nsb % (NW * P)) continue;
         /* per wave: per super-block T records of 8 x 5 16-byte image slots and 2 sum slots, 64 bytes
          * of scales; the staging of 16 rows x (9P + 1, made odd) slots; the reduction area */
         const int ni = (16 * ((9 * P + 1) | 1) + 63) / 64;

@@ -1064,6 +1064,15 @@ __device__ __forceinline__ float ms_sb_iq2s(const uint4 *sbp, const le_v4i (&A)[
     return h2f(w32[0] & 0xFFFFu) * 0.125f * t;
 }
 
+/* Ragged split of a row's nsb super-blocks over NW waves in items of P: the super-blocks of this
+ * wave (own) and of the wave with the most (most: the LDS image's size for every wave). */
+struct MsSplit {
+    int own, most;
+};
+__device__ __forceinline__ MsSplit ms_split(int nsb, int P, int NW, int wave) {
+    const int items = nsb / P;
+    return {(items + NW - 1 - wave) / NW * P, (items + NW - 1) / NW * P};
+}
 /* Staged variant: each wave streams its tile's P super-blocks per row as consecutive 16-byte
  * chunks (consecutive lanes take consecutive chunks of a row, so every load instruction reads
  * long contiguous runs), prefetched into registers one item ahead and written to a wave-private
@@ -1074,7 +1083,7 @@ template <int P, int NW, bool Q8, int TY = LE_TYPE_Q4_K>
 __device__ __forceinline__ void ms_q4k_body(const MvArgs &a) {
     extern __shared__ uint4 smem[];
     constexpr int CPS = TY == LE_TYPE_Q5_K ? 11 : 9; /* 16-byte chunks per super-block (Q4_K, Q5_K) */
-    constexpr int CPR = CPS * P + 1, NCH = 16 * CPR, NI = (NCH + 63) / 64;
+    constexpr int CPR = (CPS * P) | 1, NCH = 16 * CPS * P, NI = (NCH + 63) / 64;
     const int K = a.cols, nsb = K >> 8;
     const int slot = blockIdx.y;
     const u8 *W = a.ptrs ? a.ptrs[slot] : a.w0 + (size_t)slot * a.w_slot_bytes;
@@ -1082,24 +1091,29 @@ __device__ __forceinline__ void ms_q4k_body(const MvArgs &a) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int n = lane & 15, sq = lane >> 4;
     /* wave-private LDS: the activation image of this wave's super-blocks (local index ls, global
-     * super-block (ls/P)*NW*P + wave*P + ls%P), then the staging buffer; the host guarantees
-     * nsb % (NW*P) == 0 */
-    const int nsbw = nsb / NW;
-    uint4 *rec = smem + wave * (nsbw * 38 + NI * 64);
+     * super-block (ls/P)*NW*P + wave*P + ls%P), then the staging buffer. The host guarantees
+     * nsb % P == 0 and nsb >= NW*P; the K/(256 P) items need not divide over the waves: wave w takes
+     * items w, w + NW, ..., and the first waves then hold one item more (ms_split) */
+    const MsSplit SP = ms_split(nsb, P, NW, wave);
+    const int nsbw = SP.most;
+    uint4 *rec = smem + wave * (nsbw * 38 + 16 * CPR);
     float *dxp = (float *)(rec + nsbw * 32);
     float *fsv = dxp + nsbw * 16;
     uint4 *wb = (uint4 *)(fsv + nsbw * 8);
-    float *red = (float *)(smem + NW * (nsbw * 38 + NI * 64)); /* [2][NW][16] */
+    float *red = (float *)(smem + NW * (nsbw * 38 + 16 * CPR)); /* [2][NW][16] */
     const int ntile = (a.rows + 15) >> 4;
 
-    /* chunk i of this lane: row ri[i] of the tile, byte cb[i] of the row's P-super-block run */
-    int ri[NI], cb[NI];
+    /* chunk i of this lane: row ri[i] of the tile, byte cb[i] of the row's P-super-block run, slot
+     * wl[i] of the staging buffer (rows of an odd number CPR of 16-byte slots, so the 16 rows of a
+     * read lie in distinct banks; an even count folded them onto a half to an eighth of the
+     * banks: IQ3_XXS with 8 slots at P = 1, 14336x4096: 20.9 us, with 7 slots 12.1) */
+    int ri[NI], cb[NI], wl[NI];
 #pragma unroll
     for (int i = 0; i < NI; i++) {
         const int c = min(64 * i + lane, NCH - 1);
-        const int col = c % CPR;
-        ri[i] = c / CPR;
-        cb[i] = (col == CPS * P ? 0 : col) * 16;
+        ri[i] = c / (CPS * P);
+        cb[i] = c % (CPS * P) * 16;
+        wl[i] = c + (CPR - CPS * P) * ri[i];
     }
     /* register staging: the chunks of the next item are loaded while the current one computes */
     uint4 R[NI];
@@ -1115,7 +1129,7 @@ __device__ __forceinline__ void ms_q4k_body(const MvArgs &a) {
     /* activations of the first segment round go out first (clamped, unpredicated), then the
      * first weight item, so the quantization waits only for the activations */
     const float *xs = a.x + a.x_slot * slot;
-    const int nsegw = nsbw * 16;
+    const int nsegw = SP.own * 16;
     auto gseg = [&](int el) { /* local segment -> global segment */
         const int ls = el >> 4;
         return ((ls / P) * sstep + sfirst + ls % P) * 16 + (el & 15);
@@ -1152,7 +1166,7 @@ __device__ __forceinline__ void ms_q4k_body(const MvArgs &a) {
                 int nt = tile, ns = s0 + sstep;
                 if (ns >= nsb) { ns = sfirst; nt += gridDim.x; }
 #pragma unroll
-                for (int i = 0; i < NI; i++) wb[64 * i + lane] = R[i];
+                for (int i = 0; i < NI; i++) wb[wl[i]] = R[i];
                 if (nt < ntile) issue(nt, ns);
 #pragma unroll
                 for (int q = 0; q < P; q++) {
@@ -1378,19 +1392,20 @@ template <int P, int NW, bool Q8, int TY = LE_TYPE_Q6_K>
 __device__ __forceinline__ void ms_q6k_body(const MvArgs &a) {
     extern __shared__ uint4 smem[];
     constexpr bool Q3 = TY == LE_TYPE_Q3_K, S2 = TY == LE_TYPE_IQ2_S;
-    constexpr int CPS = Q3 ? 7 : S2 ? 6 : 14, SBB = Q3 ? 110 : S2 ? 82 : 210, CPR = CPS * P + 1, NCH = 16 * CPR, NI = (NCH + 63) / 64;
+    constexpr int CPS = Q3 ? 7 : S2 ? 6 : 14, SBB = Q3 ? 110 : S2 ? 82 : 210, CPR = (CPS * P) | 1, NCH = 16 * CPS * P, NI = (NCH + 63) / 64;
     const int K = a.cols, nsb = K >> 8;
     const int slot = blockIdx.y;
     const u8 *W = a.ptrs ? a.ptrs[slot] : a.w0 + (size_t)slot * a.w_slot_bytes;
     const size_t rb = (size_t)nsb * SBB;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int n = lane & 15, sq = lane >> 4;
-    const int nsbw = nsb / NW;
-    uint4 *rec = smem + wave * (nsbw * 38 + NI * 64);
+    const MsSplit SP = ms_split(nsb, P, NW, wave);
+    const int nsbw = SP.most;
+    uint4 *rec = smem + wave * (nsbw * 38 + 16 * CPR);
     float *dxp = (float *)(rec + nsbw * 32);
     float *fsv = dxp + nsbw * 16;
     uint4 *wb = (uint4 *)(fsv + nsbw * 8);
-    float *red = (float *)(smem + NW * (nsbw * 38 + NI * 64)); /* [2][NW][16] */
+    float *red = (float *)(smem + NW * (nsbw * 38 + 16 * CPR)); /* [2][NW][16] */
     const int ntile = (a.rows + 15) >> 4;
     __shared__ u32 tab[S2 ? LE_TAB_GRID + 2048 : 1]; /* IQ2_S: sign masks and the 1024-entry grid */
     if constexpr (S2) {
@@ -1398,14 +1413,15 @@ __device__ __forceinline__ void ms_q6k_body(const MvArgs &a) {
         __syncthreads();
     }
 
-    /* chunk i of this lane: row ri[i] of the tile, global byte gb[i] and LDS chunk index of the
-     * row's P-super-block run (the pad chunk re-reads chunk 0) */
-    int ri[NI], gb[NI];
+    /* chunk i of this lane: row ri[i] of the tile, global byte gb[i] of the row's P-super-block run,
+     * staging slot wl[i] (ms_q4k_body) */
+    int ri[NI], gb[NI], wl[NI];
 #pragma unroll
     for (int i = 0; i < NI; i++) {
         const int c = min(64 * i + lane, NCH - 1);
-        const int col = c % CPR, cc = col == CPS * P ? 0 : col;
-        ri[i] = c / CPR;
+        const int cc = c % (CPS * P);
+        ri[i] = c / (CPS * P);
+        wl[i] = c + (CPR - CPS * P) * ri[i];
         gb[i] = (cc / CPS) * SBB + (Q3 ? q3_goff(cc % CPS) : S2 ? i2s_goff(cc % CPS) : q6_goff(cc % CPS));
     }
     uint4 R[NI];
@@ -1419,7 +1435,7 @@ __device__ __forceinline__ void ms_q6k_body(const MvArgs &a) {
     const int sfirst = wave * P, sstep = NW * P;
     const bool active = sfirst < nsb;
     const float *xs = a.x + a.x_slot * slot;
-    const int nsegw = nsbw * 16;
+    const int nsegw = SP.own * 16;
     auto gseg = [&](int el) {
         const int ls = el >> 4;
         return ((ls / P) * sstep + sfirst + ls % P) * 16 + (el & 15);
@@ -1456,7 +1472,7 @@ __device__ __forceinline__ void ms_q6k_body(const MvArgs &a) {
                 int nt = tile, ns = s0 + sstep;
                 if (ns >= nsb) { ns = sfirst; nt += gridDim.x; }
 #pragma unroll
-                for (int i = 0; i < NI; i++) wb[64 * i + lane] = R[i];
+                for (int i = 0; i < NI; i++) wb[wl[i]] = R[i];
                 if (nt < ntile) issue(nt, ns);
 #pragma unroll
                 for (int q = 0; q < P; q++) {
@@ -1612,7 +1628,7 @@ template <int TY, int P, int NW, bool Q8>
 __device__ __forceinline__ void ms_iq_body(const MvArgs &a) {
     using F = MsIq<TY>;
     extern __shared__ uint4 smem[];
-    constexpr int CPS = F::CPS, CPR = CPS * P + 1, NCH = 16 * CPR, NI = (NCH + 63) / 64;
+    constexpr int CPS = F::CPS, CPR = (CPS * P) | 1, NCH = 16 * CPS * P, NI = (NCH + 63) / 64;
     __shared__ u32 tab[256 + 512];
     load_tables<TY>(tab);
     const int K = a.cols, nsb = K >> 8;
@@ -1621,19 +1637,21 @@ __device__ __forceinline__ void ms_iq_body(const MvArgs &a) {
     const size_t rb = (size_t)nsb * F::SBB;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int n = lane & 15;
-    const int nsbw = nsb / NW;
-    uint4 *rec = smem + wave * (nsbw * 38 + NI * 64);
+    const MsSplit SP = ms_split(nsb, P, NW, wave);
+    const int nsbw = SP.most;
+    uint4 *rec = smem + wave * (nsbw * 38 + 16 * CPR);
     float *dxp = (float *)(rec + nsbw * 32);
     float *fsv = dxp + nsbw * 16;
     uint4 *wb = (uint4 *)(fsv + nsbw * 8);
-    float *red = (float *)(smem + NW * (nsbw * 38 + NI * 64)); /* [2][NW][16] */
+    float *red = (float *)(smem + NW * (nsbw * 38 + 16 * CPR)); /* [2][NW][16] */
     const int ntile = (a.rows + 15) >> 4;
-    int ri[NI], gb[NI];
+    int ri[NI], gb[NI], wl[NI];
 #pragma unroll
     for (int i = 0; i < NI; i++) {
         const int c = min(64 * i + lane, NCH - 1);
-        const int col = c % CPR, cc = col == CPS * P ? 0 : col;
-        ri[i] = c / CPR;
+        const int cc = c % (CPS * P);
+        ri[i] = c / (CPS * P);
+        wl[i] = c + (CPR - CPS * P) * ri[i];
         gb[i] = (cc / CPS) * F::SBB + F::goff(cc % CPS);
     }
     uint4 R[NI];
@@ -1647,7 +1665,7 @@ __device__ __forceinline__ void ms_iq_body(const MvArgs &a) {
     const int sfirst = wave * P, sstep = NW * P;
     const bool active = sfirst < nsb;
     const float *xs = a.x + a.x_slot * slot;
-    const int nsegw = nsbw * 16;
+    const int nsegw = SP.own * 16;
     auto gseg = [&](int el) {
         const int ls = el >> 4;
         return ((ls / P) * sstep + sfirst + ls % P) * 16 + (el & 15);
@@ -1683,7 +1701,7 @@ __device__ __forceinline__ void ms_iq_body(const MvArgs &a) {
                 int nt = tile, ns = s0 + sstep;
                 if (ns >= nsb) { ns = sfirst; nt += gridDim.x; }
 #pragma unroll
-                for (int i = 0; i < NI; i++) wb[64 * i + lane] = R[i];
+                for (int i = 0; i < NI; i++) wb[wl[i]] = R[i];
                 if (nt < ntile) issue(nt, ns);
 #pragma unroll
                 for (int q = 0; q < P; q++) {
@@ -1730,7 +1748,7 @@ __device__ __forceinline__ void ms_iq_body(const MvArgs &a) {
 LE_MV_ALL(LE_PART_MV)
 #if LE_PART_MV == 12
 LE_MQ12(4, 1) LE_MQ12(4, 2) LE_MQ12(4, 4) LE_MQ12(8, 1) LE_MQ12(8, 2) LE_MQ12(8, 4) LE_MQ12(2, 1) LE_MQ12(2, 2) LE_MQ12(2, 4)
-LE_MS12(2, 12) LE_MS12(2, 14) LE_MS12(2, 16) LE_MS12(1, 1) LE_MS12(1, 2) LE_MS12(1, 4) LE_MS12(1, 8) LE_MS12(2, 1) LE_MS12(2, 2) LE_MS12(2, 4) LE_MS12(2, 8) LE_MS12(4, 1) LE_MS12(4, 2) LE_MS12(4, 4)
+LE_MS12(1, 16) LE_MS12(2, 16) LE_MS12(1, 1) LE_MS12(1, 2) LE_MS12(1, 4) LE_MS12(1, 8) LE_MS12(2, 1) LE_MS12(2, 2) LE_MS12(2, 4) LE_MS12(2, 8) LE_MS12(4, 1) LE_MS12(4, 2) LE_MS12(4, 4)
 LE_MS12T(1, 4, 2) LE_MS12T(1, 4, 4) LE_MS12T(1, 4, 8) LE_MS12T(1, 8, 2) LE_MS12T(1, 8, 4) LE_MS12T(1, 8, 8)
 LE_MS12T(2, 4, 2) LE_MS12T(2, 4, 4) LE_MS12T(2, 4, 8) LE_MS12T(2, 2, 2) LE_MS12T(2, 2, 4) LE_MS12T(2, 2, 8)
 #endif
@@ -1738,30 +1756,27 @@ LE_MS12T(2, 4, 2) LE_MS12T(2, 4, 4) LE_MS12T(2, 4, 8) LE_MS12T(2, 2, 2) LE_MS12T
 #define LE_MS13(P, NW)                                                                                     \
     extern "C" __global__ void __launch_bounds__(NW * 64) le_ms_13_p##P##_w##NW(MvArgs a) { ms_q4k_body<P, NW, false, LE_TYPE_Q5_K>(a); } \
     extern "C" __global__ void __launch_bounds__(NW * 64) le_ms_13_p##P##_w##NW##_q8(MvArgs a) { ms_q4k_body<P, NW, true, LE_TYPE_Q5_K>(a); }
-LE_MS13(2, 12) LE_MS13(2, 14) LE_MS13(2, 16) LE_MS13(1, 1) LE_MS13(1, 2) LE_MS13(1, 4) LE_MS13(1, 8) LE_MS13(2, 1) LE_MS13(2, 2) LE_MS13(2, 4) LE_MS13(2, 8) LE_MS13(4, 1) LE_MS13(4, 2) LE_MS13(4, 4)
+LE_MS13(1, 16) LE_MS13(2, 16) LE_MS13(1, 1) LE_MS13(1, 2) LE_MS13(1, 4) LE_MS13(1, 8) LE_MS13(2, 1) LE_MS13(2, 2) LE_MS13(2, 4) LE_MS13(2, 8) LE_MS13(4, 1) LE_MS13(4, 2) LE_MS13(4, 4)
 #endif
 #if LE_PART_MV == 11
 #define LE_MS11(P, NW)                                                                                     \
     extern "C" __global__ void __launch_bounds__(NW * 64) le_ms_11_p##P##_w##NW(MvArgs a) { ms_q6k_body<P, NW, false, LE_TYPE_Q3_K>(a); } \
     extern "C" __global__ void __launch_bounds__(NW * 64) le_ms_11_p##P##_w##NW##_q8(MvArgs a) { ms_q6k_body<P, NW, true, LE_TYPE_Q3_K>(a); }
-LE_MS11(2, 12) LE_MS11(2, 14) LE_MS11(2, 16) LE_MS11(1, 1) LE_MS11(1, 2) LE_MS11(1, 4) LE_MS11(1, 8) LE_MS11(2, 1) LE_MS11(2, 2) LE_MS11(2, 4) LE_MS11(2, 8) LE_MS11(4, 1) LE_MS11(4, 2) LE_MS11(4, 4)
+LE_MS11(1, 16) LE_MS11(1, 1) LE_MS11(1, 2) LE_MS11(1, 4) LE_MS11(1, 8) LE_MS11(2, 1) LE_MS11(2, 2) LE_MS11(2, 4) LE_MS11(2, 8) LE_MS11(4, 1) LE_MS11(4, 2) LE_MS11(4, 4)
 #endif
 #if LE_PART_MV == 22
 #define LE_MS22(P, NW)                                                                                     \
     extern "C" __global__ void __launch_bounds__(NW * 64) le_ms_22_p##P##_w##NW(MvArgs a) { ms_q6k_body<P, NW, false, LE_TYPE_IQ2_S>(a); } \
     extern "C" __global__ void __launch_bounds__(NW * 64) le_ms_22_p##P##_w##NW##_q8(MvArgs a) { ms_q6k_body<P, NW, true, LE_TYPE_IQ2_S>(a); }
-LE_MS22(2, 12) LE_MS22(2, 14) LE_MS22(2, 16) LE_MS22(1, 1) LE_MS22(1, 2) LE_MS22(1, 4) LE_MS22(1, 8) LE_MS22(2, 1) LE_MS22(2, 2) LE_MS22(2, 4) LE_MS22(2, 8) LE_MS22(4, 1) LE_MS22(4, 2) LE_MS22(4, 4)
+LE_MS22(1, 16) LE_MS22(1, 1) LE_MS22(1, 2) LE_MS22(1, 4) LE_MS22(1, 8) LE_MS22(2, 1) LE_MS22(2, 2) LE_MS22(2, 4) LE_MS22(2, 8) LE_MS22(4, 1) LE_MS22(4, 2) LE_MS22(4, 4)
 #endif
 #if LE_PART_MV == 14
-LE_MS14(1, 1) LE_MS14(1, 2) LE_MS14(1, 4) LE_MS14(1, 8) LE_MS14(2, 1) LE_MS14(2, 2) LE_MS14(2, 4) LE_MS14(2, 8) LE_MS14(4, 1) LE_MS14(4, 2)
+LE_MS14(1, 16) LE_MS14(2, 16) LE_MS14(1, 1) LE_MS14(1, 2) LE_MS14(1, 4) LE_MS14(1, 8) LE_MS14(2, 1) LE_MS14(2, 2) LE_MS14(2, 4) LE_MS14(2, 8) LE_MS14(4, 1) LE_MS14(4, 2)
 #endif
 #if LE_PART_MV == 16 || LE_PART_MV == 18 || LE_PART_MV == 8 || LE_PART_MV == 2
 LE_MSIQ(LE_PART_MV, 1, 1) LE_MSIQ(LE_PART_MV, 1, 2) LE_MSIQ(LE_PART_MV, 1, 4) LE_MSIQ(LE_PART_MV, 2, 1) LE_MSIQ(LE_PART_MV, 2, 2)
 LE_MSIQ(LE_PART_MV, 2, 4) LE_MSIQ(LE_PART_MV, 4, 1) LE_MSIQ(LE_PART_MV, 4, 2) LE_MSIQ(LE_PART_MV, 4, 4)
-LE_MSIQ(LE_PART_MV, 1, 8) LE_MSIQ(LE_PART_MV, 2, 8)
-#if LE_PART_MV == 18 || LE_PART_MV == 16 || LE_PART_MV == 2 /* down-projection shapes: one row tile per block, K split over 12-16 waves */
-LE_MSIQ(LE_PART_MV, 2, 12) LE_MSIQ(LE_PART_MV, 2, 14) LE_MSIQ(LE_PART_MV, 2, 16)
-#endif
+LE_MSIQ(LE_PART_MV, 1, 8) LE_MSIQ(LE_PART_MV, 2, 8) LE_MSIQ(LE_PART_MV, 1, 16)
 #endif
 #endif
 
