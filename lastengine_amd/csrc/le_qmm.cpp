@@ -16,6 +16,7 @@
 #include <cstring>
 #include <map>
 #include <string>
+#include <tuple>
 #include <vector>
 
 #include "../../include/le_qmm.h"
@@ -113,7 +114,7 @@ struct le_ctx {
                                      decode calls against the grouped form: 10 tokens 99.6 / 102.3 us, 12 tokens
                                      116.8 / 109.0, 14 tokens 128.5 / 112.9, 16 tokens 117.7 / 116.8) */
     int moe_dn_split = 0;    /* down launch blocks per row tile: 0 auto, 1, 2 */
-    std::map<std::string, int> occ; /* resident blocks per CU, by kernel name and LDS bytes */
+    std::map<std::tuple<hipFunction_t, int, size_t>, int> occ; /* resident blocks per CU, by kernel, block and LDS bytes */
     int gm_min_m = 5;        /* le_gemm uses the MFMA GEMM from this many tokens on (below: the
                                 staged matvec with 2..4 tokens per pass, faster there) */
     int gm_tile = 0;         /* MFMA GEMM tile: 0 auto, else 10*TM + TN (TM, TN in 1..2) */
@@ -148,27 +149,46 @@ struct le_ctx {
         if (e == hipSuccess) return LE_OK;
         return fail(LE_ERR_HIP, "%s: %s", what, hipGetErrorString(e));
     }
-    hipFunction_t fn(const std::string &name) {
+    /* Kernel by name (null where no code object has it). A launch looks its kernel up once or twice, so
+     * the names seen last sit in a direct-mapped table (no allocation, one hash and compare) in front of
+     * the map, which also remembers the names that do not exist. */
+    struct FnSlot {
+        char name[56];
+        hipFunction_t f;
+    };
+    FnSlot slots[256] = {};
+    hipFunction_t fn(const char *name) {
+        unsigned h = 2166136261u;
+        size_t n = 0;
+        for (; name[n]; n++) h = (h ^ (unsigned char)name[n]) * 16777619u;
+        FnSlot &s = slots[(h ^ (h >> 16)) & 255u];
+        if (n < sizeof s.name && s.f && !strcmp(s.name, name)) return s.f;
+        hipFunction_t f = nullptr;
         auto it = fns.find(name);
-        if (it != fns.end()) return it->second;
-        for (hipModule_t m : mods) {
-            hipFunction_t f = nullptr;
-            const hipError_t e = hipModuleGetFunction(&f, m, name.c_str());
-            /* a miss in one module must not leave a sticky error behind for the caller */
-            (void)hipGetLastError();
-            if (e == hipSuccess && f) {
-                fns[name] = f;
-                return f;
+        if (it != fns.end()) {
+            f = it->second;
+        } else {
+            for (hipModule_t m : mods) {
+                const hipError_t e = hipModuleGetFunction(&f, m, name);
+                /* a miss in one module must not leave a sticky error behind for the caller */
+                (void)hipGetLastError();
+                if (e == hipSuccess && f) break;
+                f = nullptr;
             }
+            fns[name] = f;
         }
-        return nullptr;
+        if (f && n < sizeof s.name) {
+            memcpy(s.name, name, n + 1);
+            s.f = f;
+        }
+        return f;
     }
     /* resident blocks per CU of kernel `name` at this block size and dynamic LDS (0 if unknown) */
-    int blocks_per_cu(const std::string &name, int block, size_t lds) {
-        const std::string key = name + "/" + std::to_string(block) + "/" + std::to_string(lds);
+    int blocks_per_cu(const char *name, int block, size_t lds) {
+        hipFunction_t f = fn(name);
+        const auto key = std::make_tuple(f, block, lds);
         auto it = occ.find(key);
         if (it != occ.end()) return it->second;
-        hipFunction_t f = fn(name);
         int per_cu = 0;
         if (!f || hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, f, block, lds) != hipSuccess) {
             (void)hipGetLastError();
@@ -177,11 +197,10 @@ struct le_ctx {
         occ[key] = per_cu;
         return per_cu;
     }
-    int launch(const std::string &name, dim3 grid, int block, size_t lds, hipStream_t st, void **args) {
+    int launch(const char *name, dim3 grid, int block, size_t lds, hipStream_t st, void **args) {
         hipFunction_t f = fn(name);
-        if (!f) return fail(LE_ERR_MODULE, "kernel %s not found in the loaded code objects", name.c_str());
-        return hip(hipModuleLaunchKernel(f, grid.x, grid.y, grid.z, block, 1, 1, (unsigned)lds, st, args, nullptr),
-                   name.c_str());
+        if (!f) return fail(LE_ERR_MODULE, "kernel %s not found in the loaded code objects", name);
+        return hip(hipModuleLaunchKernel(f, grid.x, grid.y, grid.z, block, 1, 1, (unsigned)lds, st, args, nullptr), name);
     }
 };
 
