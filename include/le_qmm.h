@@ -94,9 +94,12 @@ const char *le_last_error(const le_ctx *ctx);
  *     "gq_min_m" smallest M of the other types on the matrix-core GEMM (below: vector kernels that
  *     read the weights once per 8 tokens), "gq_cfg" its block shape (0 auto; 1..10: 32x256, 64x256,
  *     128x256, 128x128 tokens x rows on 4 waves, 64x256, 128x256, 32x256 on 8 waves, 64x128, 32x128,
- *     128x128 on 4 waves; Q4_K only, 2 x 4 waves: 11 128x256, 12 128x128), "gq_ksplit" its K
+ *     128x128 on 4 waves; Q4_K only, 2 x 4 waves: 11 128x256, 12 128x128; Q4_K and Q5_K with 256 rows
+ *     or more, the pipelined kernel: 21 128x256, 22 64x256), "gq_ksplit" its K
  *     slices (0 auto, 1, 2, 4, 8); "mmg_xw" (0/1) the grouped form's activation pre-pass one wave
  *     per pair from 256 pairs when K <= 4096 (default) or one block per pair (same results);
+ *     "mmg_gp" (0/1) grouped 64- and 128-pair tiles of Q4_K / Q5_K on the pipelined kernel (default) or
+ *     on the generic one (the sums differ by fp32 rounding);
  *     "mmg_w4" (0/1) grouped 32-pair tiles of Q6_K / Q8_0 / Q4_0 on 4-wave 32x128 blocks (default)
  *     or 8-wave 32x256 ones (same results);
  *     "moe_route1" (0/1) the grouped MoE's routing and grouping in one block up to 32 tokens

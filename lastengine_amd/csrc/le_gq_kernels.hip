@@ -25,7 +25,7 @@
  * take consecutive chunks of a row) into a 16-byte-aligned LDS slot of F::SLOT bytes, then each
  * lane builds its B fragments from them:
  *   Q4_K   code sc_j * q (<= 945, exact), offset term D2 = sum_j m_j S_j (one more MFMA per
- *          super-block), epilogue  acc += d * D1 - dmin * D2                 (src/quant.rs:72-82)
+ *          super-block), acc = acc (d' / d) + D1 - (dmin / d) D2, in units of d    (src/quant.rs:72-82)
  *   Q6_K   code (q6 - 32) * sc_u / 64 (exact where (q6 - 32) sc_u has at most 11 significant
  *          bits, else rounded once to fp16), epilogue acc += 64 d * D1           (:96-112)
  *   IQ2_XXS code (2s+1) * grid * sign (<= 1333, exact), epilogue acc += d/8 * D1   (:142-154)
@@ -180,11 +180,11 @@ __device__ __forceinline__ void gq_barrier() {
 }
 
 template <int TM, int TN>
-__device__ __forceinline__ void gq_mma(le_v16f (&d)[TM][TN], const le_v8h (&A)[TM], const le_v8h (&B)[TN], bool zero) {
+__device__ __forceinline__ void gq_mma(le_v16f (&d)[TM][TN], const le_v8h (&A)[TM], const le_v8h (&B)[TN]) {
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
-        for (int k = 0; k < TN; k++) d[i][k] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[i], B[k], zero ? (le_v16f){} : d[i][k], 0, 0, 0);
+        for (int k = 0; k < TN; k++) d[i][k] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[i], B[k], d[i][k], 0, 0, 0);
 }
 
 /* ============================ per-type formats ============================
@@ -199,6 +199,7 @@ struct GqF<LE_TYPE_Q4_K> { /* slot: [0,16) header, [16,80) this half's 64 quant 
     static constexpr int SBB = 144, NCH = 5, SLOT = 80, SREC = 1024, EPI = 1, TAB = 0;
     static constexpr bool ALIGNED = true;
     __device__ static int goff(int k, int h) { return k == 0 ? 0 : 16 + 64 * h + 16 * (k - 1); }
+    __device__ static float scale(const u8 *r) { return h2f(*(const uint16_t *)r); }
     __device__ static int loff(int k) { return 16 * k; }
 };
 template <>
@@ -209,6 +210,7 @@ struct GqF<LE_TYPE_Q6_K> { /* slot: [0,64) ql half, [64,96) qh half, [96,112) sc
     __device__ static int goff(int k, int h) {
         return k < 4 ? 64 * h + 16 * k : k < 6 ? 128 + 32 * h + 16 * (k - 4) : k == 6 ? 192 : 194;
     }
+    __device__ static float scale(const u8 *r) { return 64.f * h2f(*(const uint16_t *)(r + 126)); }
     __device__ static int loff(int k) { return 16 * k; }
 };
 template <>
@@ -216,6 +218,7 @@ struct GqF<LE_TYPE_Q5_K> { /* slot: [0,16) header, [16,48) qh (all 32 bytes), [4
     static constexpr int SBB = 176, NCH = 7, SLOT = 112, SREC = 1024, EPI = 1, TAB = 0;
     static constexpr bool ALIGNED = true;
     __device__ static int goff(int k, int h) { return k < 3 ? 16 * k : 48 + 64 * h + 16 * (k - 3); }
+    __device__ static float scale(const u8 *r) { return h2f(*(const uint16_t *)r); }
     __device__ static int loff(int k) { return 16 * k; }
 };
 template <>
@@ -224,6 +227,7 @@ struct GqF<LE_TYPE_Q3_K> { /* slot: [0,32) the half's 32 quant bytes, [32,64) hm
     static constexpr int SBB = 110, NCH = 5, SLOT = 80, SREC = 0, EPI = 1, TAB = 0;
     static constexpr bool ALIGNED = false;
     __device__ static int goff(int k, int h) { return k < 2 ? 32 + 32 * h + 16 * k : k < 4 ? 16 * (k - 2) : 94; }
+    __device__ static float scale(const u8 *r) { return h2f(*(const uint16_t *)(r + 78)); }
     __device__ static int loff(int k) { return 16 * k; }
 };
 template <>
@@ -232,6 +236,7 @@ struct GqF<LE_TYPE_IQ2_S> { /* slot: [0,16) the half's grid index bytes, [16,32)
     static constexpr int SBB = 82, NCH = 4, SLOT = 80, SREC = 0, EPI = 1, TAB = 16384 + 4096;
     static constexpr bool ALIGNED = false;
     __device__ static int goff(int k, int h) { return k == 0 ? 2 + 16 * h : k == 1 ? 34 + 16 * h : k == 2 ? 66 : 0; }
+    __device__ static float scale(const u8 *r) { return 0.125f * h2f(*(const uint16_t *)(r + 48)); }
     __device__ static int loff(int k) { return 16 * k; }
 };
 template <>
@@ -240,6 +245,7 @@ struct GqF<LE_TYPE_Q4_0> { /* 8 blocks of 18 bytes form a 144-byte super-block; 
     static constexpr int SBB = 144, NCH = 8, SLOT = 144, SREC = 0, EPI = 2, TAB = 0;
     static constexpr bool ALIGNED = false;
     __device__ static int goff(int k, int h) { return k < 4 ? 72 * h + 18 * k + 2 : 72 * h + 18 * (k - 4); }
+    __device__ static float scale(const u8 *r) { return 1.f; }
     __device__ static int loff(int k) { return 16 * k; }
 };
 template <>
@@ -249,6 +255,7 @@ struct GqF<LE_TYPE_Q8_0> { /* slot: [32b, 32b+32) quants of block b of the half,
     __device__ static int goff(int k, int h) {
         return k < 8 ? 136 * h + 34 * (k >> 1) + 2 + 16 * (k & 1) : 136 * h + 34 * (k - 8);
     }
+    __device__ static float scale(const u8 *r) { return 1.f; }
     __device__ static int loff(int k) { return 16 * k; }
 };
 template <>
@@ -256,6 +263,7 @@ struct GqF<LE_TYPE_IQ2_XXS> { /* slot: [0,32) the half's four 8-byte block recor
     static constexpr int SBB = 66, NCH = 3, SLOT = 48, SREC = 0, EPI = 1, TAB = 4096 + 2048;
     static constexpr bool ALIGNED = false;
     __device__ static int goff(int k, int h) { return k < 2 ? 2 + 32 * h + 16 * k : 0; }
+    __device__ static float scale(const u8 *r) { return 0.125f * h2f(*(const uint16_t *)(r + 32)); }
     __device__ static int loff(int k) { return 16 * k; }
 };
 template <>
@@ -264,6 +272,7 @@ struct GqF<LE_TYPE_IQ3_XXS> { /* slot: [0,32) the half's grid indices, [32,48) i
     static constexpr int SBB = 98, NCH = 4, SLOT = 80, SREC = 0, EPI = 1, TAB = 2048 + 2048;
     static constexpr bool ALIGNED = false;
     __device__ static int goff(int k, int h) { return k < 2 ? 2 + 32 * h + 16 * k : k == 2 ? 66 + 16 * h : 0; }
+    __device__ static float scale(const u8 *r) { return 0.25f * h2f(*(const uint16_t *)(r + 48)); }
     __device__ static int loff(int k) { return 16 * k; }
 };
 
@@ -533,6 +542,76 @@ __device__ __forceinline__ void gq_vm_wait() {
 }
 __device__ __forceinline__ u32 gq_lds_addr(const void *p) { return (u32)(size_t)(const __attribute__((address_space(3))) void *)p; }
 
+/* End of a block's tile: acc times the token scales into y, the K slice's partial results or (neither)
+ * atomically added into y. LDSB: bytes of LDS that may be overwritten; rows below rmin are left out. */
+template <int WM, int WN, int TM, int TN, bool GR, int LDSB>
+__device__ __forceinline__ void gq_store(const GqArgs &a, u8 *lds, const float *tsc, const le_v16f (&acc)[TM][TN], int M, int mb,
+                                         int nb, int pair0, bool second, int rmin = 0) {
+    constexpr int BN = 32 * TN * WN, NT = 64 * WM * WN;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wm = wave / WN, wn = wave % WN;
+    const int n = lane & 31, hs = lane >> 5;
+    /* D lane l element e: token 8 (e / 4) + 4 (l / 32) + e % 4 of the tile, row l % 32; the
+     * token scales of the padded tile are all loaded first (one memory round trip) */
+    float ts[TM][16];
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int e = 0; e < 16; e++) ts[i][e] = tsc[mb + (wm * TM + i) * 32 + 4 * hs + 8 * (e >> 2) + (e & 3)];
+    if (!GR && a.ksplit > 1 && !a.part) { /* K slices without a partial-result buffer: atomic adds */
+#pragma unroll
+        for (int i = 0; i < TM; i++) {
+            const int t0 = mb + (wm * TM + i) * 32 + 4 * hs;
+#pragma unroll
+            for (int k = 0; k < TN; k++) {
+                const int r = nb + (wn * TN + k) * 32 + n;
+#pragma unroll
+                for (int e = 0; e < 16; e++) {
+                    const int t = t0 + 8 * (e >> 2) + (e & 3);
+                    if (t < M && r >= rmin && r < a.rows) unsafeAtomicAdd(a.y + (size_t)t * a.rows + r, acc[i][k][e] * ts[i][e]);
+                }
+            }
+        }
+        return;
+    }
+    /* Stores through LDS, one 32-token tile of every wave row at a time: the waves place their
+     * results as [token][row] (row stride BN + 8 floats: the two 4-token halves of a fragment fall
+     * on different banks), then each token's BN outputs leave as 16-byte stores of consecutive
+     * rows (a wave covers 1 KB of one output row) instead of 4-byte stores 32 to a row. */
+    float *dst = (!GR && a.ksplit > 1) ? a.part + (size_t)blockIdx.y * a.m * a.rows : second ? a.y2 : a.y;
+    constexpr int TS = BN + 8, NQ = BN / 4;
+    static_assert((size_t)WM * 32 * TS * 4 <= (size_t)LDSB, "output staging must fit the step buffers");
+    float *T = (float *)lds;
+    const bool vec = (a.rows & 3) == 0 && ((size_t)dst & 15) == 0;
+#pragma unroll
+    for (int i = 0; i < TM; i++) {
+        __syncthreads(); /* the step buffers (or the previous round) are no longer read */
+#pragma unroll
+        for (int k = 0; k < TN; k++) {
+            const int rl = (wn * TN + k) * 32 + n;
+#pragma unroll
+            for (int e = 0; e < 16; e++)
+                T[(wm * 32 + 4 * hs + 8 * (e >> 2) + (e & 3)) * TS + rl] = acc[i][k][e] * ts[i][e];
+        }
+        __syncthreads();
+        for (int c = tid; c < WM * 32 * NQ; c += NT) {
+            const int tl = c / NQ, q = c - tl * NQ;
+            const int t = mb + ((tl >> 5) * TM + i) * 32 + (tl & 31), r = nb + 4 * q;
+            if (t >= M || r >= a.rows) continue;
+            int o = t;
+            if constexpr (GR) o = a.out_idx[pair0 + t - mb];
+            const float4 v = *(const float4 *)(T + tl * TS + 4 * q);
+            float *yp = dst + (size_t)o * a.rows + r;
+            if (vec && r >= rmin && r + 3 < a.rows) {
+                *(float4 *)yp = v;
+            } else {
+                const float vv[4] = {v.x, v.y, v.z, v.w};
+                for (int u = 0; u < 4 && r + u < a.rows; u++)
+                    if (r + u >= rmin) yp[u] = vv[u];
+            }
+        }
+    }
+}
+
 /* ============================ main kernel ============================ */
 /* NA > 0: the activation fragments go straight to LDS, a ring of NA step slots (2: loaded one
  * step ahead, issued as the step starts, in the LDS the register-staged form uses for them; 3:
@@ -680,16 +759,22 @@ __device__ __forceinline__ void gq_body(const GqArgs &a, const u8 *ws) {
         }
     };
 
-    le_v16f acc[TM][TN], d1[TM][TN];
+    le_v16f acc[TM][TN];
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
-        for (int k = 0; k < TN; k++) acc[i][k] = d1[i][k] = (le_v16f){};
+        for (int k = 0; k < TN; k++) acc[i][k] = (le_v16f){};
 
     const int n = lane & 31, hs = lane >> 5;
     int rowS[TN]; /* Q8_0 / Q4_0: the accumulator holds the row's sum times 2^rowS */
 #pragma unroll
     for (int k = 0; k < TN; k++) rowS[k] = 127;
+    /* EPI == 1: the accumulator holds the row's sum in units of unit[k], the super-block scale in use;
+     * live[k]: all ones, or zero while the super-block's scale is zero (its codes then count as zero) */
+    float unit[TN];
+    u32 live[TN];
+#pragma unroll
+    for (int k = 0; k < TN; k++) unit[k] = 1.f, live[k] = 0;
     Set RA, RB; /* RA holds odd (h = 1) steps, RB even ones */
     const int s0 = 2 * sb0;
     /* the loads must reach the memory pipeline in step order (RA's before RB's, as in the loop),
@@ -722,11 +807,24 @@ __device__ __forceinline__ void gq_body(const GqArgs &a, const u8 *ws) {
             const u8 *rs[TN];
 #pragma unroll
             for (int k = 0; k < TN; k++) rs[k] = Wb + (wn * TN * 32 + 32 * k + n) * F::SLOT;
-            /* A fragment of tile i, chunk c */
-            auto afrag = [&](int c, le_v8h (&A)[TM]) {
+            /* The step's eight chunks in the order the decoders produce them (Q4_K, Q5_K: low and high
+             * nibbles of the same bytes, chunks c and c + 2, together). The activation fragments of the
+             * next chunk are read while this chunk's MFMAs run (read right before their use, each MFMA
+             * waited out an LDS read). */
+            le_v8h Af[2][TM];
+            auto aload = [&](int p) {
+                constexpr bool PAIR = TY == LE_TYPE_Q4_K || TY == LE_TYPE_Q5_K;
+                const int c = TY == LE_TYPE_Q6_K ? 2 * (p & 3) + (p >> 2) : PAIR ? (p & 4) | ((p & 1) << 1) | ((p >> 1) & 1) : p;
 #pragma unroll
-                for (int i = 0; i < TM; i++) A[i] = as_v8h(*(const uint4 *)(Ab + i * 8192 + c * 1024 + lane * 16));
+                for (int i = 0; i < TM; i++) Af[p & 1][i] = as_v8h(*(const uint4 *)(Ab + i * 8192 + c * 1024 + lane * 16));
             };
+            auto mma = [&](int p, const le_v8h (&B)[TN]) { /* position p of that order */
+                if (p < 7) aload(p + 1);
+                __builtin_amdgcn_sched_barrier(0x016); /* LDS reads stay on their side of the MFMAs; VALU, SALU and VMEM may cross */
+                gq_mma(acc, Af[p & 1], B);
+                __builtin_amdgcn_sched_barrier(0x016);
+            };
+            aload(0);
             /* stage the next step and issue the loads two steps ahead once this step's first
              * fragments are under way */
             auto pipe = [&]() {
@@ -741,6 +839,22 @@ __device__ __forceinline__ void gq_body(const GqArgs &a, const u8 *ws) {
                 if constexpr (NA == 3) dma(s + 2); /* slot (s + 2) % 3 was last read in step s - 1 */
                 __builtin_amdgcn_sched_barrier(0);
             };
+            if (F::EPI == 1 && h == 0) {
+                /* a new super-block scale: one multiplication puts the running sum into its units, so the
+                 * MFMAs accumulate into it directly and a wave needs one accumulator, not a second one
+                 * per super-block */
+#pragma unroll
+                for (int k = 0; k < TN; k++) {
+                    const float d = F::scale(rs[k]);
+                    live[k] = d == 0.f ? 0u : ~0u;
+                    const float r = d == 0.f ? 1.f : unit[k] * __builtin_amdgcn_rcpf(d);
+                    unit[k] = d == 0.f ? unit[k] : d;
+#pragma unroll
+                    for (int i = 0; i < TM; i++)
+#pragma unroll
+                        for (int e = 0; e < 16; e++) acc[i][k][e] *= r;
+                }
+            }
             if constexpr (TY == LE_TYPE_Q4_K) {
                 const u32 mlo = 0x000F000Fu, mhi = 0x00F000F0u, c1024 = 0x64006400u;
                 uint4 hd[TN];
@@ -748,7 +862,7 @@ __device__ __forceinline__ void gq_body(const GqArgs &a, const u8 *ws) {
 #pragma unroll
                 for (int k = 0; k < TN; k++) {
                     hd[k] = *(const uint4 *)rs[k];
-                    scw[k] = h ? ((hd[k].w & 0x0F0F0F0Fu) | ((hd[k].y >> 2) & 0x30303030u)) : (hd[k].y & 0x3F3F3F3Fu);
+                    scw[k] = (h ? ((hd[k].w & 0x0F0F0F0Fu) | ((hd[k].y >> 2) & 0x30303030u)) : (hd[k].y & 0x3F3F3F3Fu)) & live[k];
                 }
 #pragma unroll
                 for (int g = 0; g < 2; g++) {
@@ -761,7 +875,6 @@ __device__ __forceinline__ void gq_body(const GqArgs &a, const u8 *ws) {
                     }
 #pragma unroll
                     for (int c1 = 0; c1 < 2; c1++) {
-                        const int c = 4 * g + c1;
                         le_v8h blo[TN], bhi[TN];
 #pragma unroll
                         for (int k = 0; k < TN; k++) {
@@ -779,11 +892,8 @@ __device__ __forceinline__ void gq_body(const GqArgs &a, const u8 *ws) {
                             blo[k] = as_v8h(make_uint4(l[0], l[1], l[2], l[3]));
                             bhi[k] = as_v8h(make_uint4(hh[0], hh[1], hh[2], hh[3]));
                         }
-                        le_v8h A[TM];
-                        afrag(c, A);
-                        gq_mma(d1, A, blo, h == 0 && c == 0);
-                        afrag(c + 2, A);
-                        gq_mma(d1, A, bhi, false);
+                        mma(4 * g + 2 * c1, blo);
+                        mma(4 * g + 2 * c1 + 1, bhi);
                         if (g == 0 && c1 == 0) pipe();
                     }
                 }
@@ -793,7 +903,7 @@ __device__ __forceinline__ void gq_body(const GqArgs &a, const u8 *ws) {
 #pragma unroll
                 for (int k = 0; k < TN; k++) {
                     const uint2 sv = *(const uint2 *)(rs[k] + 96 + 8 * h);
-                    const u32 sw[2] = {sv.x ^ 0x80808080u, sv.y ^ 0x80808080u};
+                    const u32 sw[2] = {(sv.x & live[k]) ^ 0x80808080u, (sv.y & live[k]) ^ 0x80808080u};
 #pragma unroll
                     for (int c = 0; c < 8; c++)
                         sp[k][c] = pk_mul(pk_add(h1024_dup(sw[c >> 2], c & 3), 0xE480E480u), 0x24002400u); /* (byte - 1152) / 64 */
@@ -825,9 +935,7 @@ __device__ __forceinline__ void gq_body(const GqArgs &a, const u8 *ws) {
                             B[k] = as_v8h(make_uint4(pk_mul(pk_add(h1024_02(vx), 0xE420E420u), sc), pk_mul(pk_add(h1024_13(vx), 0xE420E420u), sc),
                                                      pk_mul(pk_add(h1024_02(vy), 0xE420E420u), sc), pk_mul(pk_add(h1024_13(vy), 0xE420E420u), sc)));
                         }
-                        le_v8h A[TM];
-                        afrag(c, A);
-                        gq_mma(d1, A, B, h == 0 && c == 0);
+                        mma(4 * c1 + q, B);
                         if (c1 == 0 && q == 0) pipe();
                     }
                 }
@@ -888,9 +996,7 @@ __device__ __forceinline__ void gq_body(const GqArgs &a, const u8 *ws) {
                                                          pk_mul(pk_add(h1024_02(y), 0xE408E408u), r[k][b]), pk_mul(pk_add(h1024_13(y), 0xE408E408u), r[k][b])));
                             }
                         }
-                        le_v8h A[TM];
-                        afrag(c, A);
-                        gq_mma(acc, A, B, false);
+                        mma(c, B);
                         if (c == 0) pipe();
                     }
                 }
@@ -901,7 +1007,7 @@ __device__ __forceinline__ void gq_body(const GqArgs &a, const u8 *ws) {
 #pragma unroll
                 for (int k = 0; k < TN; k++) {
                     const uint4 hd = *(const uint4 *)rs[k];
-                    scw[k] = h ? ((hd.w & 0x0F0F0F0Fu) | ((hd.y >> 2) & 0x30303030u)) : (hd.y & 0x3F3F3F3Fu);
+                    scw[k] = (h ? ((hd.w & 0x0F0F0F0Fu) | ((hd.y >> 2) & 0x30303030u)) : (hd.y & 0x3F3F3F3Fu)) & live[k];
                 }
 #pragma unroll
                 for (int g = 0; g < 2; g++) {
@@ -915,7 +1021,6 @@ __device__ __forceinline__ void gq_body(const GqArgs &a, const u8 *ws) {
                     }
 #pragma unroll
                     for (int c1 = 0; c1 < 2; c1++) {
-                        const int c = 4 * g + c1;
                         le_v8h blo[TN], bhi[TN];
 #pragma unroll
                         for (int k = 0; k < TN; k++) {
@@ -930,11 +1035,8 @@ __device__ __forceinline__ void gq_body(const GqArgs &a, const u8 *ws) {
                             bhi[k] = as_v8h(make_uint4(pk_fma(h1024_02(hx), kc[k].z, kc[k].w), pk_fma(h1024_13(hx), kc[k].z, kc[k].w),
                                                        pk_fma(h1024_02(hy), kc[k].z, kc[k].w), pk_fma(h1024_13(hy), kc[k].z, kc[k].w)));
                         }
-                        le_v8h A[TM];
-                        afrag(c, A);
-                        gq_mma(d1, A, blo, h == 0 && c == 0);
-                        afrag(c + 2, A);
-                        gq_mma(d1, A, bhi, false);
+                        mma(4 * g + 2 * c1, blo);
+                        mma(4 * g + 2 * c1 + 1, bhi);
                         if (g == 0 && c1 == 0) pipe();
                     }
                 }
@@ -952,7 +1054,7 @@ __device__ __forceinline__ void gq_body(const GqArgs &a, const u8 *ws) {
                     const u32 v0 = ((s0 >> (4 * h)) & 0x0F0F0F0Fu) | (((s2 >> (4 * h)) & 0x03030303u) << 4);
                     const u32 v1 = ((s1 >> (4 * h)) & 0x0F0F0F0Fu) | (((s2 >> (4 * h + 2)) & 0x03030303u) << 4);
 #pragma unroll
-                    for (int c = 0; c < 8; c++) sp[k][c] = pk_add(h1024_dup(c < 4 ? v0 : v1, c & 3), 0xE420E420u); /* byte - 32 */
+                    for (int c = 0; c < 8; c++) sp[k][c] = pk_add(h1024_dup(c < 4 ? v0 : v1, c & 3), 0xE420E420u) & live[k]; /* byte - 32 */
                 }
                 uint2 qa[TN][2], hm[TN][2];
 #pragma unroll
@@ -974,9 +1076,7 @@ __device__ __forceinline__ void gq_body(const GqArgs &a, const u8 *ws) {
                         B[k] = as_v8h(make_uint4(pk_mul(pk_add(h1024_02(vx), 0xE404E404u), sc), pk_mul(pk_add(h1024_13(vx), 0xE404E404u), sc),
                                                  pk_mul(pk_add(h1024_02(vy), 0xE404E404u), sc), pk_mul(pk_add(h1024_13(vy), 0xE404E404u), sc)));
                     }
-                    le_v8h A[TM];
-                    afrag(c, A);
-                    gq_mma(d1, A, B, h == 0 && c == 0);
+                    mma(c, B);
                     if (c == 0) pipe();
                 }
             } else if constexpr (TY == LE_TYPE_IQ2_S) {
@@ -1005,14 +1105,12 @@ __device__ __forceinline__ void gq_body(const GqArgs &a, const u8 *ws) {
                         for (int k = 0; k < TN; k++) {
                             const u32 qhb = (qhw[k] >> (8 * b)) & 0xFFu;
                             const u32 gi = ((qi[k] >> (8 * l)) & 255u) | ((qhb << (8 - 2 * l)) & 0x300u);
-                            const u32 f = pk_add(h1024_dup(2u * ((scw[k] >> (8 * b + 4 * c1)) & 15u) + 1u, 0), 0xE400E400u);
+                            const u32 f = pk_add(h1024_dup(2u * ((scw[k] >> (8 * b + 4 * c1)) & 15u) + 1u, 0), 0xE400E400u) & live[k];
                             const uint4 g = *(const uint4 *)(tab + 16 * gi);
                             const uint4 m = *(const uint4 *)(sgt + 16 * ((sg[k] >> (8 * l)) & 255u));
                             B[k] = as_v8h(make_uint4(pk_mul(g.x, f) ^ m.x, pk_mul(g.y, f) ^ m.y, pk_mul(g.z, f) ^ m.z, pk_mul(g.w, f) ^ m.w));
                         }
-                        le_v8h A[TM];
-                        afrag(c, A);
-                        gq_mma(d1, A, B, h == 0 && c == 0);
+                        mma(c, B);
                         if (c == 0) pipe();
                     }
                 }
@@ -1032,7 +1130,7 @@ __device__ __forceinline__ void gq_body(const GqArgs &a, const u8 *ws) {
                             rec[k] = *(const uint2 *)(rs[k] + 8 * b);
                             aux[k] = *(const u32 *)(rs[k] + 32 + 4 * b);
                         }
-                        f[k] = pk_add(h1024_dup(2u * (aux[k] >> 28) + 1u, 0), 0xE400E400u); /* (2s+1) */
+                        f[k] = pk_add(h1024_dup(2u * (aux[k] >> 28) + 1u, 0), 0xE400E400u) & live[k]; /* (2s+1) */
                     }
 #pragma unroll
                     for (int c1 = 0; c1 < 2; c1++) {
@@ -1053,127 +1151,407 @@ __device__ __forceinline__ void gq_body(const GqArgs &a, const u8 *ws) {
                             B[k] = as_v8h(make_uint4(pk_mul(g.x, f[k]) ^ m.x, pk_mul(g.y, f[k]) ^ m.y, pk_mul(g.z, f[k]) ^ m.z,
                                                      pk_mul(g.w, f[k]) ^ m.w));
                         }
-                        le_v8h A[TM];
-                        afrag(c, A);
-                        gq_mma(d1, A, B, h == 0 && c == 0);
+                        mma(c, B);
                         if (c == 0) pipe();
                     }
                 }
             }
         }
-        /* super-block epilogue (the h = 1 buffer holds this super-block's second half) */
-        if constexpr (F::EPI == 1) {
+        /* offset term of the super-block (the h = 1 buffer holds its second half and the header) */
+        if constexpr (TY == LE_TYPE_Q4_K || TY == LE_TYPE_Q5_K) {
             const u8 *Wb = lds + BUF;
             const u8 *Sb = Sl + (sb & 1) * SBYTES + (wm * TM) * F::SREC;
 #pragma unroll
             for (int k = 0; k < TN; k++) {
-                const u8 *r = Wb + (wn * TN * 32 + 32 * k + n) * F::SLOT;
-                if constexpr (TY == LE_TYPE_Q4_K || TY == LE_TYPE_Q5_K) {
-                    const uint4 hd = *(const uint4 *)r;
-                    const u32 m0 = hd.z & 0x3F3F3F3Fu, m1 = ((hd.w >> 4) & 0x0F0F0F0Fu) | ((hd.z >> 2) & 0x30303030u);
-                    const le_v8h b2 = as_v8h(make_uint4(pk_add(h1024_02(m0), 0xE400E400u), pk_add(h1024_13(m0), 0xE400E400u),
-                                                        pk_add(h1024_02(m1), 0xE400E400u), pk_add(h1024_13(m1), 0xE400E400u)));
-                    const float dd = h2f(hd.x & 0xFFFFu), dm = h2f(hd.x >> 16);
+                const uint4 hd = *(const uint4 *)(Wb + (wn * TN * 32 + 32 * k + n) * F::SLOT);
+                const u32 m0 = hd.z & 0x3F3F3F3Fu, m1 = ((hd.w >> 4) & 0x0F0F0F0Fu) | ((hd.z >> 2) & 0x30303030u);
+                const le_v8h b2 = as_v8h(make_uint4(pk_add(h1024_02(m0), 0xE400E400u), pk_add(h1024_13(m0), 0xE400E400u),
+                                                    pk_add(h1024_02(m1), 0xE400E400u), pk_add(h1024_13(m1), 0xE400E400u)));
+                const float dm = -h2f(hd.x >> 16) * __builtin_amdgcn_rcpf(unit[k]);
 #pragma unroll
-                    for (int i = 0; i < TM; i++) {
-                        const le_v8h a2 = as_v8h(*(const uint4 *)(Sb + i * 1024 + lane * 16));
-                        const le_v16f d2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a2, b2, (le_v16f){}, 0, 0, 0);
+                for (int i = 0; i < TM; i++) {
+                    const le_v8h a2 = as_v8h(*(const uint4 *)(Sb + i * 1024 + lane * 16));
+                    const le_v16f d2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a2, b2, (le_v16f){}, 0, 0, 0);
 #pragma unroll
-                        for (int e = 0; e < 16; e++) acc[i][k][e] = __builtin_fmaf(dd, d1[i][k][e], __builtin_fmaf(-dm, d2[e], acc[i][k][e]));
-                    }
-                } else if constexpr (TY == LE_TYPE_Q6_K) {
-                    const float d64 = 64.f * h2f(*(const uint16_t *)(r + 126));
-#pragma unroll
-                    for (int i = 0; i < TM; i++)
-#pragma unroll
-                        for (int e = 0; e < 16; e++) acc[i][k][e] = __builtin_fmaf(d64, d1[i][k][e], acc[i][k][e]);
-                } else if constexpr (TY == LE_TYPE_Q3_K) {
-                    const float dd = h2f(*(const uint16_t *)(r + 78));
-#pragma unroll
-                    for (int i = 0; i < TM; i++)
-#pragma unroll
-                        for (int e = 0; e < 16; e++) acc[i][k][e] = __builtin_fmaf(dd, d1[i][k][e], acc[i][k][e]);
-                } else {
-                    const float dd = h2f(*(const uint16_t *)(r + (TY == LE_TYPE_IQ2_XXS ? 32 : 48))) *
-                                     (TY == LE_TYPE_IQ3_XXS ? 0.25f : 0.125f);
-#pragma unroll
-                    for (int i = 0; i < TM; i++)
-#pragma unroll
-                        for (int e = 0; e < 16; e++) acc[i][k][e] = __builtin_fmaf(dd, d1[i][k][e], acc[i][k][e]);
+                    for (int e = 0; e < 16; e++) acc[i][k][e] = __builtin_fmaf(dm, d2[e], acc[i][k][e]);
                 }
             }
         }
     }
     if constexpr (AD) gq_vm_wait<0>(); /* no activation load may still be writing LDS */
-    /* D lane l element e: token 8 (e / 4) + 4 (l / 32) + e % 4 of the tile, row l % 32; the
-     * token scales of the padded tile are all loaded first (one memory round trip) */
-    if constexpr (F::EPI == 2) {
+    {
 #pragma unroll
         for (int k = 0; k < TN; k++) {
-            const float f = ldexpf(1.f, -rowS[k]);
+            const float f = F::EPI == 2 ? ldexpf(1.f, -rowS[k]) : unit[k];
 #pragma unroll
             for (int i = 0; i < TM; i++)
 #pragma unroll
                 for (int e = 0; e < 16; e++) acc[i][k][e] *= f;
         }
     }
-    float ts[TM][16];
+    gq_store<WM, WN, TM, TN, GR, 2 * BUF + NA * AB>(a, lds, tsc, acc, M, mb, nb, pair0, second);
+}
+
+/* ============================ pipelined kernel ============================ */
+/* Q4_K and Q5_K from 33 tokens: a block of 4 waves computes 32 TM tokens x 256 rows, each wave all the
+ * tokens of 64 rows of its own (TN = 2).
+ *
+ * Why this shape. gq_body's 128 x 256 block has 8 waves of 128 x 32: every wave reads the whole
+ * activation tile from LDS, 32 KB per 16-value chunk and CU, which takes as long as the chunk's MFMAs
+ * (256 cycles at 128 B/cycle), and its fragment reads, decoding and MFMAs follow each other inside a
+ * step that begins and ends at a barrier. Here a wave uses each activation fragment for two row
+ * fragments (half the LDS reads), no row is decoded twice, and the stages of a 16-value position run one
+ * position apart, so that LDS reads and decoding of later positions lie between the MFMAs of this one,
+ * also across steps (128 values) and super-blocks.
+ *
+ * Position q of a step (8 positions of 16 values, in the decoder's order): weight bytes are read from
+ * LDS two positions ahead, activation fragments and B fragments are ready one ahead. All global loads go
+ * straight to LDS, a few per position (13 at once held up the wave's instructions: 131k -> 116k cycles
+ * for the loop at M = 512). Activations: two step slots; the only barrier of a step sits between its
+ * positions 6 and 7, when every wave has read its last activation fragment of the step and its loads of
+ * the next one have landed. Weights: private to the wave, three step slots, loaded two steps ahead (a
+ * register-staged form one step ahead was bound by their latency: 88 against 79 us at M = 512; the 2-byte
+ * aligned formats cannot be loaded straight to LDS and stay on gq_body, where they measured 1-15%
+ * faster than here). The accumulator holds a row's sum in units of the super-block scale; the offset
+ * term of one tile per position is added beside the MFMAs.
+ *
+ * Measured, 14336 x 4096 Q4_K, against gq_body's best tile on the same card: M = 64 31.8 -> 29.3 us, 128
+ * 40.2 -> 36.4, 256 55.0 -> 48.2, 512 80.6 -> 74.0 (813 TFLOP/s), 1024 155 -> 139; 28672 rows, M = 512
+ * 155 -> 137. Bound by the matrix cores and the clock: the loop takes 116k cycles, its MFMAs alone
+ * 82k (136 per super-block and wave, 32 cycles each), while the clock falls to 1.7 GHz under them. */
+/* bytes of a staged row per step (its header in front: 16-byte pieces of half super-block 0; of half 1
+ * the same 64 bytes further, where the header's place holds bytes that are not used) */
+template <int TY>
+constexpr int gp_slot() { return TY == LE_TYPE_Q4_K ? 80 : 112; }
+
+/* Decoder state of one 32-row fragment (lane: row rs, K half hs). head: LDS reads of a super-block's
+ * header; prep: take it (h = 0) or its second half's scales (h = 1) into use; fetch(q): LDS reads for
+ * position q; frag(q): its B fragment. */
+template <int TY>
+struct GpD;
+
+template <>
+struct GpD<LE_TYPE_Q4_K> {
+    uint4 nh;
+    u32 scw, sc1, live;
+    le_v8h b2;   /* mins of the super-block as exact halves */
+    float d, dm; /* its scale, and -offset scale (prep of the kernel: over the unit in use) */
+    uint2 raw[2];
+    uint4 kc;
+    __device__ __forceinline__ void head(const u8 *rs, int) { nh = *(const uint4 *)rs; }
+    __device__ __forceinline__ void prep(int h) {
+        if (h == 0) {
+            d = h2f(nh.x & 0xFFFFu);
+            live = d == 0.f ? 0u : ~0u;
+            scw = nh.y & 0x3F3F3F3Fu & live;
+            sc1 = ((nh.w & 0x0F0F0F0Fu) | ((nh.y >> 2) & 0x30303030u)) & live;
+            const u32 m0 = nh.z & 0x3F3F3F3Fu, m1 = ((nh.w >> 4) & 0x0F0F0F0Fu) | ((nh.z >> 2) & 0x30303030u);
+            b2 = as_v8h(make_uint4(pk_add(h1024_02(m0), 0xE400E400u), pk_add(h1024_13(m0), 0xE400E400u),
+                                   pk_add(h1024_02(m1), 0xE400E400u), pk_add(h1024_13(m1), 0xE400E400u)));
+            dm = -h2f(nh.x >> 16);
+        } else {
+            scw = sc1;
+        }
+    }
+    __device__ __forceinline__ void fetch(const u8 *rs, int q, int hs) {
+        if ((q & 1) == 0) raw[(q >> 1) & 1] = *(const uint2 *)(rs + 16 + 32 * (q >> 2) + 16 * ((q >> 1) & 1) + 8 * hs);
+    }
+    __device__ __forceinline__ le_v8h frag(int q, int, u32 mlo, u32 mhi, u32 c) {
+        if ((q & 3) == 0) { /* (sc_lo, -1024 sc_lo, sc_hi / 16, -64 sc_hi) as duplicated halves */
+            const int g = q >> 2;
+            const u32 slo = pk_add(h1024_dup(scw, 2 * g), 0xE400E400u), shi = pk_add(h1024_dup(scw, 2 * g + 1), 0xE400E400u);
+            kc = make_uint4(slo, pk_mul(slo, 0xE400E400u), pk_mul(shi, 0x2C002C00u), pk_mul(shi, 0xD400D400u));
+        }
+        const uint2 r = raw[(q >> 1) & 1];
+        const u32 m = q & 1 ? mhi : mlo, f = q & 1 ? kc.z : kc.x, o = q & 1 ? kc.w : kc.y;
+        return as_v8h(make_uint4(pk_fma((r.x & m) | c, f, o), pk_fma(((r.x >> 8) & m) | c, f, o), pk_fma((r.y & m) | c, f, o),
+                                 pk_fma(((r.y >> 8) & m) | c, f, o)));
+    }
+};
+
+template <>
+struct GpD<LE_TYPE_Q5_K> {
+    uint4 nh;
+    uint2 nq[2], qh[2];
+    u32 scw, sc1, live;
+    le_v8h b2;
+    float d, dm;
+    uint2 raw[2];
+    uint4 kc;
+    __device__ __forceinline__ void head(const u8 *rs, int hs) {
+        nh = *(const uint4 *)rs;
+        nq[0] = *(const uint2 *)(rs + 16 + 8 * hs);
+        nq[1] = *(const uint2 *)(rs + 32 + 8 * hs);
+    }
+    __device__ __forceinline__ void prep(int h) {
+        if (h == 0) {
+            d = h2f(nh.x & 0xFFFFu);
+            live = d == 0.f ? 0u : ~0u;
+            scw = nh.y & 0x3F3F3F3Fu & live;
+            sc1 = ((nh.w & 0x0F0F0F0Fu) | ((nh.y >> 2) & 0x30303030u)) & live;
+            qh[0] = nq[0];
+            qh[1] = nq[1];
+            const u32 m0 = nh.z & 0x3F3F3F3Fu, m1 = ((nh.w >> 4) & 0x0F0F0F0Fu) | ((nh.z >> 2) & 0x30303030u);
+            b2 = as_v8h(make_uint4(pk_add(h1024_02(m0), 0xE400E400u), pk_add(h1024_13(m0), 0xE400E400u),
+                                   pk_add(h1024_02(m1), 0xE400E400u), pk_add(h1024_13(m1), 0xE400E400u)));
+            dm = -h2f(nh.x >> 16);
+        } else {
+            scw = sc1;
+        }
+    }
+    __device__ __forceinline__ void fetch(const u8 *rs, int q, int hs) {
+        if ((q & 1) == 0) raw[(q >> 1) & 1] = *(const uint2 *)(rs + 48 + 32 * (q >> 2) + 16 * ((q >> 1) & 1) + 8 * hs);
+    }
+    __device__ __forceinline__ le_v8h frag(int q, int h, u32, u32, u32) {
+        const int g = q >> 2, G = 2 * h + g, hi = q & 1, c1 = (q >> 1) & 1;
+        if ((q & 3) == 0) {
+            const u32 slo = pk_add(h1024_dup(scw, 2 * g), 0xE400E400u), shi = pk_add(h1024_dup(scw, 2 * g + 1), 0xE400E400u);
+            kc = make_uint4(slo, pk_mul(slo, 0xE400E400u), shi, pk_mul(shi, 0xE400E400u));
+        }
+        const uint2 r = raw[c1], w = qh[c1];
+        const u32 x = and_or(hi ? r.x >> 4 : r.x, 0x0F0F0F0Fu, ((w.x >> (2 * G + hi)) << 4) & 0x10101010u);
+        const u32 y = and_or(hi ? r.y >> 4 : r.y, 0x0F0F0F0Fu, ((w.y >> (2 * G + hi)) << 4) & 0x10101010u);
+        const u32 f = hi ? kc.z : kc.x, o = hi ? kc.w : kc.y;
+        return as_v8h(make_uint4(pk_fma(h1024_02(x), f, o), pk_fma(h1024_13(x), f, o), pk_fma(h1024_02(y), f, o), pk_fma(h1024_13(y), f, o)));
+    }
+};
+
+/* direct-to-LDS load, scalar base + per-lane 32-bit offset (gq_lds_dma16) */
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+__device__ __forceinline__ void gp_lds_dma16(const u8 *base, u32 off, u32 lds_addr) {
+    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds_addr) : "memory", "m0");
+}
+#pragma clang diagnostic pop
+
+template <int TY, int TM, bool GR>
+__device__ __forceinline__ void gp_body(const GqArgs &a, const u8 *ws) {
+    using F = GqF<TY>;
+    constexpr int SLOT = gp_slot<TY>(), N16 = SLOT / 16;
+    constexpr int TN = 2, WN = 4, BM = 32 * TM, BN = 256;
+    constexpr int WB = BN * SLOT, AB = BM * 256, SBYTES = 2 * TM * F::SREC; /* bytes of a weight / activation step slot, sum records */
+    constexpr int NA = AB / 4096;                                            /* activation loads per thread and step */
+    static_assert((size_t)3 * WB + 2 * AB >= (size_t)32 * (BN + 8) * 4, "output staging");
+    extern __shared__ uint4 smem[];
+    u8 *lds = (u8 *)smem, *Aring = lds + 3 * WB, *Sl = Aring + 2 * AB;
+
+    const int K = a.cols, nsb = K >> 8;
+    const int NTR1 = (a.rows + BN - 1) / BN, NTR = GR && a.dual ? 2 * NTR1 : NTR1, MT = GR ? a.maxt : (a.m + BM - 1) / BM;
+    const int id = blockIdx.x, j = id >> 3; /* block order: gq_body */
+    const int mt = NTR >= 8 ? j % MT : id / NTR, nt = NTR >= 8 ? (j / MT) * 8 + (id & 7) : id % NTR;
+    if (nt >= NTR || mt >= MT) return;
+    const bool second = nt >= NTR1;
+    const int nb = (second ? nt - NTR1 : nt) * BN, nbw = min(nb, a.rows - BN), mb = mt * BM; /* rows nbw .. are computed, nb .. stored */
+    int M = a.m, pair0 = 0;
+    const u8 *Wsrc = a.w;
+    if constexpr (GR) {
+        int sl;
+        if (!gq_tile_of(a.off, a.nslot, a.bm, mt, sl, pair0)) return;
+        M = mb + min(BM, a.off[sl + 1] - pair0);
+        if (second)
+            Wsrc = a.ptrs2 ? a.ptrs2[sl] : a.w2 + (size_t)sl * a.w_slot_bytes;
+        else
+            Wsrc = a.ptrs ? a.ptrs[sl] : a.w + (size_t)sl * a.w_slot_bytes;
+    }
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n = lane & 31, hs = lane >> 5;
+    const u32 rb = (u32)nsb * F::SBB;
+    const int sb0 = blockIdx.y * (nsb / a.ksplit), sb1 = sb0 + nsb / a.ksplit, s0 = 2 * sb0, nstep = 2 * sb1;
+    const u8 *Ag = ws + (size_t)(mb / 32) * (K / 16) * 1024;
+    const u8 *Sg = ws + gq_s_off(a.mp, K) + ((size_t)(mb / 32) + (wave % TM)) * nsb * F::SREC;
+    const float *tsc = (const float *)(ws + gq_t_off(a.mp, K, F::SREC));
+
+    /* Weights of the wave's 64 rows: load i of the wave fills bytes 1024 i .. of its part of a slot, rows
+     * without padding (an odd number of 16-byte pieces each). The last row tile starts early enough to be
+     * whole: the caller has rows >= 256. */
+    u32 wd[N16];
+#pragma unroll
+    for (int i = 0; i < N16; i++) {
+        const int c = lane + 64 * i, row = c / N16, k = c - row * N16;
+        wd[i] = (u32)row * rb + F::goff(k, 0);
+    }
+    u8 *wlds = lds + 64 * wave * SLOT;
+    const u32 wlds0 = gq_lds_addr(lds) + (u32)(64 * SLOT) * (u32)wave;
+    const u8 *wrow = Wsrc + (size_t)(nbw + 64 * wave) * rb;
+    auto wdma = [&](int s_, int h, u32 slot, int i0, int i1) { /* loads i0 .. i1 of step s_ (parity h) into the step slot at LDS offset slot */
+        /* past the slice's end the last step again */
+        const u8 *w0 = wrow + (size_t)(min(s_, nstep - 2 + h) >> 1) * F::SBB + 64 * h;
+#pragma unroll
+        for (int i = i0; i < i1; i++) gp_lds_dma16(w0, wd[i], __builtin_amdgcn_readfirstlane(wlds0 + slot + 1024u * i));
+    };
+    /* activations of step s_ (parity h); grouped form: lanes of tokens past the tile's last pair re-read
+     * token 0's (their rows are never stored), so a sparse tile fetches fewer lines */
+    u32 xo[GR ? NA : 1];
+    if constexpr (GR) {
+#pragma unroll
+        for (int i = 0; i < NA; i++) {
+            const int c = tid + 256 * i, tl = c >> 9, off = c & 511;
+            const bool ok = mb + 32 * tl + (off & 31) < M;
+            xo[i] = (ok ? (u32)tl * (u32)(K / 16) * 1024u : 0u) + 16u * (u32)(ok ? off : off & ~31);
+        }
+    }
+    const u32 alds = gq_lds_addr(Aring) + 1024u * (u32)wave, slds = gq_lds_addr(Sl) + 1024u * (u32)(wave % TM);
+    auto dma = [&](int s_, int h, int p) { /* quarter p of a step's loads */
+        const u8 *x0 = Ag + (size_t)min(s_, nstep - 2 + h) * 8192;
+#pragma unroll
+        for (int i = p * NA / 4; i < (p + 1) * NA / 4; i++) {
+            const u32 la = __builtin_amdgcn_readfirstlane(alds + (u32)(h * AB) + 4096u * i);
+            if constexpr (GR)
+                gp_lds_dma16(x0, xo[i], la);
+            else
+                gp_lds_dma16(x0 + (size_t)(i >> 1) * (K / 16) * 1024 + 4096 * (i & 1), 16u * (u32)tid, la);
+        }
+    };
+    auto dmas = [&](int sb) { /* sum records of super-block sb, one 1 KB tile per wave */
+        gp_lds_dma16(Sg + (size_t)min(sb, sb1 - 1) * F::SREC, 16u * (u32)lane, __builtin_amdgcn_readfirstlane(slds + (u32)((sb & 1) * TM * F::SREC)));
+    };
+
+    le_v16f acc[TM][TN];
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
-        for (int e = 0; e < 16; e++) ts[i][e] = tsc[mb + (wm * TM + i) * 32 + 4 * hs + 8 * (e >> 2) + (e & 3)];
-    if (!GR && a.ksplit > 1 && !a.part) { /* K slices without a partial-result buffer: atomic adds */
+        for (int k = 0; k < TN; k++) acc[i][k] = (le_v16f){};
+    GpD<TY> D[TN];
+    float unit[TN], ratio[TN];
 #pragma unroll
-        for (int i = 0; i < TM; i++) {
-            const int t0 = mb + (wm * TM + i) * 32 + 4 * hs;
+    for (int k = 0; k < TN; k++) unit[k] = ratio[k] = 1.f;
+    const u8 *rs[TN];
 #pragma unroll
-            for (int k = 0; k < TN; k++) {
-                const int r = nb + (wn * TN + k) * 32 + n;
+    for (int k = 0; k < TN; k++) rs[k] = wlds + (32 * k + n) * SLOT;
+    auto head = [&](u32 slot) {
 #pragma unroll
-                for (int e = 0; e < 16; e++) {
-                    const int t = t0 + 8 * (e >> 2) + (e & 3);
-                    if (t < M && r < a.rows) unsafeAtomicAdd(a.y + (size_t)t * a.rows + r, acc[i][k][e] * ts[i][e]);
-                }
-            }
-        }
-        return;
-    }
-    /* Stores through LDS, one 32-token tile of every wave row at a time: the waves place their
-     * results as [token][row] (row stride BN + 8 floats: the two 4-token halves of a fragment fall
-     * on different banks), then each token's BN outputs leave as 16-byte stores of consecutive
-     * rows (a wave covers 1 KB of one output row) instead of 4-byte stores 32 to a row. */
-    float *dst = (!GR && a.ksplit > 1) ? a.part + (size_t)blockIdx.y * a.m * a.rows : second ? a.y2 : a.y;
-    constexpr int TS = BN + 8, NQ = BN / 4;
-    static_assert((size_t)WM * 32 * TS * 4 <= (size_t)2 * BUF + (size_t)NA * AB, "output staging must fit the step buffers");
-    float *T = (float *)lds;
-    const bool vec = (a.rows & 3) == 0 && ((size_t)dst & 15) == 0;
-#pragma unroll
-    for (int i = 0; i < TM; i++) {
-        __syncthreads(); /* the step buffers (or the previous round) are no longer read */
+        for (int k = 0; k < TN; k++) D[k].head(rs[k] + slot, hs);
+    };
+    auto prep = [&](int h) {
 #pragma unroll
         for (int k = 0; k < TN; k++) {
-            const int rl = (wn * TN + k) * 32 + n;
-#pragma unroll
-            for (int e = 0; e < 16; e++)
-                T[(wm * 32 + 4 * hs + 8 * (e >> 2) + (e & 3)) * TS + rl] = acc[i][k][e] * ts[i][e];
-        }
-        __syncthreads();
-        for (int c = tid; c < WM * 32 * NQ; c += NT) {
-            const int tl = c / NQ, q = c - tl * NQ;
-            const int t = mb + ((tl >> 5) * TM + i) * 32 + (tl & 31), r = nb + 4 * q;
-            if (t >= M || r >= a.rows) continue;
-            int o = t;
-            if constexpr (GR) o = a.out_idx[pair0 + t - mb];
-            const float4 v = *(const float4 *)(T + tl * TS + 4 * q);
-            float *yp = dst + (size_t)o * a.rows + r;
-            if (vec && r + 3 < a.rows) {
-                *(float4 *)yp = v;
-            } else {
-                const float vv[4] = {v.x, v.y, v.z, v.w};
-                for (int u = 0; u < 4 && r + u < a.rows; u++) yp[u] = vv[u];
+            D[k].prep(h);
+            if (h == 0) { /* a new super-block scale: the running sums go into its units (a zero scale keeps the old ones) */
+                ratio[k] = D[k].d == 0.f ? 1.f : unit[k] * __builtin_amdgcn_rcpf(D[k].d);
+                unit[k] = D[k].d == 0.f ? unit[k] : D[k].d;
+                D[k].dm *= __builtin_amdgcn_rcpf(unit[k]);
             }
         }
+    };
+    auto fetch = [&](u32 slot, int q) {
+#pragma unroll
+        for (int k = 0; k < TN; k++) D[k].fetch(rs[k] + slot, q, hs);
+    };
+    le_v8h A[TM], B[2][TN];
+    le_v16f d2 = {};
+    constexpr int SV = 4; /* other VALU instructions per MFMA */
+    auto aload = [&](int h, int q, int i) { /* activation fragment i of position q: its 16-value chunk of the step */
+        const int c = (q & 4) | ((q & 1) << 1) | ((q >> 1) & 1);
+        A[i] = as_v8h(*(const uint4 *)(Aring + h * AB + i * 8192 + c * 1024 + lane * 16));
+    };
+    /* the decoders' masks in registers the compiler cannot see through, so (x & m) | c becomes one
+     * v_and_or_b32 (which cannot carry literals); the inline form costs a wait state per use */
+    u32 cmlo = 0x000F000Fu, cmhi = 0x00F000F0u, c1024 = 0x64006400u;
+    __asm__("" : "+v"(cmlo), "+v"(cmhi), "+s"(c1024));
+    auto frag = [&](int h, int q) {
+#pragma unroll
+        for (int k = 0; k < TN; k++) B[q & 1][k] = D[k].frag(q, h, cmlo, cmhi, c1024);
+    };
+
+    u32 wc = 0, wn1 = WB, wn2 = 2 * WB; /* weight slots of this step and the next two */
+    wdma(s0, 0, wc, 0, N16);
+#pragma unroll
+    for (int p = 0; p < 4; p++) dma(s0, 0, p);
+    dmas(sb0);
+    wdma(s0 + 1, 1, wn1, 0, N16);
+    gq_vm_wait<N16>();
+    __syncthreads();
+    dma(s0 + 1, 1, 0);
+    head(wc);
+    fetch(wc, 0);
+#pragma unroll
+    for (int i = 0; i < TM; i++) aload(0, 0, i);
+    fetch(wc, 1);
+    prep(0);
+    frag(0, 0);
+    for (int sb = sb0; sb < sb1; sb++) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int s = 2 * sb + h;
+#pragma unroll
+            for (int q = 0; q < 8; q++) {
+                const int h1 = q == 7 ? h ^ 1 : h, q1 = (q + 1) & 7, q2 = (q + 2) & 7;
+                if (q == 7) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    /* the step's last activation fragments are in registers, the next step's have
+                     * landed (younger: the weight loads issued after them) */
+                    gq_vm_wait<N16>();
+                    gq_barrier();
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                /* a few loads at a time: a burst of them holds up the wave's instructions, MFMAs among them */
+                if (q == 7) dma(s + 2, h, 0);
+                if (q < 3) dma(s + 1, h ^ 1, q + 1);
+                if (q == 2 && h == 0) dmas(sb + 1);
+                if (q >= 3 && q < 6) wdma(s + 2, h, wn2, (q - 3) * N16 / 3, (q - 2) * N16 / 3);
+                if (q == 6) { /* the next step's weights have landed: younger are its activations, sum records and the weights after it */
+                    if (h == 0) gq_vm_wait<NA + N16 + 1>();
+                    else gq_vm_wait<NA + N16>();
+                    if (h == 1) head(wn1);
+                }
+                fetch(q >= 6 ? wn1 : wc, q2);
+                if (h == 0 && q == 0) {
+#pragma unroll
+                    for (int k = 0; k < TN; k++)
+#pragma unroll
+                        for (int i = 0; i < TM; i++)
+#pragma unroll
+                            for (int e = 0; e < 16; e++) acc[i][k][e] *= ratio[k];
+                }
+                /* offset term -dmin sum_j m_j S_j, in units, of one tile per position: its MFMA at position
+                 * g - 1 = tile of the super-block, added one position later */
+                const int g = 8 * h + q;
+                if (g >= 2 && g - 2 < TM * TN) {
+                    const int i = (g - 2) / TN, k = (g - 2) % TN;
+#pragma unroll
+                    for (int e = 0; e < 16; e++) acc[i][k][e] = __builtin_fmaf(D[k].dm, d2[e], acc[i][k][e]);
+                }
+                if (g >= 1 && g - 1 < TM * TN) {
+                    const int i = (g - 1) / TN, k = (g - 1) % TN;
+                    const le_v8h a2 = as_v8h(*(const uint4 *)(Sl + ((sb & 1) * TM + i) * 1024 + lane * 16));
+                    d2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a2, D[k].b2, (le_v16f){}, 0, 0, 0);
+                }
+#pragma unroll
+                for (int i = 0; i < TM; i++)
+#pragma unroll
+                    for (int k = 0; k < TN; k++) acc[i][k] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[i], B[q & 1][k], acc[i][k], 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < TM; i++) aload(h1, q1, i); /* each once its MFMAs have been issued: into the same registers */
+                if (q == 7) prep(h ^ 1);
+                frag(h1, q1);
+                /* MFMAs evenly among the position's other instructions */
+#pragma unroll
+                for (int i = 0; i < TM; i++) {
+#pragma unroll
+                    for (int k = 0; k < TN; k++) {
+                        if (g == 0) __builtin_amdgcn_sched_group_barrier(0x002, 17, 0); /* the rescaling */
+                        else __builtin_amdgcn_sched_group_barrier(0x002, SV, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    }
+                    __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            const u32 w = wc;
+            wc = wn1;
+            wn1 = wn2;
+            wn2 = w;
+        }
     }
+    gq_vm_wait<0>(); /* no load may still be writing LDS */
+#pragma unroll
+    for (int k = 0; k < TN; k++) {
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int e = 0; e < 16; e++) acc[i][k][e] *= unit[k];
+    }
+    gq_store<1, WN, TM, TN, GR, 3 * WB + 2 * AB>(a, lds, tsc, acc, M, mb, nbw, pair0, second, nb);
 }
 
 #define LE_GQX(TY, SK) \
@@ -1228,11 +1606,20 @@ extern "C" __global__ void __launch_bounds__(256) le_gq_ksum(GqArgs a) {
     extern "C" __global__ void __launch_bounds__(WM * WN * 64) le_gqg_##TY##_w##WM##WN##_t##TM##TN(GqArgs a, const u8 *ws) { \
         gq_body<TY, WM, WN, TM, TN, true, 2>(a, ws);                                                                     \
     }
+/* one wave per SIMD is resident (LDS), but 256 registers: with 512 the accumulators go to the
+ * accumulation registers, which the rescaling cannot reach without moves (393 reads a super-block) */
+#define LE_GP_REGS __attribute__((amdgpu_waves_per_eu(2, 2)))
+#define LE_GP_(TY, TM)                                                                                                  \
+    extern "C" __global__ void __launch_bounds__(256) LE_GP_REGS le_gp_##TY##_t##TM(GqArgs a, const u8 *ws) { gp_body<TY, TM, false>(a, ws); } \
+    extern "C" __global__ void __launch_bounds__(256) LE_GP_REGS le_gpg_##TY##_t##TM(GqArgs a, const u8 *ws) { gp_body<TY, TM, true>(a, ws); }
+#define LE_GP(TY) LE_GP_(TY, 4) LE_GP_(TY, 2)
 #define LE_GQ(TY) LE_GQ_(TY, 1, 4, 1, 2) LE_GQ_(TY, 1, 4, 2, 2) LE_GQ_(TY, 1, 4, 4, 2) LE_GQ_(TY, 2, 2, 2, 2) \
     LE_GQ_(TY, 1, 8, 2, 1) LE_GQ_(TY, 1, 8, 4, 1) LE_GQ_(TY, 1, 8, 1, 1) LE_GQ_(TY, 1, 4, 2, 1) LE_GQ_(TY, 1, 4, 1, 1) LE_GQ_(TY, 1, 4, 4, 1) LE_GQG_(TY, 1, 8, 2, 1) LE_GQG_(TY, 1, 8, 4, 1) LE_GQG_(TY, 2, 2, 2, 2) LE_GQG_(TY, 1, 8, 1, 1) LE_GQG_(TY, 1, 4, 1, 1)
 #if LE_GQ_SET == 2
 LE_GQ(2) LE_GQ(11) LE_GQ(13) LE_GQ(22)
+LE_GP(13)
 #else
 LE_GQ(8) LE_GQ(12) LE_GQ(14) LE_GQ(16) LE_GQ(18)
+LE_GP(12)
 LE_GQ_(12, 2, 4, 2, 2) LE_GQ_(12, 2, 4, 2, 1)
 #endif

@@ -127,9 +127,11 @@ struct le_ctx {
     int gq_cfg = 0;          /* generic GEMM block shape (tokens x rows, waves): 0 auto, 1 (32x256, 4), 2 (64x256, 4),
                                 3 (128x256, 4), 4 (128x128, 4), 5 (64x256, 8), 6 (128x256, 8), 7 (32x256, 8),
                                 8 (64x128, 4), 9 (32x128, 4), 10 (128x128, 4); Q4_K only: 11 (128x256, 2x4
-                                waves of 64x64), 12 (128x128, 2x4 waves of 64x32) */
+                                waves of 64x64), 12 (128x128, 2x4 waves of 64x32); Q4_K, Q5_K: 21 / 22 the
+                                pipelined kernel with 128 / 64 tokens a block */
     int gq_ksplit = 0;       /* generic GEMM K slices: 0 auto, else 1, 2, 4, 8 */
     int moe_route1 = 1;      /* grouped MoE up to 32 tokens: routing and grouping in one block */
+    int mmg_gp = 1;          /* grouped form of Q4_K / Q5_K on the pipelined kernel */
     int mmg_w4 = 1;          /* grouped 32-pair tiles: 4-wave 32 x 128 blocks where 8-wave ones fill half the LDS */
     int mmg_xw = 1;          /* grouped pre-pass: one wave per pair (K <= 4096) instead of one block */
     std::vector<hipModule_t> mods;
@@ -586,12 +588,14 @@ int le_set_option(le_ctx *c, const char *name, int value) {
         if (value < 1) return c->fail(LE_ERR_ARG, "gq_min_m must be >= 1");
         c->gq_min_m = value;
     } else if (n == "gq_cfg") {
-        if (value < 0 || value > 12) return c->fail(LE_ERR_ARG, "gq_cfg must be 0..12");
+        if (value < 0 || (value > 12 && value != 21 && value != 22)) return c->fail(LE_ERR_ARG, "gq_cfg must be 0..12, 21 or 22");
         c->gq_cfg = value;
     } else if (n == "moe_route1") {
         c->moe_route1 = value ? 1 : 0;
     } else if (n == "mmg_w4") {
         c->mmg_w4 = value ? 1 : 0;
+    } else if (n == "mmg_gp") {
+        c->mmg_gp = value ? 1 : 0;
     } else if (n == "mmg_xw") {
         c->mmg_xw = value ? 1 : 0;
     } else if (n == "gq_ksplit") {
@@ -1070,6 +1074,10 @@ static int gq_slot(int ty) {
     }
     return 0;
 }
+/* The pipelined kernel (le_gp_*: Q4_K and Q5_K, whole 256-row tiles) and its LDS: three weight step slots,
+ * two of tm 32-token activation tiles, sum records of two super-blocks. */
+static bool gp_takes(int ty, int rows) { return (ty == LE_TYPE_Q4_K || ty == LE_TYPE_Q5_K) && rows >= 256; }
+static size_t gp_lds(int ty, int tm) { return (size_t)3 * 256 * gq_slot(ty) + (size_t)2 * tm * 8192 + (size_t)2 * tm * gq_srec(ty); }
 static int gq_tab(int ty) {
     return ty == LE_TYPE_IQ2_XXS ? 6144 : ty == LE_TYPE_IQ3_XXS ? 4096 : ty == LE_TYPE_IQ2_S ? 16384 + 4096 : 0;
 }
@@ -1093,19 +1101,30 @@ static int gq_launch(le_ctx *c, int ty, const void *w, const float *x, int m, fl
     else if (m <= 128 && ty == LE_TYPE_Q6_K) ci = 9;
     else if (m <= 128 && (k45 || ty == LE_TYPE_IQ3_XXS)) ci = 4;
     else if (m <= 256 && k45) ci = 4;
-    if (c->gq_cfg) ci = c->gq_cfg - 1;
+    if (c->gq_cfg && c->gq_cfg <= 12) ci = c->gq_cfg - 1;
     const int nsb = cols / 256, srec = gq_srec(ty);
+    /* pipelined kernel, its 32-token tiles per block (0: not used): from 33 tokens (M = 64 31.8 -> 29.3 us;
+     * up to 32 the 32 x 128 tiles have more blocks); blocks of 64 tokens while they fill no more than
+     * the chip, else 128 (14336 x 4096 Q4_K, 64 / 128 tokens a block: M = 128 36.4 / 38.8 us, 256 48.2 / 52.5,
+     * 512 90.4 / 74.0; 4096 x 4096 M = 512 38.9 / 41.2) */
+    int gp = 0;
+    if (gp_takes(ty, rows)) {
+        if (c->gq_cfg) gp = c->gq_cfg == 21 ? 4 : c->gq_cfg == 22 ? 2 : 0;
+        else if (m > 32) gp = (long long)((rows + 255) / 256) * ((m + 63) / 64) <= c->cus ? 2 : 4;
+    }
     auto lds_of = [&](int i) {
+        if (gp) return gp_lds(ty, gp);
         const int BM = 32 * cfgs[i][0] * cfgs[i][2], BN = 32 * cfgs[i][1] * cfgs[i][3];
         return (size_t)2 * (BN * gq_slot(ty) + BM * 256) + (size_t)2 * (BM / 32) * srec + gq_tab(ty);
     };
     if (lds_of(ci) > c->lds_limit && (ci == 2 || ci == 5)) ci = 3;
     const size_t lds = lds_of(ci);
     if (lds > c->lds_limit) return c->fail(LE_ERR_SHAPE, "GEMM tile does not fit the LDS");
-    const int WM = cfgs[ci][0], WN = cfgs[ci][1], TM = cfgs[ci][2], TN = cfgs[ci][3];
+    const int WM = gp ? 1 : cfgs[ci][0], WN = gp ? 4 : cfgs[ci][1], TM = gp ? gp : cfgs[ci][2], TN = gp ? 2 : cfgs[ci][3];
     const int BM = 32 * TM * WM, BN = 32 * TN * WN, nthr = 64 * WM * WN;
     char name[48];
-    snprintf(name, sizeof name, "le_gq_%d_w%d%d_t%d%d", ty, WM, WN, TM, TN);
+    if (gp) snprintf(name, sizeof name, "le_gp_%d_t%d", ty, gp);
+    else snprintf(name, sizeof name, "le_gq_%d_w%d%d_t%d%d", ty, WM, WN, TM, TN);
     if (!c->fn(name)) return c->fail(LE_ERR_SHAPE, "GEMM kernel %s is not built", name);
     const long long ntr = (rows + BN - 1) / BN, mt = (m + BM - 1) / BM;
     const long long grid = (ntr >= 8 ? (ntr + 7) / 8 * 8 : ntr) * mt; /* block order: le_gq_kernels.hip */
@@ -1182,12 +1201,14 @@ static int mm_grouped(le_ctx *c, int ty, const void *const *ptrs, const void *w,
         const int BM = 32 * cfgs[i][0] * cfgs[i][2], BN = 32 * cfgs[i][1] * cfgs[i][3];
         return (size_t)2 * (BN * gq_slot(ty) + BM * 256) + (size_t)2 * (BM / 32) * srec + gq_tab(ty);
     };
-    if (lds_of(ci) > c->lds_limit) ci = 3; /* 128 x 128 on 4 waves */
+    /* Q4_K, Q5_K with 64- or 128-pair tiles: the pipelined kernel, same tiles */
+    const int gp = gp_takes(ty, rows) && c->mmg_gp && (ci == 4 || ci == 5) ? (ci == 4 ? 2 : 4) : 0;
+    if (!gp && lds_of(ci) > c->lds_limit) ci = 3; /* 128 x 128 on 4 waves */
     /* 32-pair tiles whose 8-wave block would hold more than half the LDS (Q6_K, Q8_0: one block
      * per CU): 32 x 128 on 4 waves, several blocks per CU */
     if (ci == 6 && c->mmg_w4 && 2 * lds_of(6) > c->lds_limit) ci = 7;
     const int WM = cfgs[ci][0], WN = cfgs[ci][1], TM = cfgs[ci][2], TN = cfgs[ci][3];
-    const int BM = 32 * TM * WM, BN = 32 * TN * WN, nthr = 64 * WM * WN;
+    const int BM = 32 * TM * WM, BN = 32 * TN * WN, nthr = gp ? 256 : 64 * WM * WN; /* le_gp: the same BM and BN */
     if (BM != mmg_bm(nslot, npair) && !(ci == 3 && mmg_bm(nslot, npair) == 128))
         return c->fail(LE_ERR_SHAPE, "grouped GEMM tile does not fit the LDS");
     const int maxt = mmg_maxt(nslot, npair), mp = maxt * BM;
@@ -1213,8 +1234,9 @@ static int mm_grouped(le_ctx *c, int ty, const void *const *ptrs, const void *w,
         rc = c->launch(name, dim3((unsigned)npair), 256, 0, (hipStream_t)stream, args);
     }
     if (rc) return rc;
-    snprintf(name, sizeof name, "le_gqg_%d_w%d%d_t%d%d", ty, WM, WN, TM, TN);
-    return c->launch(name, dim3((unsigned)grid), nthr, lds_of(ci), (hipStream_t)stream, args);
+    if (gp) snprintf(name, sizeof name, "le_gpg_%d_t%d", ty, gp);
+    else snprintf(name, sizeof name, "le_gqg_%d_w%d%d_t%d%d", ty, WM, WN, TM, TN);
+    return c->launch(name, dim3((unsigned)grid), nthr, gp ? gp_lds(ty, gp) : lds_of(ci), (hipStream_t)stream, args);
 }
 
 int le_mm_grouped(le_ctx *c, int ty, const void *const *ptrs, const void *w, const int *off, const int *in_idx,

@@ -40,3 +40,28 @@ def test_matvec_ragged_split(engine, name, rows, nsb):
     engine.mv_q8(ty, None, dev(xq), dev(xd), dev(xs), y, rows, cols, 0, 1, w=dev(q))
     want = oracle.matvec_q8(ty, q, rows, cols, xq, xd, xs).astype(np.float64)
     assert np.all(np.abs(y.cpu().numpy() - want) <= 1e-5 * mag + 1e-30)
+
+
+# the pipelined GEMM: its 64- and 128-token blocks (the latter where the former overfill the chip), first and last
+# token count, ragged last row tile (moved back to be whole), one super-block, K slices, super-blocks whose scale is
+# zero (offsets only) between ones whose scales differ by 2^20
+@pytest.mark.parametrize("name", ["Q4_K", "Q5_K"])
+@pytest.mark.parametrize("rows,nsb,m", [(256, 1, 33), (257, 2, 64), (511, 3, 65), (300, 4, 129), (8448, 2, 513)])
+def test_gemm_pipelined(engine, name, rows, nsb, m):
+    import torch
+    ty, cols = le.MV_TYPES[name], 256 * nsb
+    q = wbytes(ty, rows, cols, seed=rows + m).reshape(rows, nsb, -1).copy()
+    rng = np.random.default_rng(m)
+    scale = rng.choice(np.float16([0.0, 2.0 ** -14, 0.01, 64.0]), size=(rows, nsb)).astype(np.float16)
+    some = rng.random((rows, nsb)) < 0.3
+    d = q[:, :, 0:2].copy().view(np.float16)[:, :, 0]
+    q[:, :, 0:2] = np.where(some, scale, d)[:, :, None].view(np.uint8).reshape(rows, nsb, 2)
+    x = acts(m * cols, 7 + m).reshape(m, cols)
+    pick = np.unique(np.r_[0:8, rows - 264:rows - 248, rows - 8:rows].clip(0, rows - 1))  # oracle rows
+    y = torch.full((m, rows), float("nan"), device="cuda")
+    print("pipelined GEMM", name, rows, cols, m, flush=True)
+    engine.gemm(ty, dev(q), dev(x), m, y, rows, cols)
+    got = y.cpu().numpy()
+    assert np.all(np.isfinite(got))
+    sel = np.ascontiguousarray(q[pick])
+    check_close(got[:, pick], oracle.matmat(ty, sel, len(pick), cols, x), absmag(ty, sel, len(pick), cols, x))
