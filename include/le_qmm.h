@@ -91,7 +91,9 @@ const char *le_last_error(const le_ctx *ctx);
  *     "ms_t" (0/1): Q4_K with 2..8 tokens per pass on the staged kernel (one weight stream, 8 tokens
  *     per MFMA pass), used by le_gemm below "gm_min_m" tokens
  *   GEMM: "gq" (0/1) Q4_K on the generic matrix-core GEMM (default) or the older le_gm kernels,
- *     "gq_min_m" smallest M of the other types on the matrix-core GEMM (below: vector kernels that
+ *     "mt" (0/1) few-token kernel (fp16 high and low halves, tokens as MFMA rows) for the other types up to 16
+ *     tokens and for Q4_K up to 16 where K exceeds its own few-token kernel's LDS;
+ *     "gq_min_m" smallest M of the other types on the matrix-core GEMM without "mt" (below: vector kernels that
  *     read the weights once per 8 tokens), "gq_cfg" its block shape (0 auto; 1..10: 32x256, 64x256,
  *     128x256, 128x128 tokens x rows on 4 waves, 64x256, 128x256, 32x256 on 8 waves, 64x128, 32x128,
  *     128x128 on 4 waves; Q4_K only, 2 x 4 waves: 11 128x256, 12 128x128; Q4_K and Q5_K with 256 rows
@@ -167,9 +169,9 @@ int le_matvec_q8(le_ctx *ctx, int ty, const void *const *ptrs, const void *w, co
  *      src/cpu_ref.rs:266-276) ----
  * Y[t * rows + r] = W[r,:] . X[t * cols ...] for t < m. ws: device workspace of
  * le_gemm_workspace_size(ty, m, cols) bytes, the counterpart of the reference's pre-quantized
- * activation buffers (xqb/xdb/xsb, src/gpu.rs:210). Every type runs on the matrix cores from 17
- * tokens (Q4_K: 3..16 tokens on a staged f16 MFMA kernel, 2 on the staged int8 matvec; other types:
- * from "gq_min_m" = 9 tokens, vector kernels below). On the matrix cores each token is scaled by
+ * activation buffers (xqb/xdb/xsb, src/gpu.rs:210). Every type runs on the matrix cores (Q4_K: 3..16
+ * tokens on a staged f16 MFMA kernel, 2 on the staged int8 matvec; other types: 2..16 tokens on the
+ * few-token kernel, up to 8 of them with activations in two fp16 halves, about 2^-22 per value). From 17 tokens each token is scaled by
  * its own power of two and rounded to fp16 (relative error 2^-11 per value at any magnitude up to
  * 2^127); Q8_0 and Q4_0 weights enter as fp16(q * d_b * 2^S), one rounding, with a power of two per
  * row that keeps every code inside the fp16 range for any finite scales; the other types as exact

@@ -25,7 +25,7 @@
 namespace {
 
 const char *kParts[] = {"le_qmm_deq", "le_qmm_moe", "le_qmm_mv8", "le_qmm_mv12", "le_qmm_mv14", "le_qmm_mv16", "le_qmm_mv18", "le_qmm_gm",
-                        "le_qmm_gq", "le_qmm_gq2", "le_qmm_mv2", "le_qmm_mv11", "le_qmm_mv13", "le_qmm_mv22"};
+                        "le_qmm_gq", "le_qmm_gq2", "le_qmm_mt", "le_qmm_mv2", "le_qmm_mv11", "le_qmm_mv13", "le_qmm_mv22"};
 
 /* Kernel argument block of le_mv_* (mirrors MvArgs in le_qmm_kernels.hip). */
 struct MvArgs {
@@ -122,6 +122,7 @@ struct le_ctx {
     int gm_pc = 1;           /* MFMA GEMM with producer/consumer waves */
     int gm_split = 0;        /* 1: activations as two fp16 halves (22 bits); 0: one fp16 value (11 bits) */
     int gm_mh_t16 = 0;       /* 9..16 tokens: one 16-token group instead of two 8-token groups */
+    int mt = 1;              /* few tokens of the other types on the f16 matrix-core kernel le_mt_* */
     int gq = 1;              /* Q4_K GEMM on the generic kernels (le_gq_*) instead of le_gm_12_* */
     int gq_min_m = 9;        /* other types: smallest M on the matrix-core GEMM (below: vector kernels) */
     int gq_cfg = 0;          /* generic GEMM block shape (tokens x rows, waves): 0 auto, 1 (32x256, 4), 2 (64x256, 4),
@@ -582,6 +583,8 @@ int le_set_option(le_ctx *c, const char *name, int value) {
         c->rd_block = value;
     } else if (n == "gm_mh_t16") {
         c->gm_mh_t16 = value ? 1 : 0;
+    } else if (n == "mt") {
+        c->mt = value ? 1 : 0;
     } else if (n == "gq") {
         c->gq = value ? 1 : 0;
     } else if (n == "gq_min_m") {
@@ -1082,6 +1085,56 @@ static int gq_tab(int ty) {
     return ty == LE_TYPE_IQ2_XXS ? 6144 : ty == LE_TYPE_IQ3_XXS ? 4096 : ty == LE_TYPE_IQ2_S ? 16384 + 4096 : 0;
 }
 
+/* Few tokens (m <= 16), every type: le_mt_*. Returns 1 where it does not apply (the caller goes on). The
+ * partial results of K slices (needed where the activation images of all of K exceed the LDS) go to the
+ * workspace; without room for them it does not apply. */
+static int mt_launch(le_ctx *c, int ty, const void *w, const float *x, int m, float *y, int rows, int cols, void *ws,
+                     size_t ws_bytes, hipStream_t st) {
+    const int T = m <= 4 ? 4 : m <= 8 ? 8 : 16, R = T == 4 ? 8 : 16, NW = 8;
+    const int nsb = cols / 256, ntile = (rows + 15) / 16;
+    const bool ofs = ty == LE_TYPE_Q4_K || ty == LE_TYPE_Q5_K;
+    const int cps = ty == LE_TYPE_Q6_K ? 14 : ty == LE_TYPE_IQ2_XXS ? 5 : ty == LE_TYPE_IQ3_XXS ? 7 : ty == LE_TYPE_Q8_0 ? 17 : ty == LE_TYPE_Q5_K ? 11 : ty == LE_TYPE_Q3_K ? 7 : ty == LE_TYPE_IQ2_S ? 6 : 9;
+    auto lds_of = [&](int ks) {
+        const size_t most = (nsb + ks - 1) / ks;
+        return most * ((size_t)(32 + (ofs ? 2 : 0)) * (R + 1) * 16 + 64) + (size_t)NW * 16 * (cps | 1) * 16 + (size_t)2 * NW * 4 * T * 16 + gq_tab(ty);
+    };
+    int ks = 1;
+    while (ks < nsb && lds_of(ks) > c->lds_limit) ks++;
+    const size_t lds = lds_of(ks);
+    if (lds > c->lds_limit || ks > 65535) return 1;
+    float *part = nullptr;
+    if (ks > 1) {
+        if (!ws || !al16(ws) || ws_bytes < (size_t)ks * m * rows * 4) return 1;
+        part = (float *)ws;
+    }
+    char name[32];
+    snprintf(name, sizeof name, "le_mt_%d_t%d", ty, T);
+    if (!c->fn(name)) return 1;
+    /* waves per row tile: the fewest that give every CU a block (fewer: longer chains, no sum through LDS) */
+    int kw = 1;
+    while (kw < NW && (long long)ntile * kw * ks < (long long)NW * c->cus) kw *= 2;
+    const int groups = (ntile + NW / kw - 1) / (NW / kw), per_cu = c->blocks_per_cu(name, 64 * NW, lds);
+    const int cap = std::max(1, c->cus * std::max(1, per_cu) / ks), it = (groups + cap - 1) / cap, gx = (groups + it - 1) / it;
+    struct {
+        const void *w;
+        const float *x;
+        float *y, *part;
+        int rows, cols, m, kw;
+    } a{w, x, y, part, rows, cols, m, kw};
+    void *args[] = {&a};
+    int rc = c->launch(name, dim3((unsigned)gx, (unsigned)ks), 64 * NW, lds, st, args);
+    if (rc || !part) return rc;
+    GqHostArgs s{};
+    s.y = y;
+    s.rows = rows;
+    s.m = m;
+    s.ksplit = ks;
+    s.part = part;
+    void *sargs[] = {&s};
+    const size_t n4 = ((size_t)m * rows + 3) / 4;
+    return c->launch("le_gq_ksum", dim3((unsigned)std::min<size_t>((n4 + 255) / 256, (size_t)c->cus * 8)), 256, 0, st, sargs);
+}
+
 static int gq_launch(le_ctx *c, int ty, const void *w, const float *x, int m, float *y, int rows, int cols, void *ws,
                      size_t ws_bytes, hipStream_t st) {
     /* block shapes: (WM, WN, TM, TN) -> BM = 32 TM WM tokens, BN = 32 TN WN rows */
@@ -1270,6 +1323,15 @@ int le_gemm(le_ctx *c, int ty, const void *w, const float *x, int m, float *y, i
     /* Q4_K, 3..16 tokens: the staged f16 kernel (2 tokens: the int8 multi-token matvec is faster);
      * shapes whose activations do not fit its LDS, and gm_split=1 (two fp16 halves, which only
      * the le_gm GEMM carries), go to a GEMM */
+    /* The other types up to 16 tokens: the few-token kernel (4 / 8 / 16 tokens against the vector kernels,
+     * from 9 tokens the GEMM: Q6_K 4096 x 14336 67.3 -> 25.7, 124 -> 22.6, 30.6 -> 30.7 us, Q8_0 14336 x 4096
+     * 35.6 -> 18.4, 49.5 -> 21.3, 32.6 -> 22.1, Q5_K 3072 x 3072 12.3 -> 8.2, 20.6 -> 11.4, 15.9 -> 13.3);
+     * below "gq_min_m" without a workspace too */
+    const bool mt = c->mt && m >= 2 && m <= 16 && !c->gq_cfg && !c->gq_ksplit;
+    if (mt && ty != LE_TYPE_Q4_K && m < c->gq_min_m && rows > 0 && cols > 0 && cols % 256 == 0 && w && x && y && al16(x)) {
+        const int rc = mt_launch(c, ty, w, x, m, y, rows, cols, ws, ws_bytes, (hipStream_t)stream);
+        if (rc != 1) return rc;
+    }
     const bool few = ty == LE_TYPE_Q4_K && c->gm_mh && !c->gm_split && m >= 3 && m <= c->gm_mh_max;
     const bool gemm = ty == LE_TYPE_Q4_K ? (m >= c->gm_min_m || few) : m >= c->gq_min_m;
     if (gemm && m > 0 && rows > 0 && cols > 0 && cols % 256 == 0 && w && x && y) {
@@ -1279,6 +1341,12 @@ int le_gemm(le_ctx *c, int ty, const void *w, const float *x, int m, float *y, i
         if (!al16(x) || !al16(ws)) return c->fail(LE_ERR_ALIGN, "x and ws must be 16-byte aligned");
         if (few) {
             const int rc = mh_launch(c, w, x, m, y, rows, cols, (hipStream_t)stream);
+            if (rc != 1) return rc;
+        }
+        /* ... and Q4_K where its own kernel's images do not fit the LDS (4096 x 14336, 4 / 8 / 16 tokens 27.9 ->
+         * 19.7, 27.7 -> 20.3, 28.0 -> 25.8 us; where they fit, that kernel's half-size images are faster) */
+        if (mt && (ty != LE_TYPE_Q4_K || (c->gq && !c->gm_split && few))) {
+            const int rc = mt_launch(c, ty, w, x, m, y, rows, cols, ws, ws_bytes, (hipStream_t)stream);
             if (rc != 1) return rc;
         }
         if (ty != LE_TYPE_Q4_K || (c->gq && !c->gm_split))

@@ -65,3 +65,26 @@ def test_gemm_pipelined(engine, name, rows, nsb, m):
     assert np.all(np.isfinite(got))
     sel = np.ascontiguousarray(q[pick])
     check_close(got[:, pick], oracle.matmat(ty, sel, len(pick), cols, x), absmag(ty, sel, len(pick), cols, x))
+
+
+# the few-token kernel: its three token counts (4, 8, 16) and their edges, fewer rows than a tile and a ragged last one,
+# one super-block, waves without a super-block, K in slices summed through the workspace (56 super-blocks), and more
+# row tiles than one round of blocks
+@pytest.mark.parametrize("name", list(le.MV_TYPES))
+@pytest.mark.parametrize("rows,nsb,m", [(5, 1, 2), (37, 3, 4), (300, 9, 5), (40, 56, 3), (40, 56, 8), (130, 7, 9), (40, 43, 16), (33000, 1, 3)])
+def test_gemm_few_tokens(engine, name, rows, nsb, m):
+    import torch
+    ty, cols = le.MV_TYPES[name], 256 * nsb
+    q = wbytes(ty, rows, cols, seed=rows + nsb)
+    x = acts(m * cols, 3 + m).reshape(m, cols)
+    x[m - 1] *= np.float32(1e-20)  # a token of another magnitude
+    x[0, :256] = 0.0
+    y = torch.full((m, rows), float("nan"), device="cuda")
+    print("few tokens", name, rows, cols, m, flush=True)
+    engine.gemm(ty, dev(q), dev(x), m, y, rows, cols)
+    w = oracle.dequant_rows(ty, q, rows, cols).astype(np.float64)
+    want, mag = x.astype(np.float64) @ w.T, np.abs(x.astype(np.float64)) @ np.abs(w).T
+    # two fp16 halves: 2^-22 a value, fp32 sums of 8 products' chains and nsb super-blocks (2^-24 each); one half
+    # (9 tokens and more, and Q4_K's own kernel): 2^-11; 15-bit activations (Q4_K, 2 tokens): 3.1e-5 of a block's maximum
+    tol = 1e-5 if m <= 8 and ty != le.Q4_K else 1e-3
+    assert np.all(np.abs(y.cpu().numpy() - want) <= tol * mag + 1e-30), float(np.max(np.abs(y.cpu().numpy() - want) / (mag + 1e-30)))
