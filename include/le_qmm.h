@@ -100,6 +100,8 @@ const char *le_last_error(const le_ctx *ctx);
  *     or more, the pipelined kernel: 21 128x256, 22 64x256), "gq_ksplit" its K
  *     slices (0 auto, 1, 2, 4, 8); "mmg_xw" (0/1) the grouped form's activation pre-pass one wave
  *     per pair from 256 pairs when K <= 4096 (default) or one block per pair (same results);
+ *     "mmg_mt" (0/1) grouped form of up to six pairs a slot on the few-token kernel (default; activations
+ *     rounded once at their 256-value block's scale) or on the tiles of 32 pairs (at their row's scale);
  *     "mmg_gp" (0/1) grouped 64- and 128-pair tiles of Q4_K / Q5_K on the pipelined kernel (default) or
  *     on the generic one (the sums differ by fp32 rounding);
  *     "mmg_w4" (0/1) grouped 32-pair tiles of Q6_K / Q8_0 / Q4_0 on 4-wave 32x128 blocks (default)

@@ -1,5 +1,5 @@
-/* fp16 operands of the matrix-core kernels: conversions of packed codes to halves and the IQ lookup
- * tables in fragment order (the eight K positions of a lane's fragment in the order P8 = 0,2,1,3,4,6,5,7,
+/* Shared by the matrix-core GEMM kernels: the grouped form's tiles, conversions of packed codes to halves and the IQ
+ * lookup tables in fragment order (the eight K positions of a lane's fragment in the order P8 = 0,2,1,3,4,6,5,7,
  * what the byte-pair conversion produces). */
 #pragma once
 #include "le_qmm_device.h"
@@ -75,4 +75,56 @@ __device__ __forceinline__ void gq_tables(u8 *tab) {
             *(uint4 *)(sg + 16 * i) = make_uint4(m[0], m[1], m[2], m[3]);
         }
     }
+}
+
+/* Tiles of the grouped form: slot s has off[s+1] - off[s] pairs, split into tiles of bm, listed
+ * slot by slot. Each wave derives what it needs from off itself (no planning launch): the slots'
+ * counts are loaded 256 at a time, all in flight together, then scanned across the wave. */
+__device__ __forceinline__ int le_wave_scan(int v) { /* inclusive prefix sum over the wave, by DPP */
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, true); /* row_shr:1 (rows of 16 lanes) */
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, true); /* row_shr:2 */
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, true); /* row_shr:4 */
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, true); /* row_shr:8 */
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false); /* row_bcast:15 into rows 1, 3 */
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false); /* row_bcast:31 into rows 2, 3 */
+    return v;
+}
+/* Walk the slots 256 at a time (every load of a round in flight together), each lane holding one
+ * slot's first pair o0, its tile count c and the number of tiles before it; stop at the first
+ * slot for which hit(o0, o1, first, c) holds on some lane. Returns that slot (or -1) and, through
+ * the references, its first pair and first tile. Uniform over the wave. */
+template <class Hit>
+__device__ __forceinline__ int le_slot_walk(const int *__restrict__ off, int nslot, int bm, Hit hit, int &o0_out, int &first_out) {
+    const int lane = threadIdx.x & 63;
+    int base = 0;
+    for (int s0 = 0; s0 < nslot; s0 += 256) {
+        int o0[4], o1[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int s = min(s0 + 64 * q + lane, nslot - 1);
+            o0[q] = off[s];
+            o1[q] = off[s + 1];
+        }
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const bool in = s0 + 64 * q + lane < nslot;
+            const int c = in ? (max(o1[q] - o0[q], 0) + bm - 1) / bm : 0, inc = le_wave_scan(c), first = base + inc - c;
+            const unsigned long long h = __ballot(in && c > 0 && hit(o0[q], o1[q], first, c));
+            if (h) {
+                const int l = __ffsll((long long)h) - 1;
+                o0_out = __shfl(o0[q], l);
+                first_out = __shfl(first, l);
+                return s0 + 64 * q + l;
+            }
+            base += __shfl(inc, 63);
+        }
+    }
+    return -1;
+}
+/* tile mt: its slot and first pair (false past the last tile) */
+__device__ __forceinline__ bool le_tile_of(const int *__restrict__ off, int nslot, int bm, int mt, int &slot, int &pair0) {
+    int o0, first;
+    slot = le_slot_walk(off, nslot, bm, [mt](int, int, int f, int c) { return mt >= f && mt < f + c; }, o0, first);
+    pair0 = o0 + (mt - first) * bm;
+    return slot >= 0;
 }

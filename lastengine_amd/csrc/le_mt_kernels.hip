@@ -23,11 +23,15 @@
  * matvec does. blockIdx.y: K slices whose partial results le_gq_ksum adds in slice order (only where the
  * images of all of K do not fit the LDS).
  *
+ * Grouped form le_mtg_* (the MoE layer's few tokens an expert; grouped mm, src/cuda/kernels.cu:679-719): ng
+ * blocks share a tile of up to T pairs of one slot, rounded once, and optionally gate and up in one launch. It
+ * has no pre-pass (a launch and a pass over the images less) and no padding to 32 pairs; figures where it is chosen.
+ *
  * It replaces, below nine tokens, vector kernels that unpack every weight for each pair of tokens, and to 16
- * tokens the larger GEMM. Measured at 4 / 8 / 16 tokens: Q6_K 4096 x 14336 67.3 -> 25.7, 124 -> 22.6, 30.6 ->
- * 30.7 us; Q8_0 32000 x 4096 69.9 -> 32.3, 94.9 -> 36.4, 51.8 -> 36.0; IQ2_XXS 14336 x 4096 34.3 -> 16.1,
- * 47.8 -> 17.8, 27.1 -> 19.6. Bound by the decoding (Q6_K: about 250 VALU instructions a super-block) and, for
- * small matrices, by each block's image build (2 -> 8 tokens of Q4_0 4096 x 4096: 7.4 -> 10.3 us). */
+ * tokens the larger GEMM. Measured at 4 / 8 / 16 tokens: Q6_K 4096 x 14336 67.0 -> 24.8, 124 -> 22.2, 30.6 ->
+ * 29.7 us; Q8_0 32000 x 4096 69.8 -> 32.4, 94.3 -> 34.2, 51.7 -> 36.0; IQ2_XXS 14336 x 4096 34.3 -> 16.1,
+ * 47.9 -> 18.3, 27.1 -> 19.9. Bound by the decoding (Q6_K: about 240 VALU instructions a super-block, Q4_K 156) and,
+ * for small matrices, by each block's image build (2 -> 8 tokens of Q4_0 4096 x 4096: 7.6 -> 10.5 us). */
 #include "le_f16_frag.h"
 
 typedef float le_v4f __attribute__((ext_vector_type(4)));
@@ -37,6 +41,17 @@ struct MtArgs {
     const float *x;
     float *y, *part; /* part: [slices][m][rows], or null with one slice */
     int rows, cols, m, kw;
+    /* grouped form: slot s multiplies weight ptrs[s] (or w + s * w_slot_bytes) with the rows in_idx[i] of x (with
+     * up: silu(x) * up) of its pairs i in off[s] .. off[s+1], writing output rows out_idx[i]; dual: a second weight
+     * set (ptrs2 or w2, same shape) into y2 */
+    const u8 *const *ptrs;
+    unsigned long long w_slot_bytes;
+    const int *off, *in_idx, *out_idx;
+    int nslot, maxt, ng, dual;
+    const u8 *const *ptrs2;
+    const u8 *w2;
+    float *y2;
+    const float *up;
 };
 
 /* staged super-blocks: CPS 16-byte chunks, chunk c read from byte goff(c) */
@@ -103,6 +118,11 @@ __device__ __forceinline__ le_v8h mt_codes_sc(u32 x, u32 y, u32 bias, u32 sc) {
     return as_v8h(make_uint4(pk_mul(pk_add(h1024_02(x), bias), sc), pk_mul(pk_add(h1024_13(x), bias), sc),
                              pk_mul(pk_add(h1024_02(y), bias), sc), pk_mul(pk_add(h1024_13(y), bias), sc)));
 }
+/* bytes times sc, exact: (1024 + u) sc - 1024 sc in one rounding; 1024 sc has to be finite (sc < 64) */
+__device__ __forceinline__ le_v8h mt_codes_fma(u32 x, u32 y, u32 sc) {
+    const u32 k = pk_mul(sc, 0xE400E400u);
+    return as_v8h(make_uint4(pk_fma(h1024_02(x), sc, k), pk_fma(h1024_13(x), sc, k), pk_fma(h1024_02(y), sc, k), pk_fma(h1024_13(y), sc, k)));
+}
 __device__ __forceinline__ le_v8h mt_grid(uint4 g, uint4 m, u32 f) {
     return as_v8h(make_uint4(pk_mul(g.x, f) ^ m.x, pk_mul(g.y, f) ^ m.y, pk_mul(g.z, f) ^ m.z, pk_mul(g.w, f) ^ m.w));
 }
@@ -114,7 +134,12 @@ template <int TY, int R, int RS>
 __device__ __forceinline__ void mt_sb(const u8 *sb, const uint4 *a, int lane, float4 st, const u8 *tab, le_v4f &y) {
     const int g = lane >> 4, m = lane & 15;
     const u32 *w32 = (const u32 *)sb;
-    auto A = [&](int j) { return as_v8h(a[(4 * j + g) * RS + (m & (R - 1))]); }; /* R = 8: MFMA rows 8-15 repeat 0-7, unused */
+    /* the super-block's LDS reads all first: read where they are used, each MFMA waited out one of them
+     * (about 1 us an item with two waves on a SIMD) */
+    uint4 Af[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) Af[j] = a[(4 * j + g) * RS + (m & (R - 1))]; /* R = 8: MFMA rows 8-15 repeat 0-7, unused */
+    auto A = [&](int j) { return as_v8h(Af[j]); };
     auto mm = [](le_v8h x, le_v8h w, le_v4f d) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(x, w, d, 0, 0, 0); };
     le_v4f D = {0.f, 0.f, 0.f, 0.f};
     float d;
@@ -122,11 +147,15 @@ __device__ __forceinline__ void mt_sb(const u8 *sb, const uint4 *a, int lane, fl
         constexpr bool Q5 = TY == LE_TYPE_Q5_K;
         const uint4 hd = *(const uint4 *)sb;
         const u32 sc[2] = {hd.y & 0x3F3F3F3Fu, (hd.w & 0x0F0F0F0Fu) | ((hd.y >> 2) & 0x30303030u)};
-        uint2 qh = make_uint2(0, 0);
+        uint2 qh = make_uint2(0, 0), qv[4];
         if constexpr (Q5) qh = *(const uint2 *)(sb + 16 + 8 * g);
 #pragma unroll
+        for (int G = 0; G < 4; G++) qv[G] = *(const uint2 *)(sb + (Q5 ? 48 : 16) + 32 * G + 8 * g);
+        const le_v8h S = as_v8h(a[(32 + (g & 1)) * RS + (m & (R - 1))]);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
         for (int G = 0; G < 4; G++) {
-            const uint2 q = *(const uint2 *)(sb + (Q5 ? 48 : 16) + 32 * G + 8 * g);
+            const uint2 q = qv[G];
 #pragma unroll
             for (int hi = 0; hi < 2; hi++) {
                 const int j = 2 * G + hi;
@@ -135,12 +164,11 @@ __device__ __forceinline__ void mt_sb(const u8 *sb, const uint4 *a, int lane, fl
                     x |= ((qh.x >> j) & 0x01010101u) << 4;
                     z |= ((qh.y >> j) & 0x01010101u) << 4;
                 }
-                D = mm(A(j), mt_codes_sc(x, z, 0xE400E400u, pk_add(h1024_dup(sc[j >> 2], j & 3), 0xE400E400u)), D);
+                D = mm(A(j), mt_codes_fma(x, z, pk_add(h1024_dup(sc[j >> 2], j & 3), 0xE400E400u)), D);
             }
         }
         const u32 m0 = hd.z & 0x3F3F3F3Fu, m1 = ((hd.w >> 4) & 0x0F0F0F0Fu) | ((hd.z >> 2) & 0x30303030u);
         /* K positions 16-31 of the offset MFMA: zero mins */
-        const le_v8h S = as_v8h(a[(32 + (g & 1)) * RS + (m & (R - 1))]);
         const u32 k2 = g < 2 ? ~0u : 0u;
         const le_v4f O = mm(S, mt_codes(m0 & k2, m1 & k2, 0xE400E400u), (le_v4f){0.f, 0.f, 0.f, 0.f});
         d = h2f(hd.x & 0xFFFFu);
@@ -151,30 +179,37 @@ __device__ __forceinline__ void mt_sb(const u8 *sb, const uint4 *a, int lane, fl
     } else if constexpr (TY == LE_TYPE_Q6_K) {
         /* value 128 hn + 32 s + l: ql byte 64 hn + 32 (s & 1) + l (nibble s / 2), qh byte 32 hn + l bits 2s, scale 8 hn + 2 s + l / 16 */
         const uint4 scv = *(const uint4 *)(sb + 192);
-        const u32 scw[4] = {scv.x, scv.y, scv.z, scv.w};
+        const u32 scw[4] = {scv.x, scv.y, scv.z, scv.w}, dw = *(const u32 *)(sb + 220);
+        uint2 qlv[4], qhv[2];
+#pragma unroll
+        for (int i = 0; i < 4; i++) qlv[i] = *(const uint2 *)(sb + 32 * i + 8 * g);
+#pragma unroll
+        for (int hn = 0; hn < 2; hn++) qhv[hn] = *(const uint2 *)(sb + 128 + 32 * hn + 8 * g);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int hn = 0; hn < 2; hn++) {
-            const uint2 qa = *(const uint2 *)(sb + 64 * hn + 8 * g), qb = *(const uint2 *)(sb + 64 * hn + 32 + 8 * g);
-            const uint2 qh = *(const uint2 *)(sb + 128 + 32 * hn + 8 * g);
+            const uint2 qh = qhv[hn];
 #pragma unroll
             for (int s = 0; s < 4; s++) {
-                const uint2 ql = s & 1 ? qb : qa;
+                const uint2 ql = qlv[2 * hn + (s & 1)];
                 const u32 w = scw[2 * hn + (s >> 1)] ^ 0x80808080u; /* scales 8 hn + 2 s, + 1 in bytes 2 (s & 1), + 1 */
-                const u32 sc = pk_add(h1024_dup((w >> (16 * (s & 1) + 8 * (g >> 1))) & 255u, 0), 0xE480E480u); /* byte - 1152 */
+                /* scale / 16, from the byte under the exponent of 64: 1024 times the scale itself can pass 65504 */
+                const u32 sc = pk_add(__builtin_amdgcn_perm(0x54545454u, w, (s & 1 ? 0x04020402u : 0x04000400u) + (u32)(g >> 1) * 0x00010001u), 0xD480D480u);
                 const le_v8h av = A(4 * hn + s);
-                D = mm(av, mt_codes_sc((ql.x >> (4 * (s >> 1))) & 0x0F0F0F0Fu, (ql.y >> (4 * (s >> 1))) & 0x0F0F0F0Fu, 0xE400E400u, sc), D);
+                D = mm(av, mt_codes_fma((ql.x >> (4 * (s >> 1))) & 0x0F0F0F0Fu, (ql.y >> (4 * (s >> 1))) & 0x0F0F0F0Fu, sc), D);
                 const u32 hx = s < 2 ? qh.x << (4 - 2 * s) : qh.x >> (2 * s - 4), hy = s < 2 ? qh.y << (4 - 2 * s) : qh.y >> (2 * s - 4);
                 D = mm(av, mt_codes_sc(hx & 0x30303030u, hy & 0x30303030u, 0xE420E420u, sc), D); /* 16 qh - 32 */
             }
         }
-        d = h2f(*(const u32 *)(sb + 220) >> 16);
+        d = 16.f * h2f(dw >> 16);
     } else if constexpr (TY == LE_TYPE_Q3_K) {
         const uint4 c6 = *(const uint4 *)(sb + 96);
         const u32 s0 = __builtin_amdgcn_alignbyte(c6.y, c6.x, 2), s1 = __builtin_amdgcn_alignbyte(c6.z, c6.y, 2), s2 = __builtin_amdgcn_alignbyte(c6.w, c6.z, 2);
-        const uint2 hm = *(const uint2 *)(sb + 8 * g);
+        const uint2 hm = *(const uint2 *)(sb + 8 * g), qv[2] = {*(const uint2 *)(sb + 32 + 8 * g), *(const uint2 *)(sb + 64 + 8 * g)};
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int hn = 0; hn < 2; hn++) {
-            const uint2 qs = *(const uint2 *)(sb + 32 + 32 * hn + 8 * g);
+            const uint2 qs = qv[hn];
             /* scales 8 hn + i: low 4 bits nibble hn of byte i, bits 4-5 from byte 8 + i % 4 */
             const u32 v[2] = {((s0 >> (4 * hn)) & 0x0F0F0F0Fu) | (((s2 >> (4 * hn)) & 0x03030303u) << 4),
                               ((s1 >> (4 * hn)) & 0x0F0F0F0Fu) | (((s2 >> (4 * hn + 2)) & 0x03030303u) << 4)};
@@ -188,50 +223,91 @@ __device__ __forceinline__ void mt_sb(const u8 *sb, const uint4 *a, int lane, fl
         }
         d = h2f(c6.w >> 16);
     } else if constexpr (TY == LE_TYPE_IQ2_S) {
+        u32 w[24]; /* the index, sign, high-bit and scale words */
 #pragma unroll
-        for (int j = 0; j < 8; j++) { /* index byte 2 + 4 j + g, sign byte 34 + 4 j + g (2 mod 4 aligned) */
-            const u32 q = __builtin_amdgcn_alignbit(w32[j + 1], w32[j], 16), sg = __builtin_amdgcn_alignbit(w32[9 + j], w32[8 + j], 16);
-            const u32 qh = (w32[20 + (j >> 2)] >> (8 * (j & 3))) & 255u, sc = (w32[22 + (j >> 2)] >> (8 * (j & 3) + 4 * (g >> 1))) & 15u;
-            const u32 gi = ((q >> (8 * g)) & 255u) | ((qh << (8 - 2 * g)) & 0x300u);
-            const u32 f = pk_add(h1024_dup(2u * sc + 1u, 0), 0xE400E400u);
-            D = mm(A(j), mt_grid(*(const uint4 *)(tab + 16 * gi), *(const uint4 *)(tab + 16384 + 16 * ((sg >> (8 * g)) & 255u)), f), D);
+        for (int i = 0; i < 24; i++) w[i] = i == 18 || i == 19 ? 0u : w32[i];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            uint4 gv[4], sv[4];
+            u32 f[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) { /* index byte 2 + 4 j + g, sign byte 34 + 4 j + g (2 mod 4 aligned) */
+                const int j = 4 * h + i;
+                const u32 q = __builtin_amdgcn_alignbit(w[j + 1], w[j], 16), sg = __builtin_amdgcn_alignbit(w[9 + j], w[8 + j], 16);
+                const u32 qh = (w[20 + h] >> (8 * i)) & 255u, sc = (w[22 + h] >> (8 * i + 4 * (g >> 1))) & 15u;
+                const u32 gi = ((q >> (8 * g)) & 255u) | ((qh << (8 - 2 * g)) & 0x300u);
+                f[i] = pk_add(h1024_dup(2u * sc + 1u, 0), 0xE400E400u);
+                gv[i] = *(const uint4 *)(tab + 16 * gi);
+                sv[i] = *(const uint4 *)(tab + 16384 + 16 * ((sg >> (8 * g)) & 255u));
+            }
+#pragma unroll
+            for (int i = 0; i < 4; i++) D = mm(A(4 * h + i), mt_grid(gv[i], sv[i], f[i]), D);
         }
-        d = 0.125f * h2f(w32[0] & 0xFFFFu);
+        d = 0.125f * h2f(w[0] & 0xFFFFu);
     } else if constexpr (TY == LE_TYPE_IQ2_XXS || TY == LE_TYPE_IQ3_XXS) {
         constexpr bool I2 = TY == LE_TYPE_IQ2_XXS;
         const u8 *sgt = tab + (I2 ? 4096 : 2048);
+        uint2 qv[8];
+        u32 av[8];
 #pragma unroll
         for (int j = 0; j < 8; j++) {
-            const uint2 q = *(const uint2 *)(sb + 8 * j);
-            const u32 aux = I2 ? q.y : *(const u32 *)(sb + 64 + 4 * j);
-            const u32 f = pk_add(h1024_dup(2u * (aux >> 28) + 1u, 0), 0xE400E400u);
-            const uint4 sg = *(const uint4 *)(sgt + 16 * ((aux >> (7 * g)) & 127u));
-            uint4 gv;
-            if constexpr (I2) {
-                gv = *(const uint4 *)(tab + 16 * ((q.x >> (8 * g)) & 255u));
-            } else {
-                const u32 iw = (g < 2 ? q.x : q.y) >> (16 * (g & 1));
-                const uint2 g0 = *(const uint2 *)(tab + 8 * (iw & 255u)), g1 = *(const uint2 *)(tab + 8 * ((iw >> 8) & 255u));
-                gv = make_uint4(g0.x, g0.y, g1.x, g1.y);
-            }
-            D = mm(A(j), mt_grid(gv, sg, f), D);
+            qv[j] = *(const uint2 *)(sb + 8 * j);
+            av[j] = I2 ? qv[j].y : *(const u32 *)(sb + 64 + 4 * j);
         }
-        d = (I2 ? 0.125f : 0.25f) * h2f(*(const u32 *)(sb + (I2 ? 64 : 96)) & 0xFFFFu);
+        const u32 dw = *(const u32 *)(sb + (I2 ? 64 : 96));
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            uint4 gv[4], sv[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const uint2 q = qv[4 * h + i];
+                sv[i] = *(const uint4 *)(sgt + 16 * ((av[4 * h + i] >> (7 * g)) & 127u));
+                if constexpr (I2) {
+                    gv[i] = *(const uint4 *)(tab + 16 * ((q.x >> (8 * g)) & 255u));
+                } else {
+                    const u32 iw = (g < 2 ? q.x : q.y) >> (16 * (g & 1));
+                    const uint2 g0 = *(const uint2 *)(tab + 8 * (iw & 255u)), g1 = *(const uint2 *)(tab + 8 * ((iw >> 8) & 255u));
+                    gv[i] = make_uint4(g0.x, g0.y, g1.x, g1.y);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const u32 f = pk_add(h1024_dup(2u * (av[4 * h + i] >> 28) + 1u, 0), 0xE400E400u);
+                D = mm(A(4 * h + i), mt_grid(gv[i], sv[i], f), D);
+            }
+        }
+        d = (I2 ? 0.125f : 0.25f) * h2f(dw & 0xFFFFu);
     } else { /* Q8_0, Q4_0: one scale per sub-block */
         constexpr bool Q8 = TY == LE_TYPE_Q8_0;
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const u8 *b = sb + (Q8 ? 34 : 18) * j;
-            const u32 dw = *(const u32 *)(b - ((size_t)b & 3));
-            const float dj = h2f((dw >> (((size_t)b & 2) * 8)) & 0xFFFFu);
-            uint2 q = mt_lds8_a2(b + 2 + (Q8 ? 8 * g : 8 * (g & 1)));
-            if constexpr (Q8)
-                q = make_uint2(q.x ^ 0x80808080u, q.y ^ 0x80808080u);
-            else
-                q = make_uint2((q.x >> (4 * (g >> 1))) & 0x0F0F0F0Fu, (q.y >> (4 * (g >> 1))) & 0x0F0F0F0Fu);
-            const le_v4f Dj = mm(A(j), mt_codes(q.x, q.y, Q8 ? 0xE480E480u : 0xE408E408u), (le_v4f){0.f, 0.f, 0.f, 0.f});
+        for (int h = 0; h < 2; h++) {
+            uint2 qv[4];
+            u32 dw[4];
 #pragma unroll
-            for (int e = 0; e < 4; e++) D[e] = __builtin_fmaf(dj, Dj[e], D[e]);
+            for (int i = 0; i < 4; i++) {
+                const u8 *b = sb + (Q8 ? 34 : 18) * (4 * h + i);
+                dw[i] = *(const u32 *)(b - ((size_t)b & 3)) >> (((size_t)b & 2) * 8);
+                qv[i] = mt_lds8_a2(b + 2 + (Q8 ? 8 * g : 8 * (g & 1)));
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            le_v4f Dj[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                uint2 q = qv[i];
+                if constexpr (Q8)
+                    q = make_uint2(q.x ^ 0x80808080u, q.y ^ 0x80808080u);
+                else
+                    q = make_uint2((q.x >> (4 * (g >> 1))) & 0x0F0F0F0Fu, (q.y >> (4 * (g >> 1))) & 0x0F0F0F0Fu);
+                Dj[i] = mm(A(4 * h + i), mt_codes(q.x, q.y, Q8 ? 0xE480E480u : 0xE408E408u), (le_v4f){0.f, 0.f, 0.f, 0.f});
+            }
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const float dj = h2f(dw[i] & 0xFFFFu);
+#pragma unroll
+                for (int e = 0; e < 4; e++) D[e] = __builtin_fmaf(dj, Dj[i][e], D[e]);
+            }
         }
         d = 1.f;
     }
@@ -257,15 +333,23 @@ __device__ __forceinline__ float mt_dpp_add(float v) {
 /* sum over the lane's group of eight */
 __device__ __forceinline__ float mt_sum8(float v) { return mt_dpp_add<0x141>(mt_dpp_add<0x4E>(mt_dpp_add<0xB1>(v))); } /* xor 1, xor 2, half-row mirror */
 
-template <int TY, int T>
+/* T tokens (GR: pairs of one slot) per pass, HL: as two halves */
+template <int TY, int T, bool HL, bool GR>
 __device__ __forceinline__ void mt_body(const MtArgs &a) {
     using F = MtF<TY>;
-    constexpr bool HL = T <= 8, OFS = TY == LE_TYPE_Q4_K || TY == LE_TYPE_Q5_K, AL = OFS; /* AL: 16-byte aligned weights */
+    constexpr bool OFS = TY == LE_TYPE_Q4_K || TY == LE_TYPE_Q5_K, AL = OFS; /* AL: 16-byte aligned weights */
     constexpr int R = HL ? 2 * T : T, RS = R + 1;              /* live MFMA rows; slots per fragment (odd: rows of the build's stores in distinct banks) */
     constexpr int IMG = (32 + (OFS ? 2 : 0)) * RS;             /* 16-byte slots of a super-block's image */
     constexpr int NW = 8, CPR = F::CPS | 1, NCH = 16 * F::CPS, NI = (NCH + 63) / 64;
     extern __shared__ uint4 smem[];
     const int nsb = a.cols >> 8, ns = (int)gridDim.y;
+    int M = a.m, bx = blockIdx.x, gx = gridDim.x, pair0 = 0, slot = 0;
+    if constexpr (GR) { /* ng blocks share a tile of up to T pairs of one slot */
+        gx = a.ng;
+        if (!le_tile_of(a.off, a.nslot, T, bx / gx, slot, pair0)) return; /* uniform: past the last tile */
+        bx %= gx;
+        M = min(T, a.off[slot + 1] - pair0);
+    }
     const int sb0 = (int)blockIdx.y * nsb / ns, sb1 = ((int)blockIdx.y + 1) * nsb / ns, nsl = sb1 - sb0;
     const int most = (nsb + ns - 1) / ns; /* the launch's LDS holds the longest slice */
     uint4 *img = smem;
@@ -273,12 +357,12 @@ __device__ __forceinline__ void mt_body(const MtArgs &a) {
     uint4 *stg = (uint4 *)(stab + most * 16);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = lane & 15;
     uint4 *wb = stg + wave * 16 * CPR;
-    float4 *red = (float4 *)(stg + NW * 16 * CPR);             /* [2][NW][4 T lanes] */
-    u8 *tab = (u8 *)(red + 2 * NW * 4 * T);
+    u8 *tab = (u8 *)(stg + NW * 16 * CPR);
+    float4 *red = (float4 *)(tab + mt_tab<TY>());              /* [2][NW][4 T lanes], with kw > 1 */
     if constexpr (mt_tab<TY>() > 0) gq_tables<TY>(tab);
 
     const int KW = a.kw, RT = NW / KW, kw = wave % KW, rt = wave / KW;
-    const int ntile = (a.rows + 15) >> 4, mine = (nsl + KW - 1 - kw) / KW; /* super-blocks kw, kw + KW, ... of the slice */
+    const int ntr = (a.rows + 15) >> 4, ntile = GR && a.dual ? 2 * ntr : ntr, mine = (nsl + KW - 1 - kw) / KW; /* super-blocks kw, kw + KW, ... of the slice */
     const size_t rb = (size_t)nsb * F::SBB;
     int ri[NI], gb[NI], wl[NI];
 #pragma unroll
@@ -288,21 +372,27 @@ __device__ __forceinline__ void mt_body(const MtArgs &a) {
         gb[i] = F::goff(c % F::CPS);
         wl[i] = c + (CPR - F::CPS) * ri[i];
     }
+    const u8 *w1 = a.w, *w2 = nullptr;
+    if constexpr (GR) {
+        w1 = a.ptrs ? a.ptrs[slot] : a.w + (size_t)slot * a.w_slot_bytes;
+        if (a.dual) w2 = a.ptrs2 ? a.ptrs2[slot] : a.w2 + (size_t)slot * a.w_slot_bytes;
+    }
     uint4 W[NI];
     auto issue = [&](int tile, int sb) {
 #pragma unroll
         for (int i = 0; i < NI; i++) {
-            const u8 *p = a.w + (size_t)min(tile * 16 + ri[i], a.rows - 1) * rb + (size_t)sb * F::SBB + gb[i];
+            const u8 *p = (GR && tile >= ntr ? w2 : w1) + (size_t)min((GR && tile >= ntr ? tile - ntr : tile) * 16 + ri[i], a.rows - 1) * rb +
+                          (size_t)sb * F::SBB + gb[i];
             W[i] = AL ? ldg16(p) : ldg16u(p);
         }
     };
-    const int t0 = blockIdx.x * RT, tstep = gridDim.x * RT;
+    const int t0 = bx * RT, tstep = gx * RT;
 
     /* images: one (token, super-block) per wave and turn, four values per lane; a first batch of eight
      * turns' activations is loaded before the first weights (loads retire in order: behind them they
      * would wait for the weights) */
     {
-        const int j = lane >> 3, g = (lane & 7) >> 1, np = a.m * nsl;
+        const int j = lane >> 3, g = (lane & 7) >> 1, np = M * nsl;
         const float inv = __builtin_amdgcn_rcpf((float)nsl);
         const LE_GLOBAL float4 *x4 = (const LE_GLOBAL float4 *)a.x;
         auto split = [&](int p, int &t, int &sl) { /* p = t nsl + sl; p < 2^12, and p + 1/2 keeps the quotient off the integers */
@@ -315,7 +405,9 @@ __device__ __forceinline__ void mt_body(const MtArgs &a) {
             for (int u = 0; u < 8; u++) {
                 int t, sl;
                 split(__builtin_amdgcn_readfirstlane(min(p0 + u * NW, np - 1)), t, sl);
-                v[u] = x4[((size_t)t * a.cols + (size_t)(sb0 + sl) * 256) / 4 + lane];
+                const size_t o = ((size_t)(GR ? a.in_idx[pair0 + t] : t) * a.cols + (size_t)(sb0 + sl) * 256) / 4 + lane;
+                v[u] = x4[o];
+                if (GR && a.up) v[u] = le_silu_mul4(v[u], ((const LE_GLOBAL float4 *)a.up)[o]);
             }
         };
         xload(wave);
@@ -368,7 +460,7 @@ __device__ __forceinline__ void mt_body(const MtArgs &a) {
     }
     __syncthreads();
 
-    float *out = a.part ? a.part + (size_t)blockIdx.y * a.m * a.rows : a.y;
+    float *out1 = a.part ? a.part + (size_t)blockIdx.y * a.m * a.rows : a.y;
     int par = 0;
     for (int tb = t0; tb < ntile; tb += tstep) {
         const int tile = tb + rt;
@@ -403,18 +495,22 @@ __device__ __forceinline__ void mt_body(const MtArgs &a) {
                 }
             par ^= 1;
         }
-        const int r = tile * 16 + n;
+        const bool second = GR && tile >= ntr;
+        float *out = second ? a.y2 : out1;
+        const int r = (second ? tile - ntr : tile) * 16 + n;
         if (kw == 0 && lane < 4 * T && tile < ntile && r < a.rows) {
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 const int t = 4 * (lane >> 4) + e;
-                if (t < a.m) out[(size_t)t * a.rows + r] = y[e];
+                if (t < M) out[(size_t)(GR ? a.out_idx[pair0 + t] : t) * a.rows + r] = y[e];
             }
         }
     }
 }
 
 #define LE_MT_(TY, T) \
-    extern "C" __global__ void __launch_bounds__(512) le_mt_##TY##_t##T(MtArgs a) { mt_body<TY, T>(a); }
-#define LE_MT(TY) LE_MT_(TY, 4) LE_MT_(TY, 8) LE_MT_(TY, 16)
+    extern "C" __global__ void __launch_bounds__(512) le_mt_##TY##_t##T(MtArgs a) { mt_body<TY, T, T <= 8, false>(a); }
+#define LE_MTG_(TY, T) \
+    extern "C" __global__ void __launch_bounds__(512) le_mtg_##TY##_t##T(MtArgs a) { mt_body<TY, T, false, true>(a); }
+#define LE_MT(TY) LE_MT_(TY, 4) LE_MT_(TY, 8) LE_MT_(TY, 16) LE_MTG_(TY, 8) LE_MTG_(TY, 16)
 LE_MT(2) LE_MT(8) LE_MT(11) LE_MT(12) LE_MT(13) LE_MT(14) LE_MT(16) LE_MT(18) LE_MT(22)

@@ -132,6 +132,7 @@ struct le_ctx {
                                 pipelined kernel with 128 / 64 tokens a block */
     int gq_ksplit = 0;       /* generic GEMM K slices: 0 auto, else 1, 2, 4, 8 */
     int moe_route1 = 1;      /* grouped MoE up to 32 tokens: routing and grouping in one block */
+    int mmg_mt = 1;          /* grouped form of up to six pairs a slot: few-pair kernel */
     int mmg_gp = 1;          /* grouped form of Q4_K / Q5_K on the pipelined kernel */
     int mmg_w4 = 1;          /* grouped 32-pair tiles: 4-wave 32 x 128 blocks where 8-wave ones fill half the LDS */
     int mmg_xw = 1;          /* grouped pre-pass: one wave per pair (K <= 4096) instead of one block */
@@ -597,6 +598,8 @@ int le_set_option(le_ctx *c, const char *name, int value) {
         c->moe_route1 = value ? 1 : 0;
     } else if (n == "mmg_w4") {
         c->mmg_w4 = value ? 1 : 0;
+    } else if (n == "mmg_mt") {
+        c->mmg_mt = value ? 1 : 0;
     } else if (n == "mmg_gp") {
         c->mmg_gp = value ? 1 : 0;
     } else if (n == "mmg_xw") {
@@ -1088,16 +1091,32 @@ static int gq_tab(int ty) {
 /* Few tokens (m <= 16), every type: le_mt_*. Returns 1 where it does not apply (the caller goes on). The
  * partial results of K slices (needed where the activation images of all of K exceed the LDS) go to the
  * workspace; without room for them it does not apply. */
+struct MtHostArgs { /* MtArgs in le_mt_kernels.hip */
+    const void *w;
+    const float *x;
+    float *y, *part;
+    int rows, cols, m, kw;
+    const void *const *ptrs;
+    unsigned long long w_slot_bytes;
+    const int *off, *in_idx, *out_idx;
+    int nslot, maxt, ng, dual;
+    const void *const *ptrs2;
+    const void *w2;
+    float *y2;
+    const float *up;
+};
+/* LDS of a le_mt block: images of `most` super-blocks with R MFMA rows, scales, staging, the waves' sums (kw > 1) */
+static size_t mt_lds(int ty, int most, int R, int T, bool sums) {
+    const bool ofs = ty == LE_TYPE_Q4_K || ty == LE_TYPE_Q5_K;
+    const int cps = ty == LE_TYPE_Q6_K ? 14 : ty == LE_TYPE_IQ2_XXS ? 5 : ty == LE_TYPE_IQ3_XXS ? 7 : ty == LE_TYPE_Q8_0 ? 17 : ty == LE_TYPE_Q5_K ? 11 : ty == LE_TYPE_Q3_K ? 7 : ty == LE_TYPE_IQ2_S ? 6 : 9;
+    return (size_t)most * ((size_t)(32 + (ofs ? 2 : 0)) * (R + 1) * 16 + 64) + (size_t)8 * 16 * (cps | 1) * 16 + (sums ? (size_t)2 * 8 * 4 * T * 16 : 0) +
+           gq_tab(ty);
+}
 static int mt_launch(le_ctx *c, int ty, const void *w, const float *x, int m, float *y, int rows, int cols, void *ws,
                      size_t ws_bytes, hipStream_t st) {
     const int T = m <= 4 ? 4 : m <= 8 ? 8 : 16, R = T == 4 ? 8 : 16, NW = 8;
     const int nsb = cols / 256, ntile = (rows + 15) / 16;
-    const bool ofs = ty == LE_TYPE_Q4_K || ty == LE_TYPE_Q5_K;
-    const int cps = ty == LE_TYPE_Q6_K ? 14 : ty == LE_TYPE_IQ2_XXS ? 5 : ty == LE_TYPE_IQ3_XXS ? 7 : ty == LE_TYPE_Q8_0 ? 17 : ty == LE_TYPE_Q5_K ? 11 : ty == LE_TYPE_Q3_K ? 7 : ty == LE_TYPE_IQ2_S ? 6 : 9;
-    auto lds_of = [&](int ks) {
-        const size_t most = (nsb + ks - 1) / ks;
-        return most * ((size_t)(32 + (ofs ? 2 : 0)) * (R + 1) * 16 + 64) + (size_t)NW * 16 * (cps | 1) * 16 + (size_t)2 * NW * 4 * T * 16 + gq_tab(ty);
-    };
+    auto lds_of = [&](int ks) { return mt_lds(ty, (nsb + ks - 1) / ks, R, T, true); };
     int ks = 1;
     while (ks < nsb && lds_of(ks) > c->lds_limit) ks++;
     const size_t lds = lds_of(ks);
@@ -1112,15 +1131,18 @@ static int mt_launch(le_ctx *c, int ty, const void *w, const float *x, int m, fl
     if (!c->fn(name)) return 1;
     /* waves per row tile: the fewest that give every CU a block (fewer: longer chains, no sum through LDS) */
     int kw = 1;
-    while (kw < NW && (long long)ntile * kw * ks < (long long)NW * c->cus) kw *= 2;
+    while (kw < NW && 2 * kw <= nsb / ks && (long long)ntile * kw * ks < (long long)NW * c->cus) kw *= 2;
     const int groups = (ntile + NW / kw - 1) / (NW / kw), per_cu = c->blocks_per_cu(name, 64 * NW, lds);
     const int cap = std::max(1, c->cus * std::max(1, per_cu) / ks), it = (groups + cap - 1) / cap, gx = (groups + it - 1) / it;
-    struct {
-        const void *w;
-        const float *x;
-        float *y, *part;
-        int rows, cols, m, kw;
-    } a{w, x, y, part, rows, cols, m, kw};
+    MtHostArgs a{};
+    a.w = w;
+    a.x = x;
+    a.y = y;
+    a.part = part;
+    a.rows = rows;
+    a.cols = cols;
+    a.m = m;
+    a.kw = kw;
     void *args[] = {&a};
     int rc = c->launch(name, dim3((unsigned)gx, (unsigned)ks), 64 * NW, lds, st, args);
     if (rc || !part) return rc;
@@ -1247,6 +1269,47 @@ static int mm_grouped(le_ctx *c, int ty, const void *const *ptrs, const void *w,
     const size_t need = le_mm_grouped_workspace_size(ty, nslot, npair, cols);
     if (ws_bytes < need) return c->fail(LE_ERR_WORKSPACE, "workspace needs %zu bytes", need);
     if (npair == 0) return LE_OK;
+    /* Few pairs a slot: le_mtg_*, 8 or 16 pairs a pass. A whole MoE layer, tiles of 32 pairs against this, 128
+     * experts of 2048 x 768, 8 a token, Q4_K and Q6_K: 12 / 24 / 32 / 64 / 96 tokens (0.75 to 6 pairs a slot)
+     * 96.1 / 111 / 128 / 142 / 148 -> 81.6 / 103 / 114 / 129 / 132 us; at 128 tokens (8) 154 -> 182. IQ2_XXS and IQ3_XXS,
+     * 12 / 24 / 90 tokens: 82.1 / 97.7 / 124 -> 78.3 / 97.0 / 123; Q8_0, 90 tokens: 275 -> 158. Where the images of all
+     * of K do not fit the LDS (Q4_K from 17 super-blocks at 16 pairs) the tiles below stay. */
+    if (c->mmg_mt && (long long)npair <= 6LL * nslot) {
+        const int T = (long long)npair <= 2LL * nslot ? 8 : 16, nsb = cols / 256, ntile = (rows + 15) / 16 * (dual ? 2 : 1);
+        const int maxp = nslot + (npair + T - 1) / T, live = std::min(npair, nslot);
+        char name[32];
+        snprintf(name, sizeof name, "le_mtg_%d_t%d", ty, T);
+        int kw = 1;
+        while (kw < 8 && 2 * kw <= nsb && (long long)ntile * live * kw < 8LL * 2 * c->cus) kw *= 2;
+        const size_t lds = mt_lds(ty, nsb, T, T, kw > 1);
+        if (lds <= c->lds_limit && c->fn(name) && (long long)maxp * ntile <= 0x7FFFFFFFLL) {
+            /* row tiles per wave: four blocks a CU, or one where each builds 16 pairs' images (12 / 24 tokens as above:
+             * two 84.8 / 113.8 us, four 81.6 / 103; 64 / 96 tokens: one 129 / 132, two 127 / 134, four 146 / 160) */
+            const int side = 8 / kw, tpw = std::max(1LL, std::min<long long>(8, (long long)ntile * live / ((T == 16 ? 1LL : 4LL) * side * c->cus)));
+            MtHostArgs a{};
+            a.w = w;
+            a.x = x;
+            a.y = y;
+            a.rows = rows;
+            a.cols = cols;
+            a.kw = kw;
+            a.ptrs = ptrs;
+            a.w_slot_bytes = (unsigned long long)rows * le_row_bytes(ty, cols);
+            a.off = off;
+            a.in_idx = in_idx;
+            a.out_idx = out_idx;
+            a.nslot = nslot;
+            a.maxt = maxp;
+            a.ng = (ntile + side * tpw - 1) / (side * tpw);
+            a.dual = dual ? 1 : 0;
+            a.ptrs2 = ptrs2;
+            a.w2 = w2;
+            a.y2 = y2;
+            a.up = up;
+            void *args[] = {&a};
+            return c->launch(name, dim3((unsigned)(maxp * a.ng)), 512, lds, (hipStream_t)stream, args);
+        }
+    }
     static const int cfgs[8][4] = {{1, 4, 1, 2}, {1, 4, 2, 2}, {1, 4, 4, 2}, {2, 2, 2, 2}, {1, 8, 2, 1}, {1, 8, 4, 1}, {1, 8, 1, 1}, {1, 4, 1, 1}};
     int ci = mmg_cfg(nslot, npair);
     const int srec = gq_srec(ty);

@@ -88,3 +88,29 @@ def test_gemm_few_tokens(engine, name, rows, nsb, m):
     # (9 tokens and more, and Q4_K's own kernel): 2^-11; 15-bit activations (Q4_K, 2 tokens): 3.1e-5 of a block's maximum
     tol = 1e-5 if m <= 8 and ty != le.Q4_K else 1e-3
     assert np.all(np.abs(y.cpu().numpy() - want) <= tol * mag + 1e-30), float(np.max(np.abs(y.cpu().numpy() - want) / (mag + 1e-30)))
+
+
+# grouped few-pair form: a tile's edges (8 and 9 pairs at 8 a pass, 16 and 17 at 16), empty slots at both ends,
+# one super-block and one row tile (one wave), waves sharing a tile, a K whose images do not fit the LDS
+@pytest.mark.parametrize("name", list(le.MV_TYPES))
+@pytest.mark.parametrize("rows,nsb,counts", [(16, 1, (0, 1, 0)), (37, 3, (0, 8, 0, 9, 0, 0, 0, 0, 1, 0)), (272, 7, (16, 0, 17, 1, 2)),
+                                             (2064, 4, (0, 3, 9, 0, 0, 0, 0)), (50, 17, (12, 5, 0, 0)), (40, 30, (2, 1))])
+def test_grouped_few_pairs(engine, name, rows, nsb, counts):
+    import torch
+    ty, cols, nslot = le.MV_TYPES[name], 256 * nsb, len(counts)
+    q = wbytes(ty, nslot * rows, cols, seed=rows + nsb)
+    off = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    npair = int(off[-1])
+    x = acts(npair * cols, 9 + nsb).reshape(npair, cols)
+    x[npair - 1] *= np.float32(1e-20)  # a row of another magnitude
+    rng = np.random.default_rng(nsb)
+    in_idx, out_idx = rng.permutation(npair).astype(np.int32), rng.permutation(npair).astype(np.int32)
+    y = torch.full((npair, rows), float("nan"), device="cuda")
+    print("grouped few pairs", name, rows, cols, counts, flush=True)
+    engine.mm_grouped(ty, dev(off), dev(in_idx), dev(out_idx), nslot, npair, dev(x), y, rows, cols, w=dev(q))
+    got = y.cpu().numpy()[out_idx]
+    w = oracle.dequant_rows(ty, q, nslot * rows, cols).astype(np.float64).reshape(nslot, rows, cols)
+    for s in range(nslot):
+        xs = x[in_idx[off[s]:off[s + 1]]].astype(np.float64)
+        # activations rounded to fp16 (2^-11 each), fp32 sums far below it
+        assert np.all(np.abs(got[off[s]:off[s + 1]] - xs @ w[s].T) <= 1e-3 * (np.abs(xs) @ np.abs(w[s]).T) + 1e-30)
