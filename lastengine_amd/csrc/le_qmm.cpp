@@ -712,13 +712,12 @@ int le_dequant_rows(le_ctx *c, int ty, const void *w, float *out, int rows, int 
     le_block_geometry(ty, &v, &b);
     if (rows <= 0 || cols <= 0 || cols % v || cols % 32) return c->fail(LE_ERR_SHAPE, "bad shape %dx%d", rows, cols);
     if (!al16(out) || (cols % 4)) return c->fail(LE_ERR_ALIGN, "output must be 16-byte aligned");
-    unsigned long long rb = (unsigned long long)(cols / v) * b;
     const long long units = (long long)rows * (cols / 32);
     long long blocks = (units + 255) / 256;
     if (blocks > (long long)c->cus * 16) blocks = (long long)c->cus * 16;
     char name[32];
     snprintf(name, sizeof name, "le_dequant_%d", ty);
-    void *args[] = {(void *)&w, (void *)&out, (void *)&rows, (void *)&cols, (void *)&rb};
+    void *args[] = {(void *)&w, (void *)&out, (void *)&rows, (void *)&cols};
     return c->launch(name, dim3((unsigned)blocks), 256, 0, (hipStream_t)stream, args);
 }
 

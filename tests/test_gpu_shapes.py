@@ -114,3 +114,35 @@ def test_grouped_few_pairs(engine, name, rows, nsb, counts):
         xs = x[in_idx[off[s]:off[s + 1]]].astype(np.float64)
         # activations rounded to fp16 (2^-11 each), fp32 sums far below it
         assert np.all(np.abs(got[off[s]:off[s + 1]] - xs @ w[s].T) <= 1e-3 * (np.abs(xs) @ np.abs(w[s]).T) + 1e-30)
+
+
+# dequantization: waves of 64 units: a part of one, exactly one, one unit more, several grid strides (256 CUs x 16 blocks)
+@pytest.mark.parametrize("name", list(le.MV_TYPES))
+@pytest.mark.parametrize("rows,nsb", [(1, 1), (8, 1), (3, 3), (64, 16), (16500, 8)])
+def test_dequant_units(engine, name, rows, nsb):
+    import torch
+    ty, cols = le.MV_TYPES[name], 256 * nsb
+    q = wbytes(ty, min(rows, 64), cols, seed=rows + nsb)
+    reps = -(-rows // len(q))
+    w = torch.cat([dev(np.zeros(2, np.uint8)), dev(q).reshape(-1).repeat(reps)])[2:2 + rows * le.row_bytes(ty, cols)]  # 2-byte aligned
+    out = torch.full((rows * cols + 64,), 7.0, device="cuda")
+    print("dequant", name, rows, cols, flush=True)
+    engine.dequant_rows(ty, w, out, rows, cols)
+    want = np.tile(oracle.dequant_rows(ty, q, len(q), cols).reshape(len(q), cols), (reps, 1))[:rows]
+    got = out.cpu().numpy()
+    assert np.array_equal(got[:rows * cols].view(np.uint32), want.reshape(-1).view(np.uint32))
+    assert (got[rows * cols:] == 7.0).all()
+
+
+@pytest.mark.parametrize("name", ["Q8_0", "Q4_0"])
+def test_dequant_units_single_blocks(engine, name):
+    import torch
+    ty = le.MV_TYPES[name]
+    for rows, cols in ((1, 32), (65, 32), (13, 160)):
+        q = wbytes(ty, rows, cols, seed=rows)
+        out = torch.full((rows * cols + 64,), 7.0, device="cuda")
+        print("dequant", name, rows, cols, flush=True)
+        engine.dequant_rows(ty, dev(q), out, rows, cols)
+        got, want = out.cpu().numpy(), oracle.dequant_rows(ty, q, rows, cols)
+        assert np.array_equal(got[:rows * cols].view(np.uint32), np.asarray(want, np.float32).reshape(-1).view(np.uint32))
+        assert (got[rows * cols:] == 7.0).all()
