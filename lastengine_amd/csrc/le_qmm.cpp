@@ -1175,14 +1175,23 @@ static int gq_launch(le_ctx *c, int ty, const void *w, const float *x, int m, fl
     else if (m <= 128 && ty == LE_TYPE_Q6_K) ci = 9;
     else if (m <= 128 && (k45 || ty == LE_TYPE_IQ3_XXS)) ci = 4;
     else if (m <= 256 && k45) ci = 4;
-    if (c->gq_cfg && c->gq_cfg <= 12) ci = c->gq_cfg - 1;
+    /* ... while they make enough work for the chip: below, 32 x 128, then 64 x 128 tiles on 4 waves. Their work in blocks
+     * times super-blocks decides, against six (and, for 32 tokens, four) per CU: 3072 x 3072 Q8_0 M = 37 / 64 / 128 / 300
+     * 30.4 / 31.6 / 37.7 / 40.7 -> 20.0 / 20.7 / 24.9 / 33.9 us, Q5_K 20.6 / 21.5 / 23.6 / 38.8 -> 17.1 / 17.9 / 22.4 / 30.7;
+     * 1024 x 4096 Q4_K M = 64 / 500 18.6 / 26.1 -> 15.7 / 24.7. Beyond the line the wide tiles win again: 4096 x 4096
+     * Q4_K M = 200 (2048 blocks x super-blocks) 27.9 against 31.7, 14336 x 4096 M = 37 (1792) 26.3 against 30.2; of 32 x 128
+     * and 64 x 128, 4096 x 4096 M = 64 (1024 of the former) 19.6 / 21.8, M = 128 25.8 / 25.0. */
     const int nsb = cols / 256, srec = gq_srec(ty);
+    const long long r128 = (rows + 127) / 128, work = 6LL * c->cus;
+    const bool small = !c->gq_cfg && m > 32 && r128 * ((m + 63) / 64) * nsb <= work;
+    if (small) ci = r128 * ((m + 31) / 32) * nsb <= work / 3 * 2 ? 8 : 7;
+    if (c->gq_cfg && c->gq_cfg <= 12) ci = c->gq_cfg - 1;
     /* pipelined kernel, its 32-token tiles per block (0: not used): from 33 tokens (M = 64 31.8 -> 29.3 us;
      * up to 32 the 32 x 128 tiles have more blocks); blocks of 64 tokens while they fill no more than
      * the chip, else 128 (14336 x 4096 Q4_K, 64 / 128 tokens a block: M = 128 36.4 / 38.8 us, 256 48.2 / 52.5,
      * 512 90.4 / 74.0; 4096 x 4096 M = 512 38.9 / 41.2) */
     int gp = 0;
-    if (gp_takes(ty, rows)) {
+    if (gp_takes(ty, rows) && !small) {
         if (c->gq_cfg) gp = c->gq_cfg == 21 ? 4 : c->gq_cfg == 22 ? 2 : 0;
         else if (m > 32) gp = (long long)((rows + 255) / 256) * ((m + 63) / 64) <= c->cus ? 2 : 4;
     }

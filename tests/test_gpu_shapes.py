@@ -60,7 +60,11 @@ def test_gemm_pipelined(engine, name, rows, nsb, m):
     pick = np.unique(np.r_[0:8, rows - 264:rows - 248, rows - 8:rows].clip(0, rows - 1))  # oracle rows
     y = torch.full((m, rows), float("nan"), device="cuda")
     print("pipelined GEMM", name, rows, cols, m, flush=True)
-    engine.gemm(ty, dev(q), dev(x), m, y, rows, cols)
+    try:
+        engine.set_option("gq_cfg", 21 if m > 512 else 22)  # less work than the pipelined kernel is chosen for
+        engine.gemm(ty, dev(q), dev(x), m, y, rows, cols)
+    finally:
+        engine.set_option("gq_cfg", 0)
     got = y.cpu().numpy()
     assert np.all(np.isfinite(got))
     sel = np.ascontiguousarray(q[pick])
@@ -146,3 +150,22 @@ def test_dequant_units_single_blocks(engine, name):
         got, want = out.cpu().numpy(), oracle.dequant_rows(ty, q, rows, cols)
         assert np.array_equal(got[:rows * cols].view(np.uint32), np.asarray(want, np.float32).reshape(-1).view(np.uint32))
         assert (got[rows * cols:] == 7.0).all()
+
+
+# small GEMMs: the first token count, token tiles with one row of their last, a ragged last row tile, K slices (even
+# counts) and none (odd ones), both block shapes and the first sizes past each
+@pytest.mark.parametrize("name", list(le.MV_TYPES))
+@pytest.mark.parametrize("rows,nsb,m", [(1, 1, 33), (130, 3, 65), (1000, 4, 33), (640, 8, 225), (2049, 12, 100), (2176, 16, 129), (4100, 16, 193)])
+def test_gemm_small(engine, name, rows, nsb, m):
+    import torch
+    ty, cols = le.MV_TYPES[name], 256 * nsb
+    q = wbytes(ty, rows, cols, seed=rows + m)
+    x = acts(m * cols, 7 + m).reshape(m, cols)
+    pick = np.unique(np.r_[0:8, rows // 2:rows // 2 + 8, rows - 8:rows].clip(0, rows - 1))  # oracle rows
+    y = torch.full((m, rows), float("nan"), device="cuda")
+    print("small GEMM", name, rows, cols, m, flush=True)
+    engine.gemm(ty, dev(q), dev(x), m, y, rows, cols)
+    got = y.cpu().numpy()
+    assert np.all(np.isfinite(got))
+    sel = np.ascontiguousarray(q.reshape(rows, -1)[pick])
+    check_close(got[:, pick], oracle.matmat(ty, sel, len(pick), cols, x), absmag(ty, sel, len(pick), cols, x))
