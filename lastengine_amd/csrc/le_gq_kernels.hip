@@ -27,16 +27,17 @@
  *   Q4_K   code sc_j * q (<= 945, exact), offset term D2 = sum_j m_j S_j (one more MFMA per
  *          super-block), acc = acc (d' / d) + D1 - (dmin / d) D2, in units of d    (src/quant.rs:72-82)
  *   Q6_K   code (q6 - 32) * sc_u / 64 (exact where (q6 - 32) sc_u has at most 11 significant
- *          bits, else rounded once to fp16), epilogue acc += 64 d * D1           (:96-112)
- *   IQ2_XXS code (2s+1) * grid * sign (<= 1333, exact), epilogue acc += d/8 * D1   (:142-154)
- *   IQ3_XXS code (2s+1) * grid * sign (<= 1922, exact), epilogue acc += d/4 * D1   (:127-141)
+ *          bits, else rounded once to fp16), scale 64 d                          (:96-112)
+ *   IQ2_XXS code (2s+1) * grid * sign (<= 1333, exact), scale d/8                  (:142-154)
+ *   IQ3_XXS code (2s+1) * grid * sign (<= 1922, exact), scale d/4                  (:127-141)
  *   Q5_K   as Q4_K with the fifth bit from qh, code sc_j * q (<= 1953, exact)     (:83-95)
- *   Q3_K   code (q3 - 4) * (sc6 - 32) (|.| <= 128, exact), epilogue acc += d * D1 (:113-126)
- *   IQ2_S  code (2s+1) * grid * sign, 1024-entry grid, explicit sign bytes, epilogue acc += d/8 * D1
+ *   Q3_K   code (q3 - 4) * (sc6 - 32) (|.| <= 128, exact), scale d                (:113-126)
+ *   IQ2_S  code (2s+1) * grid * sign, 1024-entry grid, explicit sign bytes, scale d/8
  *                                                                                  (:155-167)
  *   Q8_0, Q4_0  per-32 scale d_b inside the code: fp16(q * d_b 2^S) (one rounding, 2^-11
  *          relative), S a per-row power of two that only decreases (the accumulator is rescaled
  *          when it does) and keeps every code inside the fp16 range, final * 2^-S  (:64-71)
+ * A scale: acc = acc (previous scale / scale) + D1, the accumulator in units of the row's last scale.
  * Integer byte -> fp16 conversion: a byte u placed under the fp16 exponent of 1024 (v_perm_b32)
  * is the half 1024 + u exactly; one packed fma (u+1024)*c - 1024*c gives u*c rounded once.
  *
