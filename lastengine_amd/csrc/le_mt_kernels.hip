@@ -33,6 +33,7 @@
  * 47.9 -> 18.3, 27.1 -> 19.9. Bound by the decoding (Q6_K: about 240 VALU instructions a super-block, Q4_K 156) and,
  * for small matrices, by each block's image build (2 -> 8 tokens of Q4_0 4096 x 4096: 7.6 -> 10.5 us). */
 #include "le_f16_frag.h"
+#include "le_mt_layout.h"
 
 typedef float le_v4f __attribute__((ext_vector_type(4)));
 
@@ -102,14 +103,13 @@ struct MtF<LE_TYPE_Q4_0> {
     static constexpr int CPS = 9, SBB = 144;
     __device__ static int goff(int c) { return 16 * c; }
 };
-template <int TY>
-constexpr int mt_tab() { return TY == LE_TYPE_IQ2_XXS ? 6144 : TY == LE_TYPE_IQ3_XXS ? 4096 : TY == LE_TYPE_IQ2_S ? 20480 : 0; }
 
-/* 8 bytes at a 2-byte-aligned LDS address */
-__device__ __forceinline__ uint2 mt_lds8_a2(const u8 *p) {
-    const u32 *w = (const u32 *)(p - ((size_t)p & 3)); /* pointer arithmetic keeps the LDS address space */
-    const u32 sh = (u32)((size_t)p & 3) * 8u, w0 = w[0], w1 = w[1], w2 = w[2];
-    return make_uint2(__builtin_amdgcn_alignbit(w1, w0, sh), __builtin_amdgcn_alignbit(w2, w1, sh));
+/* 8 bytes at byte b of a staged super-block (LDS, 16-byte aligned) that lie in `words` words: 2, or 3 from the
+ * middle of the first. No word past them is read: the last group of the last staged row ends the block's LDS. */
+__device__ __forceinline__ uint2 mt_lds8(const u8 *sb, int b, int words) {
+    const u32 *w = (const u32 *)(sb + (words == 3 ? b - 2 : b));
+    const u32 w0 = w[0], w1 = w[1];
+    return words == 3 ? make_uint2(__builtin_amdgcn_alignbit(w1, w0, 16), __builtin_amdgcn_alignbit(w[2], w1, 16)) : make_uint2(w0, w1);
 }
 __device__ __forceinline__ le_v8h mt_codes(u32 x, u32 y, u32 bias) { /* bytes minus (bias - 1024) as halves */
     return as_v8h(make_uint4(pk_add(h1024_02(x), bias), pk_add(h1024_13(x), bias), pk_add(h1024_02(y), bias), pk_add(h1024_13(y), bias)));
@@ -287,9 +287,9 @@ __device__ __forceinline__ void mt_sb(const u8 *sb, const uint4 *a, int lane, fl
             u32 dw[4];
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                const u8 *b = sb + (Q8 ? 34 : 18) * (4 * h + i);
-                dw[i] = *(const u32 *)(b - ((size_t)b & 3)) >> (((size_t)b & 2) * 8);
-                qv[i] = mt_lds8_a2(b + 2 + (Q8 ? 8 * g : 8 * (g & 1)));
+                const int j = 4 * h + i, db = le_mt_byte(TY, j, 0) - 2; /* the scale: the low half of a word in even sub-blocks */
+                dw[i] = j & 1 ? *(const u32 *)(sb + db - 2) >> 16 : *(const u32 *)(sb + db);
+                qv[i] = mt_lds8(sb, le_mt_byte(TY, j, Q8 ? g : g & 1), le_mt_words(j));
             }
             __builtin_amdgcn_sched_barrier(0);
             le_v4f Dj[4];
@@ -340,6 +340,7 @@ __device__ __forceinline__ void mt_body(const MtArgs &a) {
     constexpr bool OFS = TY == LE_TYPE_Q4_K || TY == LE_TYPE_Q5_K, AL = OFS; /* AL: 16-byte aligned weights */
     constexpr int R = HL ? 2 * T : T, RS = R + 1;              /* live MFMA rows; slots per fragment (odd: rows of the build's stores in distinct banks) */
     constexpr int IMG = (32 + (OFS ? 2 : 0)) * RS;             /* 16-byte slots of a super-block's image */
+    static_assert(F::CPS == le_mt_cps(TY), "staged super-block as the host sizes it");
     constexpr int NW = 8, CPR = F::CPS | 1, NCH = 16 * F::CPS, NI = (NCH + 63) / 64;
     extern __shared__ uint4 smem[];
     const int nsb = a.cols >> 8, ns = (int)gridDim.y;
@@ -358,8 +359,8 @@ __device__ __forceinline__ void mt_body(const MtArgs &a) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = lane & 15;
     uint4 *wb = stg + wave * 16 * CPR;
     u8 *tab = (u8 *)(stg + NW * 16 * CPR);
-    float4 *red = (float4 *)(tab + mt_tab<TY>());              /* [2][NW][4 T lanes], with kw > 1 */
-    if constexpr (mt_tab<TY>() > 0) gq_tables<TY>(tab);
+    float4 *red = (float4 *)(tab + le_mt_tab(TY));              /* [2][NW][4 T lanes], with kw > 1 */
+    if constexpr (le_mt_tab(TY) > 0) gq_tables<TY>(tab);
 
     const int KW = a.kw, RT = NW / KW, kw = wave % KW, rt = wave / KW;
     const int ntr = (a.rows + 15) >> 4, ntile = GR && a.dual ? 2 * ntr : ntr, mine = (nsl + KW - 1 - kw) / KW; /* super-blocks kw, kw + KW, ... of the slice */

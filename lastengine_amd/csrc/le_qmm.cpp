@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "../../include/le_qmm.h"
+#include "le_mt_layout.h"
 #include "le_formats.h"
 
 namespace {
@@ -1104,18 +1105,11 @@ struct MtHostArgs { /* MtArgs in le_mt_kernels.hip */
     float *y2;
     const float *up;
 };
-/* LDS of a le_mt block: images of `most` super-blocks with R MFMA rows, scales, staging, the waves' sums (kw > 1) */
-static size_t mt_lds(int ty, int most, int R, int T, bool sums) {
-    const bool ofs = ty == LE_TYPE_Q4_K || ty == LE_TYPE_Q5_K;
-    const int cps = ty == LE_TYPE_Q6_K ? 14 : ty == LE_TYPE_IQ2_XXS ? 5 : ty == LE_TYPE_IQ3_XXS ? 7 : ty == LE_TYPE_Q8_0 ? 17 : ty == LE_TYPE_Q5_K ? 11 : ty == LE_TYPE_Q3_K ? 7 : ty == LE_TYPE_IQ2_S ? 6 : 9;
-    return (size_t)most * ((size_t)(32 + (ofs ? 2 : 0)) * (R + 1) * 16 + 64) + (size_t)8 * 16 * (cps | 1) * 16 + (sums ? (size_t)2 * 8 * 4 * T * 16 : 0) +
-           gq_tab(ty);
-}
 static int mt_launch(le_ctx *c, int ty, const void *w, const float *x, int m, float *y, int rows, int cols, void *ws,
                      size_t ws_bytes, hipStream_t st) {
     const int T = m <= 4 ? 4 : m <= 8 ? 8 : 16, R = T == 4 ? 8 : 16, NW = 8;
     const int nsb = cols / 256, ntile = (rows + 15) / 16;
-    auto lds_of = [&](int ks) { return mt_lds(ty, (nsb + ks - 1) / ks, R, T, true); };
+    auto lds_of = [&](int ks) { return le_mt_lds(ty, (nsb + ks - 1) / ks, R, T, true); };
     int ks = 1;
     while (ks < nsb && lds_of(ks) > c->lds_limit) ks++;
     const size_t lds = lds_of(ks);
@@ -1289,7 +1283,7 @@ static int mm_grouped(le_ctx *c, int ty, const void *const *ptrs, const void *w,
         snprintf(name, sizeof name, "le_mtg_%d_t%d", ty, T);
         int kw = 1;
         while (kw < 8 && 2 * kw <= nsb && (long long)ntile * live * kw < 8LL * 2 * c->cus) kw *= 2;
-        const size_t lds = mt_lds(ty, nsb, T, T, kw > 1);
+        const size_t lds = le_mt_lds(ty, nsb, T, T, kw > 1);
         if (lds <= c->lds_limit && c->fn(name) && (long long)maxp * ntile <= 0x7FFFFFFFLL) {
             /* row tiles per wave: four blocks a CU, or one where each builds 16 pairs' images (12 / 24 tokens as above:
              * two 84.8 / 113.8 us, four 81.6 / 103; 64 / 96 tokens: one 129 / 132, two 127 / 134, four 146 / 160) */
