@@ -1044,9 +1044,8 @@ static size_t gq_ws_bytes(int ty, int m, int cols) {
     return mp * cols * 2 + mp / 32 * (cols / 256) * gq_srec(ty) + mp * 4;
 }
 /* K-slice partial results follow at the next 256-byte boundary: [ks][m][rows] floats, ks <= 8. A
- * launch splits K only while (row tiles) x (token tiles) x 2 fits the resident blocks, at most 512
- * on gfx950, and its tiles hold at least 256 rows x 128 tokens when that count is smallest, so a
- * shape with more than 256 such tiles never splits. */
+ * launch splits K only while (row tiles) x (token tiles) x 2 is at most one block per CU (256 on gfx950); its
+ * tiles hold at most 256 rows x 128 tokens, so a shape with more than 256 such tiles never splits. */
 static size_t gq_part_off(int ty, int m, int cols) { return (gq_ws_bytes(ty, m, cols) + 255) / 256 * 256; }
 static bool gq_may_split(int m, int rows) { return (long long)((rows + 255) / 256) * ((m + 127) / 128) <= 256; }
 /* Kernel arguments of le_gq_* (GqArgs in le_gq_kernels.hip). */
@@ -1210,12 +1209,11 @@ static int gq_launch(le_ctx *c, int ty, const void *w, const float *x, int m, fl
     if (c->gq_ksplit > 0) {
         ks = c->gq_ksplit;
     } else {
-        /* K slices while the grid stays within the resident blocks (one wave of blocks); the
-         * 4-wave tiles stop at one block per CU (measured best: Q4_K 14336x4096 M=17, 32x128
-         * tiles: 26.2 us at 224 blocks, 29.7 at 448) */
-        const int per_cu = nthr == 256 ? 1 : c->blocks_per_cu(name, nthr, lds);
-        const long long cap = (long long)c->cus * (per_cu > 0 ? per_cu : 1);
-        while (ks < 8 && ntr * mt * 2 * ks <= cap && nsb % (2 * ks) == 0) ks *= 2;
+        /* K slices while the grid stays within one block per CU, whatever the kernel's registers leave
+         * room for: a further doubling writes and reads twice the partial results (Q4_K 14336 x 4096 M = 17,
+         * 32 x 128 tiles: 26.2 us at 224 blocks, 29.7 at 448; IQ2_XXS 14336 x 4096 M = 64, 64 x 256 tiles on 8 waves:
+         * 33.0 us in 4 slices, 36.1 in 8) */
+        while (ks < 8 && ntr * mt * 2 * ks <= c->cus && nsb % (2 * ks) == 0) ks *= 2;
     }
     if (nsb % ks) return c->fail(LE_ERR_SHAPE, "gq_ksplit=%d does not divide the %d super-blocks", ks, nsb);
     const int mp = (m + 127) / 128 * 128;

@@ -200,3 +200,20 @@ def test_gemm_per_block_scale_range(engine, name, m):
     want = oracle.matmat(ty, q, rows, cols, xs)
     assert np.all(got[:, 5] == 0.0)
     check_close(got, want, absmag(ty, q, rows, cols, xs))
+
+
+@pytest.mark.parametrize("name,rows,cols,m,ks", [("IQ2_XXS", 14336, 4096, 64, 4), ("IQ3_XXS", 14336, 4096, 100, 2)])
+def test_gemm_slices_follow_tiles(fresh_engine, name, rows, cols, m, ks):
+    """K slices fill the chip with one block per CU, however many blocks a kernel's registers allow there: the same
+    bits as with that slice count set (another count sums in another order)."""
+    import torch
+    ty = le.MV_TYPES[name]
+    dq, dx = dev(random_blocks(ty, rows, cols, seed=m)), dev(acts(m * cols, m).reshape(m, cols))
+    outs = []
+    for k in (0, ks):
+        fresh_engine.set_option("gq_ksplit", k)
+        print("slices follow tiles", name, rows, cols, m, k, flush=True)
+        y = torch.empty(m, rows, dtype=torch.float32, device="cuda")
+        fresh_engine.gemm(ty, dq, dx, m, y, rows, cols)
+        outs.append(y)
+    assert torch.equal(outs[0].view(torch.int32), outs[1].view(torch.int32))
