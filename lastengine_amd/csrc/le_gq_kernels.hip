@@ -419,8 +419,10 @@ __device__ __forceinline__ void gq_vm_wait() {
 __device__ __forceinline__ u32 gq_lds_addr(const void *p) { return (u32)(size_t)(const __attribute__((address_space(3))) void *)p; }
 
 /* End of a block's tile: acc times the token scales into y, the K slice's partial results or (neither)
- * atomically added into y. LDSB: bytes of LDS that may be overwritten; rows below rmin are left out. */
-template <int WM, int WN, int TM, int TN, bool GR, int LDSB>
+ * atomically added into y. LDSB: bytes of LDS that may be overwritten. CUT: rows below rmin are left out (compared
+ * for every block, the check cost the short slices of the other kernels 1-2 us: 4096 x 4096 M = 256 Q3_K 34.5 against
+ * 33.0, Q8_0 39.0 / 37.9). */
+template <int WM, int WN, int TM, int TN, bool GR, int LDSB, bool CUT = false>
 __device__ __forceinline__ void gq_store(const GqArgs &a, u8 *lds, const float *tsc, const le_v16f (&acc)[TM][TN], int M, int mb,
                                          int nb, int pair0, bool second, int rmin = 0) {
     constexpr int BN = 32 * TN * WN, NT = 64 * WM * WN;
@@ -443,7 +445,7 @@ __device__ __forceinline__ void gq_store(const GqArgs &a, u8 *lds, const float *
 #pragma unroll
                 for (int e = 0; e < 16; e++) {
                     const int t = t0 + 8 * (e >> 2) + (e & 3);
-                    if (t < M && r >= rmin && r < a.rows) unsafeAtomicAdd(a.y + (size_t)t * a.rows + r, acc[i][k][e] * ts[i][e]);
+                    if (t < M && (!CUT || r >= rmin) && r < a.rows) unsafeAtomicAdd(a.y + (size_t)t * a.rows + r, acc[i][k][e] * ts[i][e]);
                 }
             }
         }
@@ -477,12 +479,12 @@ __device__ __forceinline__ void gq_store(const GqArgs &a, u8 *lds, const float *
             if constexpr (GR) o = a.out_idx[pair0 + t - mb];
             const float4 v = *(const float4 *)(T + tl * TS + 4 * q);
             float *yp = dst + (size_t)o * a.rows + r;
-            if (vec && r >= rmin && r + 3 < a.rows) {
+            if (vec && (!CUT || r >= rmin) && r + 3 < a.rows) {
                 *(float4 *)yp = v;
             } else {
                 const float vv[4] = {v.x, v.y, v.z, v.w};
                 for (int u = 0; u < 4 && r + u < a.rows; u++)
-                    if (r + u >= rmin) yp[u] = vv[u];
+                    if (!CUT || r + u >= rmin) yp[u] = vv[u];
             }
         }
     }
@@ -1427,7 +1429,7 @@ __device__ __forceinline__ void gp_body(const GqArgs &a, const u8 *ws) {
 #pragma unroll
             for (int e = 0; e < 16; e++) acc[i][k][e] *= unit[k];
     }
-    gq_store<1, WN, TM, TN, GR, 3 * WB + 2 * AB>(a, lds, tsc, acc, M, mb, nbw, pair0, second, nb);
+    gq_store<1, WN, TM, TN, GR, 3 * WB + 2 * AB, true>(a, lds, tsc, acc, M, mb, nbw, pair0, second, nb);
 }
 
 #define LE_GQX(TY, SK) \
