@@ -91,11 +91,11 @@ __device__ __forceinline__ void gq_barrier() {
 }
 
 template <int TM, int TN>
-__device__ __forceinline__ void gq_mma(le_v16f (&d)[TM][TN], const le_v8h (&A)[TM], const le_v8h (&B)[TN]) {
+__device__ __forceinline__ void gq_mma(le_v16f (&d)[TM][TN], const le_v8h (&A)[TM], const le_v8h (&B)[TN], bool zero) {
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
-        for (int k = 0; k < TN; k++) d[i][k] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[i], B[k], d[i][k], 0, 0, 0);
+        for (int k = 0; k < TN; k++) d[i][k] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[i], B[k], zero ? (le_v16f){} : d[i][k], 0, 0, 0);
 }
 
 /* ============================ per-type formats ============================
@@ -637,7 +637,12 @@ __device__ __forceinline__ void gq_body(const GqArgs &a, const u8 *ws) {
         }
     };
 
-    le_v16f acc[TM][TN];
+    /* SEP: a super-block's products in an accumulator of their own, which joins acc at its end. A wave of one 32 x 32
+     * tile has the registers for it; a shared one lay in accumulation registers there, so that each rescaling moved it
+     * out and back, before the wave's one chain of MFMAs went on (24 tokens, 2560 x 6912, against this form: Q3_K 53.5 /
+     * 48.9 us, Q5_K 56.5 / 51.5, IQ3_XXS 65.3 / 61.0; 14336 x 4096 Q3_K 26.6 / 25.5). */
+    constexpr bool SEP = F::EPI == 1 && TM * TN == 1;
+    le_v16f acc[TM][TN], d1[SEP ? TM : 1][SEP ? TN : 1];
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
@@ -652,7 +657,7 @@ __device__ __forceinline__ void gq_body(const GqArgs &a, const u8 *ws) {
     float unit[TN];
     u32 live[TN];
 #pragma unroll
-    for (int k = 0; k < TN; k++) unit[k] = 1.f, live[k] = 0;
+    for (int k = 0; k < TN; k++) unit[k] = 1.f, live[k] = SEP ? ~0u : 0;
     Set RA, RB; /* RA holds odd (h = 1) steps, RB even ones */
     const int s0 = 2 * sb0;
     /* the loads must reach the memory pipeline in step order (RA's before RB's, as in the loop),
@@ -690,19 +695,25 @@ __device__ __forceinline__ void gq_body(const GqArgs &a, const u8 *ws) {
              * next chunk are read while this chunk's MFMAs run (read right before their use, each MFMA
              * waited out an LDS read). */
             le_v8h Af[2][TM];
-            auto aload = [&](int p) {
+            auto aread = [&](int p, le_v8h (&A)[TM]) {
                 constexpr bool PAIR = TY == LE_TYPE_Q4_K || TY == LE_TYPE_Q5_K;
                 const int c = TY == LE_TYPE_Q6_K ? 2 * (p & 3) + (p >> 2) : PAIR ? (p & 4) | ((p & 1) << 1) | ((p >> 1) & 1) : p;
 #pragma unroll
-                for (int i = 0; i < TM; i++) Af[p & 1][i] = as_v8h(*(const uint4 *)(Ab + i * 8192 + c * 1024 + lane * 16));
+                for (int i = 0; i < TM; i++) A[i] = as_v8h(*(const uint4 *)(Ab + i * 8192 + c * 1024 + lane * 16));
             };
             auto mma = [&](int p, const le_v8h (&B)[TN]) { /* position p of that order */
-                if (p < 7) aload(p + 1);
-                __builtin_amdgcn_sched_barrier(0x016); /* LDS reads stay on their side of the MFMAs; VALU, SALU and VMEM may cross */
-                gq_mma(acc, Af[p & 1], B);
-                __builtin_amdgcn_sched_barrier(0x016);
+                if constexpr (SEP) { /* one MFMA a fragment: nothing to read behind */
+                    le_v8h A[TM];
+                    aread(p, A);
+                    gq_mma(d1, A, B, h == 0 && p == 0);
+                } else {
+                    if (p < 7) aread(p + 1, Af[(p + 1) & 1]);
+                    __builtin_amdgcn_sched_barrier(0x016); /* LDS reads stay on their side of the MFMAs; VALU, SALU and VMEM may cross */
+                    gq_mma(acc, Af[p & 1], B, false);
+                    __builtin_amdgcn_sched_barrier(0x016);
+                }
             };
-            aload(0);
+            if constexpr (!SEP) aread(0, Af[0]);
             /* stage the next step and issue the loads two steps ahead once this step's first
              * fragments are under way */
             auto pipe = [&]() {
@@ -717,7 +728,7 @@ __device__ __forceinline__ void gq_body(const GqArgs &a, const u8 *ws) {
                 if constexpr (NA == 3) dma(s + 2); /* slot (s + 2) % 3 was last read in step s - 1 */
                 __builtin_amdgcn_sched_barrier(0);
             };
-            if (F::EPI == 1 && h == 0) {
+            if (F::EPI == 1 && !SEP && h == 0) {
                 /* a new super-block scale: one multiplication puts the running sum into its units, so the
                  * MFMAs accumulate into it directly and a wave needs one accumulator, not a second one
                  * per super-block */
@@ -1045,7 +1056,7 @@ __device__ __forceinline__ void gq_body(const GqArgs &a, const u8 *ws) {
                 const u32 m0 = hd.z & 0x3F3F3F3Fu, m1 = ((hd.w >> 4) & 0x0F0F0F0Fu) | ((hd.z >> 2) & 0x30303030u);
                 const le_v8h b2 = as_v8h(make_uint4(pk_add(h1024_02(m0), 0xE400E400u), pk_add(h1024_13(m0), 0xE400E400u),
                                                     pk_add(h1024_02(m1), 0xE400E400u), pk_add(h1024_13(m1), 0xE400E400u)));
-                const float dm = -h2f(hd.x >> 16) * __builtin_amdgcn_rcpf(unit[k]);
+                const float dm = SEP ? -h2f(hd.x >> 16) : -h2f(hd.x >> 16) * __builtin_amdgcn_rcpf(unit[k]);
 #pragma unroll
                 for (int i = 0; i < TM; i++) {
                     const le_v8h a2 = as_v8h(*(const uint4 *)(Sb + i * 1024 + lane * 16));
@@ -1055,9 +1066,14 @@ __device__ __forceinline__ void gq_body(const GqArgs &a, const u8 *ws) {
                 }
             }
         }
+        if constexpr (SEP) {
+            const float d = F::scale(lds + BUF + (wn * 32 + n) * F::SLOT);
+#pragma unroll
+            for (int e = 0; e < 16; e++) acc[0][0][e] = __builtin_fmaf(d, d1[0][0][e], acc[0][0][e]);
+        }
     }
     if constexpr (AD) gq_vm_wait<0>(); /* no activation load may still be writing LDS */
-    {
+    if constexpr (!SEP) {
 #pragma unroll
         for (int k = 0; k < TN; k++) {
             const float f = F::EPI == 2 ? ldexpf(1.f, -rowS[k]) : unit[k];

@@ -64,6 +64,27 @@ def test_code_objects_use_no_flat_memory_ops(tmp_path):
     assert not found, found
 
 
+def test_small_tiles_keep_their_accumulator_in_vector_registers(tmp_path):
+    """The GEMM's 32 x 128 tiles (17..32 tokens) move their accumulator out of the accumulation registers at most once
+    (16 values, at the end), not at every super-block (checked on the disassembly of the built code objects)."""
+    import subprocess
+    bundler = os.path.join(ROCM, "llvm", "bin", "clang-offload-bundler")
+    objdump = os.path.join(ROCM, "llvm", "bin", "llvm-objdump")
+    if not (os.path.exists(bundler) and os.path.exists(objdump)):
+        pytest.skip("ROCm LLVM tools not installed")
+    moves = {}
+    for part, types in (("gq", (12, 14, 16, 18)), ("gq2", (11, 13, 22))):  # Q8_0 and Q4_0 rescale by their block scales
+        elf = str(tmp_path / (part + ".elf"))
+        subprocess.run([bundler, "--type=o", "--targets=hipv4-amdgcn-amd-amdhsa--gfx950",
+                        "--input=" + os.path.join(qmm.LIB_DIR, "le_qmm_%s.hsaco" % part), "--output=" + elf, "--unbundle"], check=True)
+        for ty in types:
+            name = "le_gq_%d_w14_t11" % ty
+            asm = subprocess.run([objdump, "-d", "--disassemble-symbols=" + name, elf], check=True, capture_output=True, text=True).stdout
+            assert "v_mfma" in asm
+            moves[name] = len(re.findall(r"\bv_accvgpr_(read|write|mov)", asm))
+    assert max(moves.values()) <= 32, moves
+
+
 @pytest.mark.parametrize("ty,cols,want", [(8, 4096, 4352), (12, 4096, 2304), (14, 14336, 11760),
                                           (16, 4096, 1056), (18, 14336, 5488), (12, 2048, 1152),
                                           (14, 768, 630)])
