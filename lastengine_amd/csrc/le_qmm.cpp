@@ -1175,9 +1175,31 @@ static int gq_launch(le_ctx *c, int ty, const void *w, const float *x, int m, fl
      * Q4_K M = 200 (2048 blocks x super-blocks) 27.9 against 31.7, 14336 x 4096 M = 37 (1792) 26.3 against 30.2; of 32 x 128
      * and 64 x 128, 4096 x 4096 M = 64 (1024 of the former) 19.6 / 21.8, M = 128 25.8 / 25.0. */
     const int nsb = cols / 256, srec = gq_srec(ty);
+    /* K slices while the grid stays within one block per CU, whatever the kernel's registers leave room for: a further
+     * doubling writes and reads twice the partial results (Q4_K 14336 x 4096 M = 17, 32 x 128 tiles: 26.2 us at 224
+     * blocks, 29.7 at 448; IQ2_XXS 14336 x 4096 M = 64, 64 x 256 tiles on 8 waves: 33.0 us in 4 slices, 36.1 in 8) */
+    auto slices = [&](long long tiles) {
+        int k = 1;
+        while (k < 8 && tiles * 2 * k <= c->cus && nsb % (2 * k) == 0) k *= 2;
+        return k;
+    };
     const long long r128 = (rows + 127) / 128, work = 6LL * c->cus;
-    const bool small = !c->gq_cfg && m > 32 && r128 * ((m + 63) / 64) * nsb <= work;
-    if (small) ci = r128 * ((m + 31) / 32) * nsb <= work / 3 * 2 ? 8 : 7;
+    bool small = !c->gq_cfg && m > 32 && r128 * ((m + 63) / 64) * nsb <= work;
+    if (small) {
+        ci = r128 * ((m + 31) / 32) * nsb <= work / 3 * 2 ? 8 : 7;
+        /* ... but not where a 64 x 128 tile keeps a long chain of super-blocks (8; 6 for Q4_K and Q5_K, whose wide tile is
+         * the pipelined kernel) that a 64 x 256 tile cuts in half by K slices, its blocks (row tiles padded to the 8 XCDs)
+         * still one per CU: 2048 x 4096 M = 320 IQ3_XXS 36.0 against 30.7 us, IQ2_S 36.9 / 31.4, Q6_K 32.5 / 29.6; 4096 x 4096
+         * M = 192 Q5_K 34.4 / 28.5, IQ3_XXS 35.5 / 32.6, Q4_K 31.1 / 28.0; 3072 x 3072 M = 160 Q5_K 28.1 / 25.5, but M = 320
+         * (320 padded blocks) 31.0 / 38.0. Q8_0, 36.4 / 36.9, stays. */
+        const long long t256 = (long long)((rows + 255) / 256) * ((m + 63) / 64);
+        const int k64 = slices(r128 * ((m + 63) / 64)), k256 = slices(t256);
+        if (ci == 7 && ty != LE_TYPE_Q8_0 && nsb / k64 >= (k45 ? 6 : 8) && k256 >= 2 * k64 &&
+            (rows + 2047) / 2048 * 8LL * ((m + 63) / 64) * k256 <= c->cus) {
+            small = false;
+            ci = 4;
+        }
+    }
     if (c->gq_cfg && c->gq_cfg <= 12) ci = c->gq_cfg - 1;
     /* pipelined kernel, its 32-token tiles per block (0: not used): from 33 tokens (M = 64 31.8 -> 29.3 us;
      * up to 32 the 32 x 128 tiles have more blocks); blocks of 64 tokens while they fill no more than
@@ -1209,11 +1231,7 @@ static int gq_launch(le_ctx *c, int ty, const void *w, const float *x, int m, fl
     if (c->gq_ksplit > 0) {
         ks = c->gq_ksplit;
     } else {
-        /* K slices while the grid stays within one block per CU, whatever the kernel's registers leave
-         * room for: a further doubling writes and reads twice the partial results (Q4_K 14336 x 4096 M = 17,
-         * 32 x 128 tiles: 26.2 us at 224 blocks, 29.7 at 448; IQ2_XXS 14336 x 4096 M = 64, 64 x 256 tiles on 8 waves:
-         * 33.0 us in 4 slices, 36.1 in 8) */
-        while (ks < 8 && ntr * mt * 2 * ks <= c->cus && nsb % (2 * ks) == 0) ks *= 2;
+        ks = slices(ntr * mt);
     }
     if (nsb % ks) return c->fail(LE_ERR_SHAPE, "gq_ksplit=%d does not divide the %d super-blocks", ks, nsb);
     const int mp = (m + 127) / 128 * 128;

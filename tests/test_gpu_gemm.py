@@ -217,3 +217,21 @@ def test_gemm_slices_follow_tiles(fresh_engine, name, rows, cols, m, ks):
         fresh_engine.gemm(ty, dq, dx, m, y, rows, cols)
         outs.append(y)
     assert torch.equal(outs[0].view(torch.int32), outs[1].view(torch.int32))
+
+
+@pytest.mark.parametrize("name,rows,cols,m,cfg", [("Q5_K", 4096, 4096, 192, 22), ("Q4_K", 2048, 8192, 160, 22), ("IQ3_XXS", 2048, 4096, 320, 5),
+                                                  ("Q6_K", 6144, 4096, 100, 5), ("Q5_K", 3072, 3072, 320, 8), ("IQ2_S", 3072, 3072, 256, 8)])
+def test_gemm_tile_by_chain(fresh_engine, name, rows, cols, m, cfg):
+    """Where 64 x 128 tiles would keep a long chain of super-blocks that 64 x 256 tiles cut by K slices, the wide tile
+    runs (first four), else the small one: the same bits as with that block shape set."""
+    import torch
+    ty = le.MV_TYPES[name]
+    dq, dx = dev(random_blocks(ty, rows, cols, seed=m)), dev(acts(m * cols, m).reshape(m, cols))
+    outs = []
+    for k in (0, cfg):
+        fresh_engine.set_option("gq_cfg", k)
+        print("tile by chain", name, rows, cols, m, k, flush=True)
+        y = torch.empty(m, rows, dtype=torch.float32, device="cuda")
+        fresh_engine.gemm(ty, dq, dx, m, y, rows, cols)
+        outs.append(y)
+    assert torch.equal(outs[0].view(torch.int32), outs[1].view(torch.int32))
