@@ -85,6 +85,25 @@ def test_small_tiles_keep_their_accumulator_in_vector_registers(tmp_path):
     assert max(moves.values()) <= 32, moves
 
 
+def test_iq3_int8_matvec_reads_its_tables_ahead(tmp_path):
+    """The IQ3_XXS matvec of the int8 mode runs the same loop as the fp32 one: between its first and last MFMA it drains
+    the LDS counter no more often (checked on the disassembly of the built code object)."""
+    import subprocess
+    bundler = os.path.join(ROCM, "llvm", "bin", "clang-offload-bundler")
+    objdump = os.path.join(ROCM, "llvm", "bin", "llvm-objdump")
+    if not (os.path.exists(bundler) and os.path.exists(objdump)):
+        pytest.skip("ROCm LLVM tools not installed")
+    elf = str(tmp_path / "mv18.elf")
+    subprocess.run([bundler, "--type=o", "--targets=hipv4-amdgcn-amd-amdhsa--gfx950",
+                    "--input=" + os.path.join(qmm.LIB_DIR, "le_qmm_mv18.hsaco"), "--output=" + elf, "--unbundle"], check=True)
+
+    def drains(name):
+        asm = subprocess.run([objdump, "-d", "--disassemble-symbols=" + name, elf], check=True, capture_output=True, text=True).stdout
+        return len(re.findall(r"s_waitcnt lgkmcnt\(0\)", asm[asm.index("v_mfma"):asm.rindex("v_mfma")]))
+
+    assert drains("le_ms_18_p2_w4_q8") <= drains("le_ms_18_p2_w4") + 2
+
+
 @pytest.mark.parametrize("ty,cols,want", [(8, 4096, 4352), (12, 4096, 2304), (14, 14336, 11760),
                                           (16, 4096, 1056), (18, 14336, 5488), (12, 2048, 1152),
                                           (14, 768, 630)])
