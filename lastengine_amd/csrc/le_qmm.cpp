@@ -295,29 +295,34 @@ int mq_launch(le_ctx *c, int ty, const void *const *ptrs, const void *w, const f
      *    14336 8.8 against 10.4 on 8, Q6_K 13.2 / 14.1, IQ3_XXS 11.3 / 11.9, Q8_0 16.3 / 16.6; at 28
      *    super-blocks 8 waves win, Q4_K 5.2 / 5.9), items of two for the K-quants that gain by it
      *    (Q4_K 8.8 / 9.4, Q6_K 13.2 / 13.9) and one otherwise; fewer super-blocks: 8 waves, items
-     *    of one (Q6_K 2304 x 7168 6.9 / 8.1), but two for Q4_K where that shortens the chain (1536 x
-     *    5632 4.4 / 5.0);
+     *    of one (Q6_K 2304 x 7168 6.9 / 8.1), but two for Q4_K and IQ2_XXS where that shortens the chain (1536 x
+     *    5632 Q4_K 4.4 / 5.0, 2048 x 8192 IQ2_XXS 7.3 / 7.6);
      *  - more row tiles: 4 waves, items of two from 16 super-blocks (14336 x 4096 Q4_K 8.8 / 9.8, Q5_K
      *    11.0 / 11.7, Q6_K 13.9 / 14.9, IQ3_XXS 11.6 / 12.1; not Q8_0, 32000 x 4096 25.8 / 25.4), of
-     *    one below (12288 x 3072: within 2%). */
+     *    one below (12288 x 3072: within 2%), and of one where only their smaller staging leaves the LDS room for
+     *    two blocks a CU (8192 x 28672 Q5_K 40.3 / 48.0, Q4_K 35.2 / 39.3, IQ3_XXS 38.7 / 52.2; 8192 x 22528 Q6_K 38.8 /
+     *    43.2). */
     const int pset = ty == LE_TYPE_Q6_K ? c->ms_p6 : ty == LE_TYPE_Q4_K ? c->ms_p : ty == LE_TYPE_Q8_0 ? c->ms_p80 : ty == LE_TYPE_Q4_0 ? c->ms_p40 : ty == LE_TYPE_Q5_K ? c->ms_p5k : ty == LE_TYPE_Q3_K ? c->ms_p3k : ty == LE_TYPE_IQ2_S ? c->ms_p2s : c->ms_piq;
+    const int cps = ty == LE_TYPE_Q6_K ? 14 : ty == LE_TYPE_IQ2_XXS ? 5 : ty == LE_TYPE_IQ3_XXS ? 7 : ty == LE_TYPE_Q8_0 ? 17 : ty == LE_TYPE_Q5_K ? 11 : ty == LE_TYPE_Q3_K ? 7 : ty == LE_TYPE_IQ2_S ? 6 : 9;
+    const size_t tab = ty == LE_TYPE_IQ2_S ? 9216 : ty == LE_TYPE_IQ2_XXS || ty == LE_TYPE_IQ3_XXS ? 3072 : 0;
+    auto lds_ms = [&](int p, int nw) {               /* without the tables, which are static */
+        const int cpr = (cps * p) | 1;               /* 16-byte slots of a staged row */
+        const int most = (nsb / p + nw - 1) / nw * p; /* super-blocks of the wave that has the most */
+        return (size_t)nw * ((size_t)most * 608 + (size_t)cpr * 256 + 128);
+    };
     const bool k456 = ty == LE_TYPE_Q4_K || ty == LE_TYPE_Q5_K || ty == LE_TYPE_Q6_K;
     int NWs = few && c->ms_wide && nsb >= 40 ? 16 : NW, P = pset;
     if (!pset) {
-        if (!few) P = nsb >= 16 && ty != LE_TYPE_Q8_0 ? 2 : 1;
+        if (!few) P = nsb >= 16 && ty != LE_TYPE_Q8_0 && (2 * (lds_ms(2, NWs) + tab) <= c->lds_limit || 2 * (lds_ms(1, NWs) + tab) > c->lds_limit) ? 2 : 1;
         else if (NWs == 16) P = k456 ? 2 : 1;
-        else P = ty == LE_TYPE_Q4_K && nsb >= 2 * NWs && (nsb + 2 * NWs - 1) / (2 * NWs) * 2 <= (nsb + NWs - 1) / NWs + 1 ? 2 : 1;
+        else P = (ty == LE_TYPE_Q4_K || ty == LE_TYPE_IQ2_XXS) && nsb >= 2 * NWs && (nsb + 2 * NWs - 1) / (2 * NWs) * 2 <= (nsb + NWs - 1) / NWs + 1 ? 2 : 1;
     }
     while (P > 1 && nsb % P) P >>= 1;
     /* Only some (P, NWs) pairs are instantiated (no P = 4 with 8 waves, P = 2 with 16 for the K-quants
      * only), every wave needs an item, and the waves' images, staging and tables must fit the LDS:
      * smaller items, then fewer waves, until one does; else the unstaged or vector kernels. */
-    const int cps = ty == LE_TYPE_Q6_K ? 14 : ty == LE_TYPE_IQ2_XXS ? 5 : ty == LE_TYPE_IQ3_XXS ? 7 : ty == LE_TYPE_Q8_0 ? 17 : ty == LE_TYPE_Q5_K ? 11 : ty == LE_TYPE_Q3_K ? 7 : ty == LE_TYPE_IQ2_S ? 6 : 9;
-    const size_t tab = ty == LE_TYPE_IQ2_S ? 9216 : ty == LE_TYPE_IQ2_XXS || ty == LE_TYPE_IQ3_XXS ? 3072 : 0;
     while (c->ms) {
-        const int cpr = (cps * P) | 1;                   /* 16-byte slots of a staged row */
-        const int most = (nsb / P + NWs - 1) / NWs * P;  /* super-blocks of the wave that has the most */
-        const size_t need = (size_t)NWs * ((size_t)most * 608 + (size_t)cpr * 256 + 128);
+        const size_t need = lds_ms(P, NWs);
         snprintf(name, sizeof name, "le_ms_%d_p%d_w%d%s", ty, P, NWs, xq8 ? "_q8" : "");
         if (nsb >= NWs * P && need + tab <= c->lds_limit && c->fn(name))
             return c->launch(name, dim3((unsigned)gx, (unsigned)slots), NWs * 64, need, st, args);

@@ -169,3 +169,23 @@ def test_gemm_small(engine, name, rows, nsb, m):
     assert np.all(np.isfinite(got))
     sel = np.ascontiguousarray(q.reshape(rows, -1)[pick])
     check_close(got[:, pick], oracle.matmat(ty, sel, len(pick), cols, x), absmag(ty, sel, len(pick), cols, x))
+
+
+# long K on 4 waves: items of one where only they leave room for two blocks a CU (112 super-blocks; Q6_K 88), of two
+# otherwise; two super-blocks an item for IQ2_XXS on 8 waves: the same bits as with the item size set
+@pytest.mark.parametrize("name,opt,rows,nsb,p", [("Q5_K", "ms_p5k", 4112, 112, 1), ("Q4_K", "ms_p", 4112, 112, 1), ("Q6_K", "ms_p6", 4112, 88, 1),
+                                                 ("Q6_K", "ms_p6", 4112, 112, 2), ("Q5_K", "ms_p5k", 4112, 88, 2), ("IQ2_XXS", "ms_piq", 2048, 32, 2)])
+def test_matvec_item_size(engine, fresh_engine, name, opt, rows, nsb, p):
+    import torch
+    ty, cols = le.MV_TYPES[name], 256 * nsb
+    dq = dev(wbytes(ty, 64, cols, seed=nsb)).reshape(-1).repeat(-(-rows // 64))[:rows * le.row_bytes(ty, cols)].clone()
+    dx = dev(acts(cols, nsb))
+    fresh_engine.set_option(opt, p)
+    print("item size", name, rows, cols, p, flush=True)
+    a, b = torch.empty(rows, device="cuda"), torch.empty(rows, device="cuda")
+    engine.mv(ty, dq, dx, a, rows, cols)
+    fresh_engine.mv(ty, dq, dx, b, rows, cols)
+    assert torch.equal(a.view(torch.int32), b.view(torch.int32))
+    fresh_engine.set_option(opt, 3 - p)
+    fresh_engine.mv(ty, dq, dx, b, rows, cols)
+    assert not torch.equal(a.view(torch.int32), b.view(torch.int32))  # the item sizes sum in different orders
