@@ -121,10 +121,59 @@ __device__ __forceinline__ int le_slot_walk(const int *__restrict__ off, int nsl
     }
     return -1;
 }
+/* A round of the walk: 256 slots from s0, every load in flight together; lane l of group q holds slot s0 + 64 q + l's
+ * pairs o0 .. o1, its tile count c and the number of tiles before it, first (from base tiles of earlier rounds). */
+struct LeRound {
+    int o0[4], o1[4], c[4], first[4];
+};
+__device__ __forceinline__ LeRound le_slot_round(const int *__restrict__ off, int nslot, int bm, int s0, int &base) {
+    const int lane = threadIdx.x & 63;
+    LeRound r;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const int s = min(s0 + 64 * q + lane, nslot - 1);
+        r.o0[q] = off[s];
+        r.o1[q] = off[s + 1];
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        r.c[q] = 0;
+        if (s0 + 64 * q >= nslot) continue; /* uniform */
+        if (s0 + 64 * q + lane < nslot) r.c[q] = (max(r.o1[q] - r.o0[q], 0) + bm - 1) / bm;
+        const int inc = le_wave_scan(r.c[q]);
+        r.first[q] = base + inc - r.c[q];
+        base += __builtin_amdgcn_readlane(inc, 63);
+    }
+    return r;
+}
 /* tile mt: its slot and first pair (false past the last tile) */
 __device__ __forceinline__ bool le_tile_of(const int *__restrict__ off, int nslot, int bm, int mt, int &slot, int &pair0) {
     int o0, first;
     slot = le_slot_walk(off, nslot, bm, [mt](int, int, int f, int c) { return mt >= f && mt < f + c; }, o0, first);
     pair0 = o0 + (mt - first) * bm;
     return slot >= 0;
+}
+/* Block bx of a launch whose blocks share the tiles, share(tiles) blocks each: that number, the tile's slot and its
+ * first pair (false past the last tile). The first round's offsets serve the count and the search. */
+template <class Share>
+__device__ __forceinline__ bool le_tile_shared(const int *__restrict__ off, int nslot, int bm, int bx, Share share, int &ng, int &slot, int &pair0) {
+    int base = 0;
+    const LeRound r = le_slot_round(off, nslot, bm, 0, base);
+    const int in0 = base;
+    for (int s0 = 256; s0 < nslot; s0 += 256) le_slot_round(off, nslot, bm, s0, base);
+    ng = share(base);
+    const int mt = bx / ng;
+    if (mt >= base) return false;
+    if (mt >= in0) return le_tile_of(off, nslot, bm, mt, slot, pair0);
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        if (64 * q >= nslot) break; /* uniform */
+        const unsigned long long h = __ballot(r.c[q] && mt >= r.first[q] && mt < r.first[q] + r.c[q]);
+        if (h) {
+            const int l = __ffsll((long long)h) - 1;
+            slot = 64 * q + l;
+            pair0 = __builtin_amdgcn_readlane(r.o0[q], l) + (mt - __builtin_amdgcn_readlane(r.first[q], l)) * bm;
+        }
+    }
+    return true;
 }

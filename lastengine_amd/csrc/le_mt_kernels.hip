@@ -48,7 +48,7 @@ struct MtArgs {
     const u8 *const *ptrs;
     unsigned long long w_slot_bytes;
     const int *off, *in_idx, *out_idx;
-    int nslot, maxt, ng, dual;
+    int nslot, cus, units, ng, dual; /* units: groups of row tiles; ng: blocks that share them under an even routing */
     const u8 *const *ptrs2;
     const u8 *w2;
     float *y2;
@@ -345,9 +345,16 @@ __device__ __forceinline__ void mt_body(const MtArgs &a) {
     extern __shared__ uint4 smem[];
     const int nsb = a.cols >> 8, ns = (int)gridDim.y;
     int M = a.m, bx = blockIdx.x, gx = gridDim.x, pair0 = 0, slot = 0;
-    if constexpr (GR) { /* ng blocks share a tile of up to T pairs of one slot */
+    if constexpr (GR) { /* gx blocks share a tile of up to T pairs of one slot */
         gx = a.ng;
-        if (!le_tile_of(a.off, a.nslot, T, bx / gx, slot, pair0)) return; /* uniform: past the last tile */
+        bool found;
+        if (T == 16 && !(a.kw > 1 && gx == a.units)) { /* a share that the number of tiles can change */
+            auto share = [&](int tiles) { return le_mtg_share(tiles, a.units, a.ng, a.kw, (int)gridDim.x, a.cus); };
+            found = le_tile_shared(a.off, a.nslot, T, bx, share, gx, slot, pair0);
+        } else {
+            found = le_tile_of(a.off, a.nslot, T, bx / gx, slot, pair0);
+        }
+        if (!found) return; /* uniform: past the last tile */
         bx %= gx;
         M = min(T, a.off[slot + 1] - pair0);
     }

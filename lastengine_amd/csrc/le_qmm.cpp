@@ -1103,7 +1103,7 @@ struct MtHostArgs { /* MtArgs in le_mt_kernels.hip */
     const void *const *ptrs;
     unsigned long long w_slot_bytes;
     const int *off, *in_idx, *out_idx;
-    int nslot, maxt, ng, dual;
+    int nslot, cus, units, ng, dual;
     const void *const *ptrs2;
     const void *w2;
     float *y2;
@@ -1299,13 +1299,13 @@ static int mm_grouped(le_ctx *c, int ty, const void *const *ptrs, const void *w,
      * of K do not fit the LDS (Q4_K from 17 super-blocks at 16 pairs) the tiles below stay. */
     if (c->mmg_mt && (long long)npair <= 6LL * nslot) {
         const int T = (long long)npair <= 2LL * nslot ? 8 : 16, nsb = cols / 256, ntile = (rows + 15) / 16 * (dual ? 2 : 1);
-        const int maxp = nslot + (npair + T - 1) / T, live = std::min(npair, nslot);
+        const int live = std::min(npair, nslot), maxt = le_mtg_tiles(npair, nslot, T);
         char name[32];
         snprintf(name, sizeof name, "le_mtg_%d_t%d", ty, T);
         int kw = 1;
         while (kw < 8 && 2 * kw <= nsb && (long long)ntile * live * kw < 8LL * 2 * c->cus) kw *= 2;
         const size_t lds = le_mt_lds(ty, nsb, T, T, kw > 1);
-        if (lds <= c->lds_limit && c->fn(name) && (long long)maxp * ntile <= 0x7FFFFFFFLL) {
+        if (lds <= c->lds_limit && c->fn(name) && (long long)maxt * ntile <= 0x7FFFFFFFLL) {
             /* row tiles per wave: four blocks a CU, or one where each builds 16 pairs' images (12 / 24 tokens as above:
              * two 84.8 / 113.8 us, four 81.6 / 103; 64 / 96 tokens: one 129 / 132, two 127 / 134, four 146 / 160) */
             const int side = 8 / kw, tpw = std::max(1LL, std::min<long long>(8, (long long)ntile * live / ((T == 16 ? 1LL : 4LL) * side * c->cus)));
@@ -1322,15 +1322,16 @@ static int mm_grouped(le_ctx *c, int ty, const void *const *ptrs, const void *w,
             a.in_idx = in_idx;
             a.out_idx = out_idx;
             a.nslot = nslot;
-            a.maxt = maxp;
-            a.ng = (ntile + side * tpw - 1) / (side * tpw);
+            a.cus = c->cus;
+            a.units = (ntile + side - 1) / side;
+            a.ng = (a.units + tpw - 1) / tpw;
             a.dual = dual ? 1 : 0;
             a.ptrs2 = ptrs2;
             a.w2 = w2;
             a.y2 = y2;
             a.up = up;
             void *args[] = {&a};
-            return c->launch(name, dim3((unsigned)(maxp * a.ng)), 512, lds, (hipStream_t)stream, args);
+            return c->launch(name, dim3((unsigned)le_mtg_grid(maxt, a.units, T, a.ng, c->cus)), 512, lds, (hipStream_t)stream, args);
         }
     }
     static const int cfgs[8][4] = {{1, 4, 1, 2}, {1, 4, 2, 2}, {1, 4, 4, 2}, {2, 2, 2, 2}, {1, 8, 2, 1}, {1, 8, 4, 1}, {1, 8, 1, 1}, {1, 4, 1, 1}};

@@ -95,10 +95,12 @@ def test_gemm_few_tokens(engine, name, rows, nsb, m):
 
 
 # grouped few-pair form: a tile's edges (8 and 9 pairs at 8 a pass, 16 and 17 at 16), empty slots at both ends,
-# one super-block and one row tile (one wave), waves sharing a tile, a K whose images do not fit the LDS
+# one super-block and one row tile (one wave), waves sharing a tile, a K whose images do not fit the LDS, every pair to one
+# slot (few tiles, each shared by more blocks), tiles past the first 256 slots
 @pytest.mark.parametrize("name", list(le.MV_TYPES))
 @pytest.mark.parametrize("rows,nsb,counts", [(16, 1, (0, 1, 0)), (37, 3, (0, 8, 0, 9, 0, 0, 0, 0, 1, 0)), (272, 7, (16, 0, 17, 1, 2)),
-                                             (2064, 4, (0, 3, 9, 0, 0, 0, 0)), (50, 17, (12, 5, 0, 0)), (40, 30, (2, 1))])
+                                             (2064, 4, (0, 3, 9, 0, 0, 0, 0)), (50, 17, (12, 5, 0, 0)), (40, 30, (2, 1)),
+                                             (1300, 3, (0,) * 9 + (70,) + (0,) * 7), (33, 2, (1, 9) + (0,) * 260 + (700, 0, 17, 1))])
 def test_grouped_few_pairs(engine, name, rows, nsb, counts):
     import torch
     ty, cols, nslot = le.MV_TYPES[name], 256 * nsb, len(counts)
