@@ -13,7 +13,8 @@
  *   - All pointers named w, x, y, out, logits, h, ws, ptrs, off, in_idx, out_idx are DEVICE
  *     pointers owned by the caller. Weights are raw GGUF row bytes (src/gpu.rs:79-83), row-major:
  *     `rows` rows of le_row_bytes(ty, cols) bytes; an expert slab e of a 3D tensor starts at
- *     e * rows * row_bytes (src/cpu_ref.rs:110-115).
+ *     e * rows * row_bytes (src/cpu_ref.rs:110-115). They, and the entries of a pointer table, may lie at
+ *     any even address; Q4_K and Q5_K from 33 tokens (64-pair grouped tiles) are faster 16-byte aligned.
  *   - `stream` is a hipStream_t (NULL = the null stream). Calls are asynchronous on it.
  *   - A context is thread-compatible, not thread-safe: use one per host thread or lock around
  *     it, as the reference drives one engine from one thread (src/local.rs:20,217).

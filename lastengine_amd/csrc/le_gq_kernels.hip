@@ -74,7 +74,7 @@ struct GqArgs {
     const u8 *const *ptrs2;
     const u8 *w2;
     float *y2;
-    int dual, pad2;
+    int dual, ids; /* ids: blocks of the whole grouped launch (le_gqu_*) */
     const float *up; /* non-null: the activation rows are silu(x) * up (the MoE down input) */
 };
 
@@ -497,8 +497,9 @@ __device__ __forceinline__ void gq_store(const GqArgs &a, u8 *lds, const float *
  * register staging. Every launched kernel uses NA = 2 (measured against registers at M=512: Q4_K
  * 109 -> 95 us, Q6_K 147 -> 114, Q8_0 252 -> 230, IQ2_XXS 98 -> 92; the three-slot ring 100 us for
  * Q4_K); the results are the same bits in every form. */
-template <int TY, int WM, int WN, int TM, int TN, bool GR = false, int NA = 0>
-__device__ __forceinline__ void gq_body(const GqArgs &a, const u8 *ws) {
+/* UA: only the tiles whose weights are not 16-byte aligned (gqu_body) */
+template <int TY, int WM, int WN, int TM, int TN, bool GR = false, int NA = 0, bool UA = false>
+__device__ __forceinline__ void gq_body(const GqArgs &a, const u8 *ws, const int id) {
     using F = GqF<TY>;
     constexpr bool AD = NA > 0;
     static_assert(NA == 0 || NA == 2 || NA == 3, "activation ring of 2 or 3 slots");
@@ -517,7 +518,7 @@ __device__ __forceinline__ void gq_body(const GqArgs &a, const u8 *ws) {
     const int NTR1 = (a.rows + BN - 1) / BN, NTR = GR && a.dual ? 2 * NTR1 : NTR1, MT = GR ? a.maxt : (a.m + BM - 1) / BM;
     /* 8 or more row tiles: blocks of one row tile (its token tiles) share blockIdx % 8, the XCD
      * and its L2; fewer: row tiles vary fastest, so consecutive blocks spread over every XCD */
-    const int id = blockIdx.x, j = id >> 3;
+    const int j = id >> 3;
     const int mt = NTR >= 8 ? j % MT : id / NTR, nt = NTR >= 8 ? (j / MT) * 8 + (id & 7) : id % NTR;
     if (nt >= NTR || mt >= MT) return; /* uniform over the block */
     const bool second = nt >= NTR1; /* dual grouped form: a row tile of the second weight set */
@@ -533,6 +534,7 @@ __device__ __forceinline__ void gq_body(const GqArgs &a, const u8 *ws) {
             Wsrc = a.ptrs2 ? a.ptrs2[sl] : a.w2 + (size_t)sl * a.w_slot_bytes;
         else
             Wsrc = a.ptrs ? a.ptrs[sl] : a.w + (size_t)sl * a.w_slot_bytes;
+        if (UA && ((size_t)Wsrc & 15) == 0) return;
     }
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave / WN, wn = wave % WN;
@@ -1086,6 +1088,23 @@ __device__ __forceinline__ void gq_body(const GqArgs &a, const u8 *ws) {
     gq_store<WM, WN, TM, TN, GR, 2 * BUF + NA * AB>(a, lds, tsc, acc, M, mb, nb, pair0, second);
 }
 
+/* Grouped form over a pointer table, behind the pipelined kernel: the tiles of the slots whose weights are not 16-byte
+ * aligned, which loads straight to LDS do not take (the grouped launch's `ids` blocks dealt to this one's). The host
+ * cannot look at a device table's entries; where all are aligned, as the tensors of a model file are, the blocks end
+ * after one look at it (2 us a launch; handled inside the pipelined kernel, a second way to load cost its 128-pair
+ * tiles 5-10% in spilled registers, and the check alone 2-3%: le_gpgt_*, with it, beside le_gpg_*). */
+template <int TY, int WM, int WN, int TM, int TN>
+__device__ __forceinline__ void gqu_body(const GqArgs &a, const u8 *ws) {
+    const int lane = threadIdx.x & 63;
+    u32 low = 0;
+    for (int s = lane; s < a.nslot; s += 64) low |= (u32)(size_t)a.ptrs[s] | (a.ptrs2 ? (u32)(size_t)a.ptrs2[s] : 0u);
+    if (!__any((int)(low & 15u))) return; /* uniform over the block: every wave looks at the whole table */
+    for (int id = blockIdx.x; id < a.ids; id += gridDim.x) {
+        gq_body<TY, WM, WN, TM, TN, true, 2, true>(a, ws, id);
+        __syncthreads(); /* the tile's staging is no longer read */
+    }
+}
+
 /* ============================ pipelined kernel ============================ */
 /* Q4_K and Q5_K from 33 tokens: a block of 4 waves computes 32 TM tokens x 256 rows, each wave all the
  * tokens of 64 rows of its own (TN = 2).
@@ -1218,7 +1237,7 @@ __device__ __forceinline__ void gp_lds_dma16(const u8 *base, u32 off, u32 lds_ad
 }
 #pragma clang diagnostic pop
 
-template <int TY, int TM, bool GR>
+template <int TY, int TM, bool GR, bool TB = false> /* TB: grouped form over a pointer table */
 __device__ __forceinline__ void gp_body(const GqArgs &a, const u8 *ws) {
     using F = GqF<TY>;
     constexpr int SLOT = gp_slot<TY>(), N16 = SLOT / 16;
@@ -1242,10 +1261,8 @@ __device__ __forceinline__ void gp_body(const GqArgs &a, const u8 *ws) {
         int sl;
         if (!le_tile_of(a.off, a.nslot, a.bm, mt, sl, pair0)) return;
         M = mb + min(BM, a.off[sl + 1] - pair0);
-        if (second)
-            Wsrc = a.ptrs2 ? a.ptrs2[sl] : a.w2 + (size_t)sl * a.w_slot_bytes;
-        else
-            Wsrc = a.ptrs ? a.ptrs[sl] : a.w + (size_t)sl * a.w_slot_bytes;
+        Wsrc = TB ? (second ? a.ptrs2 : a.ptrs)[sl] : (second ? a.w2 : a.w) + (size_t)sl * a.w_slot_bytes;
+        if (TB && ((size_t)Wsrc & 15)) return; /* left to le_gqu_* */
     }
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 31, hs = lane >> 5;
@@ -1494,19 +1511,22 @@ extern "C" __global__ void __launch_bounds__(256) le_gq_ksum(GqArgs a) {
 
 #define LE_GQ_(TY, WM, WN, TM, TN)                                                                                     \
     extern "C" __global__ void __launch_bounds__(WM * WN * 64) le_gq_##TY##_w##WM##WN##_t##TM##TN(GqArgs a, const u8 *ws) { \
-        gq_body<TY, WM, WN, TM, TN, false, 2>(a, ws);                                                                  \
+        gq_body<TY, WM, WN, TM, TN, false, 2>(a, ws, blockIdx.x);                                                                  \
     }
 #define LE_GQG_(TY, WM, WN, TM, TN)                                                                                     \
     extern "C" __global__ void __launch_bounds__(WM * WN * 64) le_gqg_##TY##_w##WM##WN##_t##TM##TN(GqArgs a, const u8 *ws) { \
-        gq_body<TY, WM, WN, TM, TN, true, 2>(a, ws);                                                                     \
+        gq_body<TY, WM, WN, TM, TN, true, 2>(a, ws, blockIdx.x);                                                                     \
     }
 /* one wave per SIMD is resident (LDS), but 256 registers: with 512 the accumulators go to the
  * accumulation registers, which the rescaling cannot reach without moves (393 reads a super-block) */
 #define LE_GP_REGS __attribute__((amdgpu_waves_per_eu(2, 2)))
 #define LE_GP_(TY, TM)                                                                                                  \
     extern "C" __global__ void __launch_bounds__(256) LE_GP_REGS le_gp_##TY##_t##TM(GqArgs a, const u8 *ws) { gp_body<TY, TM, false>(a, ws); } \
-    extern "C" __global__ void __launch_bounds__(256) LE_GP_REGS le_gpg_##TY##_t##TM(GqArgs a, const u8 *ws) { gp_body<TY, TM, true>(a, ws); }
-#define LE_GP(TY) LE_GP_(TY, 4) LE_GP_(TY, 2)
+    extern "C" __global__ void __launch_bounds__(256) LE_GP_REGS le_gpg_##TY##_t##TM(GqArgs a, const u8 *ws) { gp_body<TY, TM, true>(a, ws); } \
+    extern "C" __global__ void __launch_bounds__(256) LE_GP_REGS le_gpgt_##TY##_t##TM(GqArgs a, const u8 *ws) { gp_body<TY, TM, true, true>(a, ws); }
+#define LE_GQU_(TY, WM, WN, TM, TN) \
+    extern "C" __global__ void __launch_bounds__(WM * WN * 64) le_gqu_##TY##_w##WM##WN##_t##TM##TN(GqArgs a, const u8 *ws) { gqu_body<TY, WM, WN, TM, TN>(a, ws); }
+#define LE_GP(TY) LE_GP_(TY, 4) LE_GP_(TY, 2) LE_GQU_(TY, 1, 8, 4, 1) LE_GQU_(TY, 1, 8, 2, 1)
 #define LE_GQ(TY) LE_GQ_(TY, 1, 4, 1, 2) LE_GQ_(TY, 1, 4, 2, 2) LE_GQ_(TY, 1, 4, 4, 2) LE_GQ_(TY, 2, 2, 2, 2) \
     LE_GQ_(TY, 1, 8, 2, 1) LE_GQ_(TY, 1, 8, 4, 1) LE_GQ_(TY, 1, 8, 1, 1) LE_GQ_(TY, 1, 4, 2, 1) LE_GQ_(TY, 1, 4, 1, 1) LE_GQ_(TY, 1, 4, 4, 1) LE_GQG_(TY, 1, 8, 2, 1) LE_GQG_(TY, 1, 8, 4, 1) LE_GQG_(TY, 2, 2, 2, 2) LE_GQG_(TY, 1, 8, 1, 1) LE_GQG_(TY, 1, 4, 1, 1)
 #if LE_GQ_SET == 2

@@ -1067,7 +1067,7 @@ struct GqHostArgs {
     const void *const *ptrs2;
     const void *w2;
     float *y2;
-    int dual, pad2;
+    int dual, ids;
     const float *up;
 };
 static int gq_slot(int ty) {
@@ -1084,7 +1084,8 @@ static int gq_slot(int ty) {
     }
     return 0;
 }
-/* The pipelined kernel (le_gp_*: Q4_K and Q5_K, whole 256-row tiles) and its LDS: three weight step slots,
+/* The pipelined kernel (le_gp_*: Q4_K and Q5_K, whole 256-row tiles, weights loaded straight to LDS and so 16-byte
+ * aligned; others run on le_gq_*, whose loads go through registers) and its LDS: three weight step slots,
  * two of tm 32-token activation tiles, sum records of two super-blocks. */
 static bool gp_takes(int ty, int rows) { return (ty == LE_TYPE_Q4_K || ty == LE_TYPE_Q5_K) && rows >= 256; }
 static size_t gp_lds(int ty, int tm) { return (size_t)3 * 256 * gq_slot(ty) + (size_t)2 * tm * 8192 + (size_t)2 * tm * gq_srec(ty); }
@@ -1211,7 +1212,7 @@ static int gq_launch(le_ctx *c, int ty, const void *w, const float *x, int m, fl
      * the chip, else 128 (14336 x 4096 Q4_K, 64 / 128 tokens a block: M = 128 36.4 / 38.8 us, 256 48.2 / 52.5,
      * 512 90.4 / 74.0; 4096 x 4096 M = 512 38.9 / 41.2) */
     int gp = 0;
-    if (gp_takes(ty, rows) && !small) {
+    if (gp_takes(ty, rows) && al16(w) && !small) {
         if (c->gq_cfg) gp = c->gq_cfg == 21 ? 4 : c->gq_cfg == 22 ? 2 : 0;
         else if (m > 32) gp = (long long)((rows + 255) / 256) * ((m + 63) / 64) <= c->cus ? 2 : 4;
     }
@@ -1341,8 +1342,10 @@ static int mm_grouped(le_ctx *c, int ty, const void *const *ptrs, const void *w,
         const int BM = 32 * cfgs[i][0] * cfgs[i][2], BN = 32 * cfgs[i][1] * cfgs[i][3];
         return (size_t)2 * (BN * gq_slot(ty) + BM * 256) + (size_t)2 * (BM / 32) * srec + gq_tab(ty);
     };
-    /* Q4_K, Q5_K with 64- or 128-pair tiles: the pipelined kernel, same tiles */
-    const int gp = gp_takes(ty, rows) && c->mmg_gp && (ci == 4 || ci == 5) ? (ci == 4 ? 2 : 4) : 0;
+    /* Q4_K, Q5_K with 64- or 128-pair tiles: the pipelined kernel, same tiles (for a pointer table, whose entries the host
+     * cannot look at, with le_gqu_* behind it for the slots that are not aligned) */
+    const bool one = !dual || !ptrs == !ptrs2; /* both weight sets the same way: always so from the MoE layer */
+    const int gp = gp_takes(ty, rows) && c->mmg_gp && one && al16(w) && al16(w2) && (ci == 4 || ci == 5) ? (ci == 4 ? 2 : 4) : 0;
     if (!gp && lds_of(ci) > c->lds_limit) ci = 3; /* 128 x 128 on 4 waves */
     /* 32-pair tiles whose 8-wave block would hold more than half the LDS (Q6_K, Q8_0: one block
      * per CU): 32 x 128 on 4 waves, several blocks per CU */
@@ -1374,9 +1377,13 @@ static int mm_grouped(le_ctx *c, int ty, const void *const *ptrs, const void *w,
         rc = c->launch(name, dim3((unsigned)npair), 256, 0, (hipStream_t)stream, args);
     }
     if (rc) return rc;
-    if (gp) snprintf(name, sizeof name, "le_gpg_%d_t%d", ty, gp);
+    if (gp) snprintf(name, sizeof name, "le_gpg%s_%d_t%d", ptrs ? "t" : "", ty, gp);
     else snprintf(name, sizeof name, "le_gqg_%d_w%d%d_t%d%d", ty, WM, WN, TM, TN);
-    return c->launch(name, dim3((unsigned)grid), nthr, gp ? gp_lds(ty, gp) : lds_of(ci), (hipStream_t)stream, args);
+    rc = c->launch(name, dim3((unsigned)grid), nthr, gp ? gp_lds(ty, gp) : lds_of(ci), (hipStream_t)stream, args);
+    if (rc || !gp || !ptrs) return rc;
+    a.ids = (int)grid;
+    snprintf(name, sizeof name, "le_gqu_%d_w%d%d_t%d%d", ty, WM, WN, TM, TN);
+    return c->launch(name, dim3((unsigned)std::min<long long>(grid, c->cus)), 64 * WM * WN, lds_of(ci), (hipStream_t)stream, args);
 }
 
 int le_mm_grouped(le_ctx *c, int ty, const void *const *ptrs, const void *w, const int *off, const int *in_idx,

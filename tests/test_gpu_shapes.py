@@ -191,3 +191,55 @@ def test_matvec_item_size(engine, fresh_engine, name, opt, rows, nsb, p):
     fresh_engine.set_option(opt, 3 - p)
     fresh_engine.mv(ty, dq, dx, b, rows, cols)
     assert not torch.equal(a.view(torch.int32), b.view(torch.int32))  # the item sizes sum in different orders
+
+
+# weights that are not 16-byte aligned (a tensor inside a file image): tiles loaded straight to LDS are not taken for
+# them, in a pointer table slot by slot
+@pytest.mark.parametrize("name", ["Q4_K", "Q5_K"])
+@pytest.mark.parametrize("shift", [2, 8])
+@pytest.mark.parametrize("rows,nsb,m", [(300, 3, 40), (4096, 8, 300), (256, 1, 3)])
+def test_gemm_unaligned_weights(engine, fresh_engine, name, shift, rows, nsb, m):
+    import torch
+    ty, cols = le.MV_TYPES[name], 256 * nsb
+    q = wbytes(ty, rows, cols, seed=rows)
+    x = acts(m * cols, m).reshape(m, cols)
+    at = torch.zeros(q.size + 32, dtype=torch.uint8, device="cuda")
+    at[shift:shift + q.size] = dev(q).reshape(-1)
+    dw, dx, y = at[shift:shift + q.size], dev(x), torch.full((m, rows), float("nan"), device="cuda")
+    assert dw.data_ptr() % 16 == shift
+    print("unaligned GEMM", name, shift, rows, cols, m, flush=True)
+    for cfg in (0, 21, 22) if m > 32 else (0,):
+        fresh_engine.set_option("gq_cfg", cfg)
+        y.fill_(float("nan"))
+        fresh_engine.gemm(ty, dw, dx, m, y, rows, cols)
+        pick = np.unique(np.r_[0:8, rows - 8:rows])
+        sel = np.ascontiguousarray(q.reshape(rows, -1)[pick])
+        check_close(y.cpu().numpy()[:, pick], oracle.matmat(ty, sel, len(pick), cols, x), absmag(ty, sel, len(pick), cols, x))
+
+
+@pytest.mark.parametrize("name", ["Q4_K", "Q5_K"])
+@pytest.mark.parametrize("counts", [(20, 70, 0, 45), (150, 3, 200, 64), (3, 1, 0, 2)])  # tiles of 64, 128 and few pairs
+def test_grouped_unaligned_tables(engine, name, counts):
+    import torch
+    ty, rows, cols, nslot = le.MV_TYPES[name], 600, 768, len(counts)
+    q = wbytes(ty, nslot * rows, cols, seed=70).reshape(nslot, -1)
+    off = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    npair = int(off[-1])
+    x, perm = acts(npair * cols, 9).reshape(npair, cols), np.random.default_rng(1).permutation(npair).astype(np.int32)
+    dx, idx = dev(x), dev(perm)
+    rb = q.shape[1] + 64
+    outs = []
+    for shifts in ((0, 0, 0, 0), (2, 0, 8, 6)):
+        arena = torch.zeros(nslot * rb, dtype=torch.uint8, device="cuda")
+        for s, sh in enumerate(shifts):
+            arena[s * rb + sh:s * rb + sh + q.shape[1]] = dev(q[s])
+        ptrs = dev(np.array([arena.data_ptr() + s * rb + sh for s, sh in enumerate(shifts)], dtype=np.uint64))
+        y = torch.full((npair, rows), float("nan"), device="cuda")
+        print("unaligned tables", name, counts, shifts, flush=True)
+        engine.mm_grouped(ty, dev(off), idx, idx, nslot, npair, dx, y, rows, cols, ptrs=ptrs)
+        outs.append(y.cpu().numpy())
+    # the same codes and activations in both kernels, fp32 sums in another order: 2^-24 for each of K / 16 + K / 256 additions
+    for s in range(nslot):
+        p = perm[off[s]:off[s + 1]]
+        mag = absmag(ty, q[s], rows, cols, x[p])
+        assert np.all(np.abs(outs[0][p] - outs[1][p]) <= 6e-6 * mag)
