@@ -174,7 +174,10 @@ int le_matvec_q8(le_ctx *ctx, int ty, const void *const *ptrs, const void *w, co
  * le_gemm_workspace_size(ty, m, cols) bytes, the counterpart of the reference's pre-quantized
  * activation buffers (xqb/xdb/xsb, src/gpu.rs:210). Every type runs on the matrix cores (Q4_K: 3..16
  * tokens on a staged f16 MFMA kernel, 2 on the staged int8 matvec; other types: 2..16 tokens on the
- * few-token kernel, up to 8 of them with activations in two fp16 halves, about 2^-22 per value). From 17 tokens each token is scaled by
+ * few-token kernel, up to 8 of them with activations in two fp16 halves, about 2^-22 per value). Long K
+ * (from 13..34 super-blocks by type and tokens) runs there in slices whose partial results need the workspace of
+ * le_gemm_workspace_size_rows; with less, the vector kernels run below 9 tokens (15-bit activations; ws may be NULL),
+ * the larger GEMM from 9. From 17 tokens each token is scaled by
  * its own power of two and rounded to fp16 (relative error 2^-11 per value at any magnitude up to
  * 2^127); Q8_0 and Q4_0 weights enter as fp16(q * d_b * 2^S), one rounding, with a power of two per
  * row that keeps every code inside the fp16 range for any finite scales; the other types as exact

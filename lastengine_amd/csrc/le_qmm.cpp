@@ -1094,8 +1094,8 @@ static int gq_tab(int ty) {
 }
 
 /* Few tokens (m <= 16), every type: le_mt_*. Returns 1 where it does not apply (the caller goes on). The
- * partial results of K slices (needed where the activation images of all of K exceed the LDS) go to the
- * workspace; without room for them it does not apply. */
+ * partial results of K slices (needed where the activation images of all of K exceed the LDS, from 13..34
+ * super-blocks by type and tokens) go to the workspace; without room for them it does not apply. */
 struct MtHostArgs { /* MtArgs in le_mt_kernels.hip */
     const void *w;
     const float *x;
@@ -1110,15 +1110,29 @@ struct MtHostArgs { /* MtArgs in le_mt_kernels.hip */
     float *y2;
     const float *up;
 };
+/* K slices of le_mt_*, the fewest whose images fit the LDS of a gfx950 CU (0: none do): le_gemm_workspace_size_rows
+ * and the launch go by the same number. */
+struct MtShape {
+    int T, R, ks; /* tokens a pass, live MFMA rows, slices */
+    size_t lds;
+};
+static MtShape mt_shape(int ty, int m, int cols) {
+    MtShape s{m <= 4 ? 4 : m <= 8 ? 8 : 16, m <= 4 ? 8 : 16, 1, 0};
+    const int nsb = cols / 256;
+    for (; s.ks <= nsb; s.ks++) {
+        s.lds = le_mt_lds(ty, (nsb + s.ks - 1) / s.ks, s.R, s.T, true);
+        if (s.lds <= 160 * 1024) return s;
+    }
+    s.ks = 0;
+    return s;
+}
 static int mt_launch(le_ctx *c, int ty, const void *w, const float *x, int m, float *y, int rows, int cols, void *ws,
                      size_t ws_bytes, hipStream_t st) {
-    const int T = m <= 4 ? 4 : m <= 8 ? 8 : 16, R = T == 4 ? 8 : 16, NW = 8;
+    const MtShape s = mt_shape(ty, m, cols);
+    const int T = s.T, ks = s.ks, NW = 8;
     const int nsb = cols / 256, ntile = (rows + 15) / 16;
-    auto lds_of = [&](int ks) { return le_mt_lds(ty, (nsb + ks - 1) / ks, R, T, true); };
-    int ks = 1;
-    while (ks < nsb && lds_of(ks) > c->lds_limit) ks++;
-    const size_t lds = lds_of(ks);
-    if (lds > c->lds_limit || ks > 65535) return 1;
+    const size_t lds = s.lds;
+    if (!ks || lds > c->lds_limit || ks > 65535) return 1;
     float *part = nullptr;
     if (ks > 1) {
         if (!ws || !al16(ws) || ws_bytes < (size_t)ks * m * rows * 4) return 1;
@@ -1144,13 +1158,13 @@ static int mt_launch(le_ctx *c, int ty, const void *w, const float *x, int m, fl
     void *args[] = {&a};
     int rc = c->launch(name, dim3((unsigned)gx, (unsigned)ks), 64 * NW, lds, st, args);
     if (rc || !part) return rc;
-    GqHostArgs s{};
-    s.y = y;
-    s.rows = rows;
-    s.m = m;
-    s.ksplit = ks;
-    s.part = part;
-    void *sargs[] = {&s};
+    GqHostArgs k{};
+    k.y = y;
+    k.rows = rows;
+    k.m = m;
+    k.ksplit = ks;
+    k.part = part;
+    void *sargs[] = {&k};
     const size_t n4 = ((size_t)m * rows + 3) / 4;
     return c->launch("le_gq_ksum", dim3((unsigned)std::min<size_t>((n4 + 255) / 256, (size_t)c->cus * 8)), 256, 0, st, sargs);
 }
@@ -1405,9 +1419,14 @@ size_t le_gemm_workspace_size(int ty, int m, int cols) {
 
 size_t le_gemm_workspace_size_rows(int ty, int m, int rows, int cols) {
     const size_t base = le_gemm_workspace_size(ty, m, cols);
-    if (!base || rows <= 0 || !gq_may_split(m, rows)) return base;
-    const size_t full = gq_part_off(ty, m, cols) + (size_t)8 * m * rows * 4;
-    return full > base ? full : base;
+    if (!base || rows <= 0) return base;
+    size_t need = base;
+    if (gq_may_split(m, rows)) need = std::max(need, gq_part_off(ty, m, cols) + (size_t)8 * m * rows * 4);
+    if (m >= 2 && m <= 16) { /* the few-token kernel's slices, at any number of rows */
+        const int ks = mt_shape(ty, m, cols).ks;
+        if (ks > 1) need = std::max(need, (size_t)ks * m * rows * 4);
+    }
+    return need;
 }
 
 int le_gemm(le_ctx *c, int ty, const void *w, const float *x, int m, float *y, int rows, int cols, void *ws,
@@ -1419,8 +1438,8 @@ int le_gemm(le_ctx *c, int ty, const void *w, const float *x, int m, float *y, i
      * the le_gm GEMM carries), go to a GEMM */
     /* The other types up to 16 tokens: the few-token kernel (4 / 8 / 16 tokens against the vector kernels,
      * from 9 tokens the GEMM: Q6_K 4096 x 14336 67.3 -> 25.7, 124 -> 22.6, 30.6 -> 30.7 us, Q8_0 14336 x 4096
-     * 35.6 -> 18.4, 49.5 -> 21.3, 32.6 -> 22.1, Q5_K 3072 x 3072 12.3 -> 8.2, 20.6 -> 11.4, 15.9 -> 13.3);
-     * below "gq_min_m" without a workspace too */
+     * 35.6 -> 18.4, 49.5 -> 21.3, 32.6 -> 22.1, Q5_K 3072 x 3072 12.3 -> 8.2, 20.6 -> 11.4, 15.9 -> 13.3). Below "gq_min_m"
+     * a workspace is needed only for its K slices; without room for them the vector kernels run */
     const bool mt = c->mt && m >= 2 && m <= 16 && !c->gq_cfg && !c->gq_ksplit;
     if (mt && ty != LE_TYPE_Q4_K && m < c->gq_min_m && rows > 0 && cols > 0 && cols % 256 == 0 && w && x && y && al16(x)) {
         const int rc = mt_launch(c, ty, w, x, m, y, rows, cols, ws, ws_bytes, (hipStream_t)stream);

@@ -190,6 +190,18 @@ def test_gemm_workspace_size():
     assert L.le_gemm_workspace_size_rows(12, 0, 4096, 4096) == 0
 
 
+def test_gemm_workspace_size_few_tokens():
+    """Up to 16 tokens the workspace holds the few-token kernel's K slices at any number of rows: Q6_K at 16 super-blocks
+    and 8 tokens runs in two (8 waves' images of 8 tokens: 8768 bytes a super-block and 47 KB beside them)."""
+    L = qmm.lib()
+    L.le_gemm_workspace_size_rows.restype = ctypes.c_size_t
+    assert L.le_gemm_workspace_size_rows(14, 8, 128256, 4096) >= 2 * 8 * 128256 * 4
+    assert L.le_gemm_workspace_size_rows(14, 16, 128256, 4096) >= 2 * 16 * 128256 * 4
+    assert L.le_gemm_workspace_size_rows(8, 4, 128256, 14336) >= 2 * 4 * 128256 * 4
+    assert L.le_gemm_workspace_size_rows(14, 8, 128256, 2048) == L.le_gemm_workspace_size(14, 8, 2048)  # one slice
+    assert L.le_gemm_workspace_size_rows(14, 17, 128256, 4096) == L.le_gemm_workspace_size(14, 17, 4096)
+
+
 def test_moe_check_rejects_null_context():
     """le_moe_check validates its arguments on the host before touching the device."""
     L = qmm.lib()

@@ -94,6 +94,28 @@ def test_gemm_few_tokens(engine, name, rows, nsb, m):
     assert np.all(np.abs(y.cpu().numpy() - want) <= tol * mag + 1e-30), float(np.max(np.abs(y.cpu().numpy() - want) / (mag + 1e-30)))
 
 
+# ... an output head's rows with K in slices, on the workspace that le_gemm_workspace_size_rows states (by default) and on
+# the one without room for the slices' sums, below nine tokens none at all: the vector kernels' 15-bit activations there
+@pytest.mark.parametrize("name", ["Q6_K", "IQ2_S"])
+def test_gemm_few_tokens_head(engine, name):
+    import torch
+    ty, rows, cols, m = le.MV_TYPES[name], 70000, 4096, 8
+    q = wbytes(ty, 64, cols, seed=3)
+    dw = dev(q).reshape(-1).repeat(-(-rows // 64))[:rows * le.row_bytes(ty, cols)].clone()
+    x = acts(m * cols, 4).reshape(m, cols)
+    w = oracle.dequant_rows(ty, q, 64, cols).astype(np.float64)
+    want, mag = x.astype(np.float64) @ w.T, np.abs(x.astype(np.float64)) @ np.abs(w).T
+    small = torch.empty(engine.gemm_workspace_size(ty, m, cols), dtype=torch.uint8, device="cuda")
+    for kw, tol in (({}, 1e-5), ({"ws": small}, 1e-3), ({"ws": 0, "ws_bytes": 0}, 1e-3)):
+        y = torch.full((m, rows), float("nan"), device="cuda")
+        print("few tokens head", name, list(kw), flush=True)
+        engine.gemm(ty, dw, dev(x), m, y, rows, cols, **kw)
+        for r in (0, 64 * 500, rows - rows % 64):
+            got = y[:, r:r + 64].cpu().numpy()
+            n = got.shape[1]
+            assert np.all(np.abs(got - want[:, :n]) <= tol * mag[:, :n])
+
+
 # grouped few-pair form: a tile's edges (8 and 9 pairs at 8 a pass, 16 and 17 at 16), empty slots at both ends,
 # one super-block and one row tile (one wave), waves sharing a tile, a K whose images do not fit the LDS, every pair to one
 # slot (few tiles, each shared by more blocks), tiles past the first 256 slots
