@@ -78,12 +78,13 @@ void le_destroy(le_ctx *ctx);
 const char *le_last_error(const le_ctx *ctx);
 /* Launch-policy knobs (the counterpart of the reference's LE_MMQ* / LE_TMAX env switches,
  * src/gpu/dense.rs:182-192). Defaults are the measured best on MI355X; results do not depend on
- * them beyond fp32 summation order, except "gm_split". Unknown names or values give LE_ERR_ARG.
+ * them beyond fp32 summation order, except where a knob selects a kernel that rounds activations
+ * otherwise: "gm_split", "mt" and "mmg_mt" (below). Unknown names or values give LE_ERR_ARG.
  *   decode matvec, vector path:  "mv_block" threads per block (512, 1024), "mv_blocks_per_cu" grid
  *     cap, "mv_shape" rows x super-blocks in flight per lane (0 auto, 1: 1x2, 2: 2x1, 3: 2x2, 4: 4x1)
  *   decode matvec, matrix cores: "mq" (0/1), "ms" staged variant (0/1), "mq_waves" (2, 4, 8),
  *     "mq_waves_auto" (0/1: twice the waves when the row tiles do not fill the chip),
- *     "mq_steps", "mq_blocks_per_cu", super-blocks per row and step "ms_p" (Q4_K), "ms_p6" (Q6_K),
+ *     "mq_steps", "mq_blocks_per_cu", super-blocks per row and step (0 auto, 1, 2, 4) "ms_p" (Q4_K), "ms_p6" (Q6_K, not 4),
  *     "ms_piq" (IQ2_XXS, IQ3_XXS), "ms_p80" (Q8_0), "ms_p40" (Q4_0), "ms_p5k" (Q5_K), "ms_p3k"
  *     (Q3_K), "ms_p2s" (IQ2_S), and "mq6" / "mqiq" / "ms80" / "ms40" / "ms5k" / "ms3k" / "ms2s"
  *     (0/1) for the Q6_K / IQ / Q8_0 / Q4_0 / Q5_K / Q3_K / IQ2_S staged kernels (0: vector kernels);

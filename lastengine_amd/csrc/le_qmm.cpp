@@ -567,12 +567,12 @@ int le_set_option(le_ctx *c, const char *name, int value) {
     } else if (n == "mqiq") {
         c->mqiq = value ? 1 : 0;
     } else if (n == "ms_piq") {
-        if (value != 1 && value != 2 && value != 4) return c->fail(LE_ERR_ARG, "ms_piq must be 1, 2 or 4");
+        if (value != 0 && value != 1 && value != 2 && value != 4) return c->fail(LE_ERR_ARG, "ms_piq must be 0 (auto), 1, 2 or 4");
         c->ms_piq = value;
     } else if (n == "mq6") {
         c->mq6 = value ? 1 : 0;
     } else if (n == "ms_p6") {
-        if (value != 1 && value != 2) return c->fail(LE_ERR_ARG, "ms_p6 must be 1 or 2");
+        if (value < 0 || value > 2) return c->fail(LE_ERR_ARG, "ms_p6 must be 0 (auto), 1 or 2");
         c->ms_p6 = value;
     } else if (n == "gm_split") {
         if (value != 0 && value != 1) return c->fail(LE_ERR_ARG, "gm_split must be 0 or 1");
@@ -646,27 +646,27 @@ int le_set_option(le_ctx *c, const char *name, int value) {
     } else if (n == "ms_wide") {
         c->ms_wide = value ? 1 : 0;
     } else if (n == "ms_p2s") {
-        if (value != 1 && value != 2 && value != 4) return c->fail(LE_ERR_ARG, "ms_p2s must be 1, 2 or 4");
+        if (value != 0 && value != 1 && value != 2 && value != 4) return c->fail(LE_ERR_ARG, "ms_p2s must be 0 (auto), 1, 2 or 4");
         c->ms_p2s = value;
     } else if (n == "ms2s") {
         c->ms2s = value ? 1 : 0;
     } else if (n == "ms_p3k") {
-        if (value != 1 && value != 2 && value != 4) return c->fail(LE_ERR_ARG, "ms_p3k must be 1, 2 or 4");
+        if (value != 0 && value != 1 && value != 2 && value != 4) return c->fail(LE_ERR_ARG, "ms_p3k must be 0 (auto), 1, 2 or 4");
         c->ms_p3k = value;
     } else if (n == "ms3k") {
         c->ms3k = value ? 1 : 0;
     } else if (n == "ms_p5k") {
-        if (value != 1 && value != 2 && value != 4) return c->fail(LE_ERR_ARG, "ms_p5k must be 1, 2 or 4");
+        if (value != 0 && value != 1 && value != 2 && value != 4) return c->fail(LE_ERR_ARG, "ms_p5k must be 0 (auto), 1, 2 or 4");
         c->ms_p5k = value;
     } else if (n == "ms5k") {
         c->ms5k = value ? 1 : 0;
     } else if (n == "ms_p40") {
-        if (value != 1 && value != 2 && value != 4) return c->fail(LE_ERR_ARG, "ms_p40 must be 1, 2 or 4");
+        if (value != 0 && value != 1 && value != 2 && value != 4) return c->fail(LE_ERR_ARG, "ms_p40 must be 0 (auto), 1, 2 or 4");
         c->ms_p40 = value;
     } else if (n == "ms40") {
         c->ms40 = value ? 1 : 0;
     } else if (n == "ms_p80") {
-        if (value != 1 && value != 2 && value != 4) return c->fail(LE_ERR_ARG, "ms_p80 must be 1, 2 or 4");
+        if (value != 0 && value != 1 && value != 2 && value != 4) return c->fail(LE_ERR_ARG, "ms_p80 must be 0 (auto), 1, 2 or 4");
         c->ms_p80 = value;
     } else if (n == "ms80") {
         c->ms80 = value ? 1 : 0;
@@ -690,7 +690,7 @@ int le_set_option(le_ctx *c, const char *name, int value) {
     } else if (n == "ms_t") {
         c->ms_t = value ? 1 : 0;
     } else if (n == "ms_p") {
-        if (value != 1 && value != 2 && value != 4) return c->fail(LE_ERR_ARG, "ms_p must be 1, 2 or 4");
+        if (value != 0 && value != 1 && value != 2 && value != 4) return c->fail(LE_ERR_ARG, "ms_p must be 0 (auto), 1, 2 or 4");
         c->ms_p = value;
     } else if (n == "mq_waves") {
         if (value != 2 && value != 4 && value != 8) return c->fail(LE_ERR_ARG, "mq_waves must be 2, 4 or 8");

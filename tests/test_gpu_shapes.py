@@ -42,6 +42,34 @@ def test_matvec_ragged_split(engine, name, rows, nsb):
     assert np.all(np.abs(y.cpu().numpy() - want) <= 1e-5 * mag + 1e-30)
 
 
+# an item size can be handed back to the automatic choice, and the GEMM knobs take the values that the header names
+def test_options_automatic(fresh_engine):
+    import torch
+    opts = {"Q4_K": "ms_p", "Q6_K": "ms_p6", "Q8_0": "ms_p80", "Q4_0": "ms_p40", "Q5_K": "ms_p5k", "Q3_K": "ms_p3k", "IQ2_S": "ms_p2s",
+            "IQ2_XXS": "ms_piq", "IQ3_XXS": "ms_piq"}
+    rows, cols = 4112, 8192
+    for name, opt in opts.items():
+        ty = le.MV_TYPES[name]
+        dq, dx = dev(wbytes(ty, 257, cols, seed=ty)).reshape(-1).repeat(16), dev(acts(cols, 1))
+        outs = []
+        for v in (None, 1, 2, 0):
+            if v is not None:
+                fresh_engine.set_option(opt, v)
+            outs.append(torch.empty(rows, device="cuda"))
+            fresh_engine.mv(ty, dq, dx, outs[-1], rows, cols)
+        assert torch.equal(outs[0].view(torch.int32), outs[3].view(torch.int32)), opt
+        assert not torch.equal(outs[1].view(torch.int32), outs[2].view(torch.int32)), opt
+        for bad in (3, -1):
+            with pytest.raises(le.LeError) as e:
+                fresh_engine.set_option(opt, bad)
+            assert e.value.code == -1, opt
+    for k, v in [("mt", 0), ("mt", 1), ("mmg_mt", 0), ("mmg_mt", 1), ("mmg_gp", 0), ("mmg_gp", 1), ("gq_cfg", 21), ("gq_cfg", 22), ("gq_cfg", 0)]:
+        fresh_engine.set_option(k, v)
+    for v in (20, 23, -1):
+        with pytest.raises(le.LeError):
+            fresh_engine.set_option("gq_cfg", v)
+
+
 # the pipelined GEMM: its 64- and 128-token blocks (the latter where the former overfill the chip), first and last
 # token count, ragged last row tile (moved back to be whole), one super-block, K slices, super-blocks whose scale is
 # zero (offsets only) between ones whose scales differ by 2^20
