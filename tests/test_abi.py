@@ -33,7 +33,7 @@ def test_library_exports_every_declared_symbol():
 
 
 def test_code_objects_built():
-    for part in ("deq", "moe", "gm", "gq", "mv2", "mv8", "mv11", "mv12", "mv13", "mv14", "mv16", "mv18", "mv22"):
+    for part in ("deq", "moe", "gm", "mt", "gq", "gq2", "mv2", "mv8", "mv11", "mv12", "mv13", "mv14", "mv16", "mv18", "mv22"):
         assert os.path.getsize(os.path.join(qmm.LIB_DIR, "le_qmm_%s.hsaco" % part)) > 1000
 
 

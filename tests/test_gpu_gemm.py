@@ -118,12 +118,9 @@ def test_gemm_random_blocks(engine, name, m):
 @pytest.mark.parametrize("m", [5, 12, 40])
 def test_gemm_activation_magnitudes(engine, name, m):
     """Tokens of very different magnitude in one call (1e-6 .. 1e6, a zero token, one token with a
-    single non-zero value): each token (3..16-token Q4_K kernel: each token's super-block) is
-    scaled by its own power of two before fp16, so none overflows and none loses relative
-    precision."""
-    if m < 9 and name != "Q4_K":
-        pytest.skip("below 9 tokens the other types run on the vector kernels (per-block int8 images, "
-                    "no fp16 range); their offset form leaves 2^-15-level residues where sum|wx| is 0")
+    single non-zero value): each token (up to 16 tokens: each token's super-block) is scaled by its
+    own power of two before fp16, so none overflows and none loses relative precision. Up to 8
+    tokens of the types other than Q4_K, two fp16 halves keep about 2^-22 of it."""
     ty = le.MV_TYPES[name]
     rows, cols = 256, 1024
     zt, st = (3, 7) if m > 7 else (1, m - 1)
@@ -144,6 +141,10 @@ def test_gemm_activation_magnitudes(engine, name, m):
         if t == zt:
             continue
         check_close(got[t:t + 1], want[t:t + 1], mag[t:t + 1])
+    if m <= 8 and name != "Q4_K":
+        w = oracle.dequant_rows(ty, q, rows, cols).astype(np.float64)
+        exact, mag = xs.astype(np.float64) @ w.T, np.abs(xs.astype(np.float64)) @ np.abs(w).T
+        assert np.all(np.abs(got - exact) <= 1e-5 * mag)
 
 
 @pytest.mark.parametrize("name", NAMES)
@@ -220,10 +221,12 @@ def test_gemm_slices_follow_tiles(fresh_engine, name, rows, cols, m, ks):
 
 
 @pytest.mark.parametrize("name,rows,cols,m,cfg", [("Q5_K", 4096, 4096, 192, 22), ("Q4_K", 2048, 8192, 160, 22), ("IQ3_XXS", 2048, 4096, 320, 5),
-                                                  ("Q6_K", 6144, 4096, 100, 5), ("Q5_K", 3072, 3072, 320, 8), ("IQ2_S", 3072, 3072, 256, 8)])
+                                                  ("Q6_K", 6144, 4096, 100, 5), ("Q5_K", 3072, 3072, 320, 8), ("IQ2_S", 3072, 3072, 256, 8),
+                                                  ("Q5_K", 14336, 4096, 64, 22), ("Q4_K", 8192, 4096, 600, 21)])
 def test_gemm_tile_by_chain(fresh_engine, name, rows, cols, m, cfg):
     """Where 64 x 128 tiles would keep a long chain of super-blocks that 64 x 256 tiles cut by K slices, the wide tile
-    runs (first four), else the small one: the same bits as with that block shape set."""
+    runs (first four), else the small one; beyond the small tiles' work Q4_K and Q5_K run the pipelined kernel, 64 tokens a
+    block and, past one block a CU, 128 (last two): the same bits as with that block shape set."""
     import torch
     ty = le.MV_TYPES[name]
     dq, dx = dev(random_blocks(ty, rows, cols, seed=m)), dev(acts(m * cols, m).reshape(m, cols))

@@ -105,8 +105,8 @@ def test_moe_pointer_tables(engine, n_tok):
 @pytest.mark.parametrize("name", ["Q4_K", "Q6_K"])
 def test_mm_grouped_many_slots(engine, name):
     """More slots than one round of the blocks' slot walk (256 per round): pairs only in a few
-    slots on both sides of the round and wave boundaries (63/64, 255/256), one slot spanning two
-    32-pair tiles, the rest empty."""
+    slots on both sides of the round and wave boundaries (63/64, 255/256), one slot spanning
+    several tiles (of 8 pairs: so few pairs a slot run the few-pair form), the rest empty."""
     import torch
     ty = le.MV_TYPES[name]
     nslot, rows, cols, n_src = 300, 128, 512, 64

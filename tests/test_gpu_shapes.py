@@ -150,6 +150,7 @@ def test_gemm_few_tokens_head(engine, name):
 @pytest.mark.parametrize("name", list(le.MV_TYPES))
 @pytest.mark.parametrize("rows,nsb,counts", [(16, 1, (0, 1, 0)), (37, 3, (0, 8, 0, 9, 0, 0, 0, 0, 1, 0)), (272, 7, (16, 0, 17, 1, 2)),
                                              (2064, 4, (0, 3, 9, 0, 0, 0, 0)), (50, 17, (12, 5, 0, 0)), (40, 30, (2, 1)),
+                                             (40, 13, (12, 5, 0, 0)), (40, 14, (12, 5, 0, 0)), (40, 16, (12, 5, 0, 0)),
                                              (1300, 3, (0,) * 9 + (70,) + (0,) * 7), (33, 2, (1, 9) + (0,) * 260 + (700, 0, 17, 1))])
 def test_grouped_few_pairs(engine, name, rows, nsb, counts):
     import torch
@@ -170,6 +171,31 @@ def test_grouped_few_pairs(engine, name, rows, nsb, counts):
         xs = x[in_idx[off[s]:off[s + 1]]].astype(np.float64)
         # activations rounded to fp16 (2^-11 each), fp32 sums far below it
         assert np.all(np.abs(got[off[s]:off[s + 1]] - xs @ w[s].T) <= 1e-3 * (np.abs(xs) @ np.abs(w[s]).T) + 1e-30)
+
+
+# grouped tiles of 32, 64 and 128 pairs past the first 256 slots (the blocks' walk takes 256 at a time), some slots empty,
+# tiles with one pair of their last
+@pytest.mark.parametrize("name", ["Q4_K", "Q6_K", "Q5_K"])
+@pytest.mark.parametrize("mean,bm", [(8, 32), (20, 64), (70, 128)])
+def test_grouped_tiles_many_slots(engine, name, mean, bm):
+    import torch
+    ty, rows, cols, nslot = le.MV_TYPES[name], 300, 256, 270
+    counts = np.random.default_rng(mean).poisson(mean, nslot)
+    counts[[0, 7, 255, 256, 269]] = (0, 2 * bm + 1, bm + 1, 0, bm)
+    off = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    npair = int(off[-1])
+    assert 6 * nslot < npair and (npair <= 16 * nslot) == (bm == 32) and (npair > 64 * nslot) == (bm == 128)
+    q = wbytes(ty, nslot * rows, cols, seed=mean).reshape(nslot, -1)
+    x, perm = acts(npair * cols, mean).reshape(npair, cols), np.random.default_rng(2).permutation(npair).astype(np.int32)
+    y = torch.full((npair, rows), float("nan"), device="cuda")
+    print("grouped tiles, many slots", name, npair, flush=True)
+    engine.mm_grouped(ty, dev(off), dev(perm), dev(perm), nslot, npair, dev(x), y, rows, cols, w=dev(q))
+    got = y.cpu().numpy()
+    assert np.isfinite(got).all()
+    for s in (1, 7, 63, 64, 254, 255, 257, 269):
+        p = perm[off[s]:off[s + 1]]
+        if len(p):
+            check_close(got[p], oracle.matmat(ty, q[s], rows, cols, x[p]), absmag(ty, q[s], rows, cols, x[p]))
 
 
 # dequantization: waves of 64 units: a part of one, exactly one, one unit more, several grid strides (256 CUs x 16 blocks)
