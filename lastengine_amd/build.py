@@ -16,7 +16,7 @@ LIB = os.path.join(HERE, "lib")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 HIPCC = os.environ.get("HIPCC", ROCM + "/bin/hipcc")
 
-# Packed FP32 instructions are disabled for all device code (they are not trusted on this pool).
+# Packed FP32 instructions are disabled for all device code (some of their forms have given wrong results on this hardware).
 DEVICE_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang",
                 "-packed-fp32-ops", "-I" + CSRC]
 PARTS = {"deq": ["-DLE_PART_DEQ"], "moe": ["-DLE_PART_MOE"]}

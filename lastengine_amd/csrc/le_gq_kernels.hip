@@ -1119,8 +1119,7 @@ __device__ __forceinline__ void gqu_body(const GqArgs &a, const u8 *ws) {
  *
  * Position q of a step (8 positions of 16 values, in the decoder's order): weight bytes are read from
  * LDS two positions ahead, activation fragments and B fragments are ready one ahead. All global loads go
- * straight to LDS, a few per position (13 at once held up the wave's instructions: 131k -> 116k cycles
- * for the loop at M = 512). Activations: two step slots; the only barrier of a step sits between its
+ * straight to LDS, a few per position (13 at once held up the wave's instructions). Activations: two step slots; the only barrier of a step sits between its
  * positions 6 and 7, when every wave has read its last activation fragment of the step and its loads of
  * the next one have landed. Weights: private to the wave, three step slots, loaded two steps ahead (a
  * register-staged form one step ahead was bound by their latency: 88 against 79 us at M = 512; the 2-byte
@@ -1128,10 +1127,12 @@ __device__ __forceinline__ void gqu_body(const GqArgs &a, const u8 *ws) {
  * faster than here). The accumulator holds a row's sum in units of the super-block scale; the offset
  * term of one tile per position is added beside the MFMAs.
  *
- * Measured, 14336 x 4096 Q4_K, against gq_body's best tile on the same card: M = 64 31.8 -> 29.3 us, 128
- * 40.2 -> 36.4, 256 55.0 -> 48.2, 512 80.6 -> 74.0 (813 TFLOP/s), 1024 155 -> 139; 28672 rows, M = 512
- * 155 -> 137. Bound by the matrix cores and the clock: the loop takes 116k cycles, its MFMAs alone
- * 82k (136 per super-block and wave, 32 cycles each), while the clock falls to 1.7 GHz under them. */
+ * Measured, whole calls (pre-pass and slice sums included) on weights that no cache holds, in turn with gq_body's best
+ * tile, 14336 x 4096: Q4_K M = 64 30.6 -> 29.1 us, 128 41.9 -> 38.3, 256 62.8 -> 54.2, 512 92.9 -> 78.9 (762 TFLOP/s); Q5_K
+ * M = 512 98.3 -> 82.5. Under a benchmark's minutes of load, where the clock falls, 4% of M = 512 are left (96.8 ->
+ * 93.0). Counters of the launch at M = 512 (profiles/counters_gemm_few_tokens.md): matrix cores busy 38% of the SIMD
+ * cycles (gq_body 33%), half its LDS instructions, 0.8 conflict cycles each; its 448 blocks are a round and three
+ * quarters of the 256 CUs. */
 /* bytes of a staged row per step (its header in front: 16-byte pieces of half super-block 0; of half 1
  * the same 64 bytes further, where the header's place holds bytes that are not used) */
 template <int TY>

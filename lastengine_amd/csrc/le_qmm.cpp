@@ -1173,14 +1173,13 @@ static int gq_launch(le_ctx *c, int ty, const void *w, const float *x, int m, fl
                      size_t ws_bytes, hipStream_t st) {
     /* block shapes: (WM, WN, TM, TN) -> BM = 32 TM WM tokens, BN = 32 TN WN rows */
     static const int cfgs[12][4] = {{1, 4, 1, 2}, {1, 4, 2, 2}, {1, 4, 4, 2}, {2, 2, 2, 2}, {1, 8, 2, 1}, {1, 8, 4, 1}, {1, 8, 1, 1}, {1, 4, 2, 1}, {1, 4, 1, 1}, {1, 4, 4, 1}, {2, 4, 2, 2}, {2, 4, 2, 1}};
-    /* block shape by token count and type, from sweeps of every type at its config shape
-     * (14336 x 4096; Q6_K and IQ3_XXS 4096 x 14336, Q8_0 32000 x 4096), activations loaded straight
-     * into LDS: up to 32 tokens 32 x 128 tiles on 4 waves; 33..64 tokens 64 x 128 on 4 waves for
-     * Q6_K and IQ3_XXS, 64 x 256 on 8 waves otherwise; 65..128 tokens 128 x 128 on 4 waves for
-     * Q6_K (M=128 47.6 -> 46.3 us against 64 x 256), 64 x 256 on 8 waves for Q4_K, Q5_K and
-     * IQ3_XXS (M=128 against 128 x 256: Q4_K 44.8 -> 40.9, Q5_K 46.1 -> 43.0); 129..256 tokens
-     * 64 x 256 on 8 waves for Q4_K and Q5_K; everything else 128 x 256 on 8 waves (Q6_K M=256 72.8
-     * -> 66.0 us and M=512 126.5 -> 107.8 against 64 x 256) */
+    /* block shape by token count and type, from sweeps of every type (14336 x 4096; Q6_K and IQ3_XXS 4096 x 14336, Q8_0
+     * 32000 x 4096), activations loaded straight into LDS: up to 32 tokens 32 x 128 tiles on 4 waves; 33..64 tokens
+     * 64 x 128 on 4 waves for Q6_K and IQ3_XXS, 64 x 256 on 8 waves otherwise; 65..128 tokens 128 x 128 on 4 waves for Q6_K
+     * (M = 128 47.6 -> 46.3 us against 64 x 256), 64 x 256 on 8 waves for IQ3_XXS; everything else 128 x 256 on 8 waves
+     * (Q6_K M = 256 72.8 -> 66.0 us and M = 512 126.5 -> 107.8 against 64 x 256). Q4_K and Q5_K leave these tiles from 33
+     * tokens (small tiles, pipelined kernel below), but for fewer than 256 rows and for weights that are not 16-byte
+     * aligned: 64 x 256 up to 256 tokens there (M = 128 against 128 x 256: Q4_K 44.8 -> 40.9, Q5_K 46.1 -> 43.0) */
     int ci = 5;
     const bool k45 = ty == LE_TYPE_Q4_K || ty == LE_TYPE_Q5_K;
     if (m <= 32) ci = 8;
@@ -1311,7 +1310,10 @@ static int mm_grouped(le_ctx *c, int ty, const void *const *ptrs, const void *w,
      * experts of 2048 x 768, 8 a token, Q4_K and Q6_K: 12 / 24 / 32 / 64 / 96 tokens (0.75 to 6 pairs a slot)
      * 96.1 / 111 / 128 / 142 / 148 -> 81.6 / 103 / 114 / 129 / 132 us; at 128 tokens (8) 154 -> 182. IQ2_XXS and IQ3_XXS,
      * 12 / 24 / 90 tokens: 82.1 / 97.7 / 124 -> 78.3 / 97.0 / 123; Q8_0, 90 tokens: 275 -> 158. Where the images of all
-     * of K do not fit the LDS (Q4_K from 17 super-blocks at 16 pairs) the tiles below stay. */
+     * of K do not fit the LDS (le_mt_lds; Q4_K at 16 pairs from 16 super-blocks, from 14 with several waves a row tile)
+     * the tiles below stay. The host sees the mean only: at two or six pairs a slot with half of them on eight experts this
+     * form is 5-20% behind the tiles below, at an even routing 15-30% ahead (768 x 2048 Q4_K, 256 pairs 34 / 31 and 35 / 48
+     * us, 768 pairs 52 / 50 and 39 / 50). */
     if (c->mmg_mt && (long long)npair <= 6LL * nslot) {
         const int T = (long long)npair <= 2LL * nslot ? 8 : 16, nsb = cols / 256, ntile = (rows + 15) / 16 * (dual ? 2 : 1);
         const int live = std::min(npair, nslot), maxt = le_mtg_tiles(npair, nslot, T);
