@@ -131,6 +131,7 @@ __device__ __forceinline__ LeRound le_slot_round(const int *__restrict__ off, in
     LeRound r;
 #pragma unroll
     for (int q = 0; q < 4; q++) {
+        if (s0 + 64 * q >= nslot) break; /* uniform */
         const int s = min(s0 + 64 * q + lane, nslot - 1);
         r.o0[q] = off[s];
         r.o1[q] = off[s + 1];
@@ -153,16 +154,16 @@ __device__ __forceinline__ bool le_tile_of(const int *__restrict__ off, int nslo
     pair0 = o0 + (mt - first) * bm;
     return slot >= 0;
 }
-/* Block bx of a launch whose blocks share the tiles, share(tiles) blocks each: that number, the tile's slot and its
- * first pair (false past the last tile). The first round's offsets serve the count and the search. */
+/* Block bx of a launch whose blocks share the tiles, share(tiles) blocks each (most often the given ng): that number, the
+ * tile's slot and its first pair (false past the last tile). The first round's offsets serve the count and the search. */
 template <class Share>
 __device__ __forceinline__ bool le_tile_shared(const int *__restrict__ off, int nslot, int bm, int bx, Share share, int &ng, int &slot, int &pair0) {
-    int base = 0;
+    int base = 0, mt = bx / ng; /* the division while the offsets load */
     const LeRound r = le_slot_round(off, nslot, bm, 0, base);
-    const int in0 = base;
+    const int in0 = base, even = ng;
     for (int s0 = 256; s0 < nslot; s0 += 256) le_slot_round(off, nslot, bm, s0, base);
     ng = share(base);
-    const int mt = bx / ng;
+    if (ng != even) mt = bx / ng;
     if (mt >= base) return false;
     if (mt >= in0) return le_tile_of(off, nslot, bm, mt, slot, pair0);
 #pragma unroll
